@@ -60,12 +60,12 @@ def build(verbose: bool = False) -> str:
 
 
 def build_oracle(with_reference: bool = True) -> None:
-    """Compile the parity oracle (and, where /root/reference exists, the
-    compiled reference under oracle/_ref).  Test infrastructure only."""
+    """Compile the parity oracle (and, where /root/reference holds the
+    sources, the compiled reference under oracle/_ref).  Test infrastructure only."""
     odir = os.path.join(ROOT, "oracle")
     _run(["make", "-s", "-C", odir, "all"])
     ref = os.environ.get("TBQ_REFERENCE", "/root/reference")
-    if with_reference and os.path.isdir(ref) and shutil.which("make"):
+    if with_reference and os.path.isdir(os.path.join(ref, "layer4")) and shutil.which("make"):
         _run(["make", "-s", "-C", odir, f"REF={ref}", "ref"])
 
 
