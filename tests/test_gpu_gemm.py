@@ -3,9 +3,9 @@ fp16 MFMA kernel with fp32 accumulation, for W as fp16 halves or as Q4_K
 rows dequantised inside the kernel.
 
 * fp16 W: against a torch fp32 product of the same fp16 values (only the
-  summation order differs), over tile edges (T and N not multiples of the
-  128 x 128 tile), a row stride ldc > N and the split-K shapes (partial sums
-  added in slice order).
+  summation order differs), over tile edges (T and N not multiples of a
+  tile), a row stride ldc > N and the split-K shapes (partial sums added in
+  slice order).
 * Q4_K W: close to the fp16 path on the fp16 values of the oracle's
   dequantised weights (the kernel's packed fp16 decode rounds 16 S, M and
   S q - M to fp16, about one fp16 ulp per weight), and to the fp64 product
@@ -73,6 +73,31 @@ def test_gemm_q4k_fused_matches_f16_path(oracle, T, N, K):
     ref = X.astype(np.float64) @ wf.astype(np.float64).T
     assert rel_l2(a, ref) <= 1e-3   # fp16 rounding of the weights
     assert rel_l2(b, ref) <= 1e-3
+
+
+# One shape on each side of the tiles' edges (32, 64, 128 and 256 tokens, 128
+# and 256 weight rows), one super-block, uneven slices, more tiles than CUs.
+@pytest.mark.parametrize("T,N,K", [
+    (1, 4, 256), (31, 124, 512), (33, 132, 256), (64, 260, 8192), (65, 1028, 2304), (127, 256, 5120),
+    (129, 6148, 768), (257, 516, 1792), (513, 3076, 256), (1030, 5124, 512),
+])
+def test_gemm_tile_edges(oracle, T, N, K):
+    import torch
+    rng = np.random.default_rng(T * 7 + N + K)
+    Wq = synth.kquant_matrix(fm.Q4_K, N, K, rng)
+    wf = oracle.dequant_rows(Wq, fm.Q4_K, N, K)
+    w16 = wf.astype(np.float16)
+    X = _x16(T, K, rng)
+    x64 = torch.from_numpy(X).cuda().double()
+    prod = lambda w: (x64 @ _dev(w).double().t().contiguous()).cpu().numpy()   # noqa: E731
+    for qt, W, ref, tol in ((fm.F16, w16, prod(w16), 1e-6), (fm.Q4_K, Wq, prod(wf), 1e-3)):
+        print("gemm edges", T, N, K, fm.NAMES[qt], flush=True)
+        C = torch.full((T + 1, N), 7.0, dtype=torch.float32, device="cuda")
+        tb.gemm(_dev(W), qt, _dev(X), T, N, K, C)
+        got = C.cpu().numpy()
+        assert rel_l2(got[:T], ref) <= tol            # fp32 sums; fp16 rounding of the decoded weights
+        assert np.abs(got[:T] - ref).max() <= 20 * tol * np.sqrt(np.mean(ref ** 2)) # no single row or column off
+        assert np.all(got[T] == 7.0)                  # nothing past the last row
 
 
 def test_gemm_rejects_bad_shapes():

@@ -5,7 +5,7 @@
 //
 // Per layer (x: fp32 residual rows [T][H]; h16: fp16 rows with per-row
 // power-of-two scales, the GEMMs' activation operand; the GEMMs are
-// k_hgemm (tbq_gemm.hip): Q4_K weights are dequantised inside it, any other
+// k_hgemm_* (tbq_gemm.hip): Q4_K weights are dequantised inside it, any other
 // format to fp16 first (k_dequant_f16, one reused buffer)):
 //   k_pf_norm        x += y (the previous sublayer's output, unscaled by
 //                    its row scales), h16 = rmsnorm(x) * attn_norm

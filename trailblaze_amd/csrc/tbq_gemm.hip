@@ -5,31 +5,52 @@
 //                                      rows or Q4_K rows, fp32 accumulate and
 //                                      output
 //
-// Tiling.  A workgroup of 4 waves owns a 128 (n) x 128 (t) tile of C (rows
-// past N or T are clamped on load and not stored), two workgroups per CU;
-// wave w owns the 64 x 64 block (n half w & 1, t half w >> 1) as 2 x 2
-// blocks of v_mfma_f32_32x32x16_f16 (A = 32 weight rows x 16 k, B = 16 k x
-// 32 tokens).  Measured alternatives, all slower on the Qwen3-4B prefill
-// shapes: 128 x 256 and 256 x 128 tiles of 8 waves (one workgroup per CU),
-// 128 x 64 blocks per wave, K steps of 32 with four workgroups per CU.
-// K advances 64 columns per step through two LDS stages of both operands
-// ([row][64 + 8 halves]: the 8-half pad puts any 8 consecutive rows of a
-// 16-byte column read on 8 disjoint 4-bank groups).  Step s+2's global loads
-// are issued two steps ahead into one of two register sets and written to
-// the other LDS stage after step s's MFMAs, with one barrier per step.
+// Both kernels own a tile of weight rows x tokens in blocks of
+// v_mfma_f32_32x32x16_f16 (A = 32 weight rows x 16 k, B = 16 k x 32 tokens),
+// advance K by 64 columns a step, and bring their operands into two LDS
+// stages with direct global-to-LDS copies (tbq_dma.hpp): a step's copies are
+// issued at the start of the step before and waited for at its end, so no
+// register holds data in flight.  LDS rows are 128 bytes (64 halves) without
+// padding; the 16-byte segment of row r sits at slot seg ^ (r & 7) ^ (r >> 3
+// & 1), so the 32 rows of a column read spread over all banks (the copies'
+// per-lane source addresses place them there).
 //
-// Weights.  fp16 rows are copied.  Q4_K rows (reference layout) are
-// dequantised on the way into LDS: per step a thread takes a piece of one
-// 32-weight sub-block of one row (its quant bytes, the super-block's d/dmin
-// and the sub-block's 6-bit scale and min, with the reference's reading of
-// the scale bytes, layer4/tb_gguf.c:148-180) and writes its fp16 weights
-// (q4sub_f16).
+// What bounds them (MI355X): on random operands the matrix cores alone reach
+// 1.6 PFLOP/s here (2.16 on zeros: the power limit sets the clock), and every
+// VALU instruction beside an MFMA costs clock as well (1.28 PFLOP/s at 4 per
+// MFMA).  k_hgemm_q4k without its copies and without the dequantisation runs
+// at 1.18 PFLOP/s.
 //
-// Split K.  When the n x t tiles are fewer than the CUs can run, K is split
-// over gridDim.z slices; slice z writes its partial sums to P[z][T][N] and
-// k_gemm_reduce adds the slices in slice order into C.
+// k_hgemm_q4k (Q4_K rows, reference layout).  Wave w owns 64 weight rows and
+// all of the tile's tokens, so a weight is dequantised once per tile by the
+// one wave that uses it and never passes through LDS as fp16: only the packed
+// bytes are staged (4.5 bits a weight), each lane reads its own row's 16
+// quant bytes of a step and makes its A fragments in registers between the
+// MFMAs of the fragments before (the k order inside a step is permuted: lane
+// half h covers columns 32 h .. + 31, for both operands).  64 x 128 blocks
+// per wave read 4 KiB of LDS per 8 MFMAs.  Two workgroups of 256 x 128 per CU
+// overlap each other's barriers: one workgroup of 256 x 256 that dequantises
+// into LDS (8 waves in step) was slower on every shape (T = 1999: 19456 x
+// 2560 295 against 198 us).  Against the kernel this replaces (128 x 128
+// tiles, operands through registers into padded LDS): T = 512: 6144 x 2560
+// 45.1 -> 26.8 us, 2560 x 4096 37.0 -> 22.9, 2560 x 9728 67.4 -> 39.8, gate |
+// up 19456 x 2560 106.1 -> 66.1 (SwiGLU included); T = 1999: 124.6 -> 72.4,
+// 102.6 -> 56.4, 211.3 -> 126.0 and 330.8 -> 198.2 us (1.0 PFLOP/s).
+//
+// k_hgemm_f16 (fp16 rows).  Both operands through LDS, waves in a WN x WT
+// grid.  Here the L2-to-LDS traffic bounds the tile: 256 x 256 (64 KiB a
+// step) beats two workgroups of 256 x 128 (T = 1999, 19456 x 2560: 240
+// against 274 us); a ring of three or four 32-column stages with counted
+// waits was slower than these two of 64 (261 us).  T = 512: 40.3 -> 26.5,
+// 33.3 -> 21.3, 59.5 -> 38.6 and 89.8 -> 67.4 us on the shapes above; T =
+// 1999: 95.9 -> 69.1, 85.9 -> 56.3, 204.7 -> 120.4 and 338.9 -> 239.9 us.
+//
+// Split K.  When the tiles are too few for the CUs, K is split over
+// gridDim.y slices; slice z writes its partial sums to P[z][T][N] and
+// k_gemm_reduce (or the consumer) adds the slices in slice order.
 #include <algorithm>
 
+#include "tbq_dma.hpp"
 #include "tbq_kernels.h"
 #include "tbq_kquant.hpp"
 
@@ -38,347 +59,337 @@ namespace tbq {
 namespace {
 
 typedef _Float16 hg_f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 hg_f16x2 __attribute__((ext_vector_type(2)));
 typedef float hg_f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned hg_u32x4 __attribute__((ext_vector_type(4)));
 
-#ifndef TBQ_HG_BT
-#define TBQ_HG_BT 128
-#endif
-#ifndef TBQ_HG_BN
-#define TBQ_HG_BN 128
-#endif
-#ifndef TBQ_HG_BK
-#define TBQ_HG_BK 64
-#endif
-#ifndef TBQ_HG_WPE
-#define TBQ_HG_WPE 2
-#endif
-constexpr int HG_BN = TBQ_HG_BN, HG_BT = TBQ_HG_BT, HG_BK = TBQ_HG_BK;
-constexpr int HG_LD = HG_BK + 8;                  // LDS row stride in halves
-#ifndef TBQ_HG_WI
-#define TBQ_HG_WI 2
-#endif
-constexpr int HG_WI = TBQ_HG_WI, HG_WJ = 2;       // 32 x 32 blocks per wave along n and t
-constexpr int HG_WN = HG_BN / (32 * HG_WI);       // waves along n
-constexpr int HG_THREADS = 64 * HG_WN * (HG_BT / (32 * HG_WJ));
-constexpr int HG_ASEG = HG_BN * HG_BK / 8 / HG_THREADS;   // 16-byte A segments per thread and step
-constexpr int HG_BSEG = HG_BT * HG_BK / 8 / HG_THREADS;   // 16-byte B segments per thread and step
-constexpr int HG_SUBS = HG_BK / 32;                        // Q4_K sub-blocks per row and step
-// Q4_K tasks: whole sub-blocks (4 quant dwords) when there are no more of
-// them than threads, else halves; HG_QTPT tasks per thread and step
-constexpr int HG_QD = HG_BN * HG_SUBS >= HG_THREADS ? 4 : 2;
-constexpr int HG_QPS = 4 / HG_QD;                          // tasks per sub-block
-constexpr int HG_QTPT = HG_BN * HG_SUBS * HG_QPS / HG_THREADS;
-static_assert(HG_QTPT >= 1 && HG_QTPT * HG_THREADS == HG_BN * HG_SUBS * HG_QPS, "Q4_K tasks must divide evenly");
+// Slot swizzles: 128-byte rows of eight 16-byte segments, and 64-byte rows of
+// four.  Any 8 consecutive rows of a column read fall on 8 different 16-byte
+// bank groups of 128 bytes, any 16 on 16 of 256.
+__device__ __forceinline__ int swz8(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+__device__ __forceinline__ int swz4(int r) { return (((r >> 2) & 1) << 1) | (((r >> 1) ^ (r >> 3)) & 1); }
 
-struct HgStage {
-    _Float16 a[HG_BN * HG_LD];
-    _Float16 b[HG_BT * HG_LD];
-};
+// blockIdx.x -> tile.  Workgroup i runs on XCD i % 8, so each XCD takes a
+// contiguous range of tiles (token tiles fastest): the token tiles of a
+// weight row block meet in one L2.  -1: no tile (grid rounded up to 8).
+__device__ __forceinline__ int hg_tile(int ntile) {
+    const int per = (ntile + 7) >> 3, i = blockIdx.x >> 3, tile = (blockIdx.x & 7) * per + i;
+    return tile < ntile && i < per ? tile : -1;
+}
 
-// A Q4_K sub-block of a row, or half of one (HG_QD quant dwords).
-struct Q4Sub {
-    uint32_t hdr;      // d | dmin << 16
-    uint32_t sw, mw;   // the dwords holding this sub-block's scale and min bytes
-    uint32_t q[HG_QD]; // its quant dwords
-};
-
-__device__ __forceinline__ void q4sub_load(const uint8_t *sb, int j, int piece, Q4Sub &r) {
-    r.hdr = *reinterpret_cast<const uint32_t *>(sb);
-    // j < 4: scale byte 4 + j, min byte 8 + j; j >= 4: scale byte 8 + j,
-    // min byte 12 + j (the block's first quant dword)
-    r.sw = *reinterpret_cast<const uint32_t *>(sb + (j < 4 ? 4 : 12));
-    r.mw = *reinterpret_cast<const uint32_t *>(sb + (j < 4 ? 8 : 16));
-    const uint8_t *q = sb + 16 + 16 * j + 4 * HG_QD * piece;
-    if constexpr (HG_QD == 4) {
-        const hg_u32x4 v = *reinterpret_cast<const hg_u32x4 *>(q);
-        r.q[0] = v.x; r.q[1] = v.y; r.q[2] = v.z; r.q[3] = v.w;
-    } else {
-        const uint2 v = *reinterpret_cast<const uint2 *>(q);
-        r.q[0] = v.x; r.q[1] = v.y;
+// Accumulator register r of lane l: weight row 8(r/4) + 4(l/32) + r%4 of the
+// 32-row block, token l % 32 of the 32-token block.  Row blocks of one wave
+// start at output row nb + 32 i, its token blocks at tb + 32 j.  GLU: block 2p
+// holds gate and block 2p + 1 up rows of outputs nb + 32 p .. of F = N / 2,
+// out[t][c] = silu(g xs[t]) (u xs[t]).
+template <bool GLU, int NA, int NB>
+__device__ __forceinline__ void hg_store(const hg_f32x16 (&acc)[NA][NB], int nb, int tb, int T, int N,
+                                         float *__restrict__ out, int ldo, const float *__restrict__ xs) {
+    const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
+    static_assert(!GLU || NA % 2 == 0, "GLU pairs the wave's 32-row blocks");
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        const int t = tb + 32 * j + li;
+        if (t >= T) continue;
+        float *o = out + (long long)t * ldo;
+        float sx = 1.f;
+        if constexpr (GLU) sx = xs[t];
+#pragma unroll
+        for (int i = 0; i < (GLU ? NA / 2 : NA); i++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int n = nb + 32 * i + 8 * g + 4 * lh;
+                if (n >= (GLU ? N / 2 : N)) continue;   // rows past the end (clamped loads) are not stored
+                float r[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if constexpr (GLU) r[e] = pro_swiglu(acc[2 * i][j][4 * g + e] * sx, acc[2 * i + 1][j][4 * g + e] * sx);
+                    else r[e] = acc[i][j][4 * g + e];
+                }
+                *reinterpret_cast<float4 *>(o + n) = make_float4(r[0], r[1], r[2], r[3]);
+            }
     }
 }
 
-#ifndef TBQ_HG_EXACT
-#define TBQ_HG_EXACT 0
-#endif
-typedef _Float16 hg_f16x2 __attribute__((ext_vector_type(2)));
+template <int NW, int NB>
+struct HqLds {
+    static constexpr int ROWS = 64 * NW, TOK = 32 * NB;
+    unsigned char act[2][TOK * 128];   // two 64-column steps of the activation rows
+    unsigned char q[2][ROWS * 64];     // quants of a super-block's two 128-column halves
+    unsigned char hdr[ROWS * 16];      // its first 16 bytes: d, dmin and the scale bytes
+};
 
-// The piece's fp16 weights in element order (weights 2i, 2i+1 are the low
-// and high nibbles of quant byte i).  A nibble q becomes the fp16 number
-// 1 + q/16 by placing it in the mantissa (0x3C00 | q << 6, both nibbles of
-// a byte from one 24-bit multiply and one v_bitop3 (a & b) | c), and one
-// packed fp16 fma with (16 S, C = -16 S - M) gives 16 S (1 + q/16) + C =
-// S q - M (exact before its one rounding): 1.5 VALU per weight, with the
-// fp16 roundings of 16 S, C and the result (16 d 63 + dmin 63 must stay
-// below 65504).  TBQ_HG_EXACT instead rounds fl(fl(S q) - M) once
-// from fp32, as k_dequant_f16_q4k does.
-__device__ __forceinline__ void q4sub_f16(const Q4Sub &r, int j, hg_f16x8 (&o)[HG_QD]) {
-    const int jb = 8 * (j & 3);
-    const float S = f16_ref(r.hdr & 0xFFFFu) * (float)((r.sw >> jb) & 63);
-    const float Mn = f16_ref(r.hdr >> 16) * (float)((r.mw >> jb) & 63);
-    if constexpr (TBQ_HG_EXACT) {
-#pragma unroll
-        for (int c = 0; c < HG_QD; c++) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int qq = (int)((r.q[c] >> (8 * (i >> 1) + 4 * (i & 1))) & 15);
-                const float tt = S * (float)qq;
-                o[c][i] = (_Float16)(tt - Mn);
-            }
-        }
-    } else {
-        const _Float16 s16 = (_Float16)(16.f * S), cc = (_Float16)(-(float)s16 - Mn);
-        const hg_f16x2 S16 = {s16, s16}, C = {cc, cc};
-#pragma unroll
-        for (int c = 0; c < HG_QD; c++) {
-            unsigned w[4];
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const unsigned y = (r.q[c] >> (8 * b)) & 0xFFu;
-                const unsigned t = __builtin_amdgcn_bitop3_b32(__umul24(y, 0x40040u), 0x03C003C0u, 0x3C003C00u, 0xEA);   // (a & b) | c
-                w[b] = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(hg_f16x2, t), S16, C));
-            }
-            o[c] = __builtin_bit_cast(hg_f16x8, hg_u32x4{w[0], w[1], w[2], w[3]});
-        }
-    }
-}
+template <int WN, int WT, int NA, int NB>
+struct HfLds {
+    static constexpr int ROWS = WN * NA * 32, TOK = WT * NB * 32;
+    unsigned char s[2][(ROWS + TOK) * 128];   // two 64-column steps: weight rows, then activation rows
+};
 
 }  // namespace
 
-// AF: 0 = W fp16 rows, 1 = W Q4_K rows (reference layout).  kper = K columns
-// per slice (a multiple of HG_BK); out = C with row stride ldo (gridDim.z ==
-// 1) or the slice partials P[z][T][N] (ldo = N).
-// GLU (one slice only): W holds N = 2F rows, gate rows then up rows, and
-// out[t][c] = silu(g xs[t]) (u xs[t]) with g, u = rows c and F + c of the
-// product (xs: the row scales of X).  The A tile's 32-row blocks alternate
-// gate and up rows of the same 32 outputs (tile n-block b holds outputs
-// 64 b .. 64 b + 63), so a lane's accumulators of blocks 0 and 1 hold the
-// gate and up of the same (output, token).
-template <int AF, bool GLU = false>
-__global__ __launch_bounds__(HG_THREADS) __attribute__((amdgpu_waves_per_eu(TBQ_HG_WPE))) void k_hgemm(const void *__restrict__ Wv, const _Float16 *__restrict__ X,
-                                                         int T, int N, int K, int kper, float *__restrict__ out,
-                                                         int ldo, const float *__restrict__ xs = nullptr) {
-    static_assert(!GLU || HG_WI == 2, "GLU pairs the wave's two 32-row blocks");
-    extern __shared__ __attribute__((aligned(16))) unsigned char hg_lds[];   // two HgStage (72 KiB)
-    HgStage *st = reinterpret_cast<HgStage *>(hg_lds);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, lh = lane >> 5;
-    const int n0 = blockIdx.x * HG_BN, t0 = blockIdx.y * HG_BT;
-    const int kb = blockIdx.z * kper, ke = min(K, kb + kper), nsteps = (ke - kb) / HG_BK;
-    const int wn = (wave % HG_WN) * 32 * HG_WI, wt = (wave / HG_WN) * 32 * HG_WJ;
+// kper = K columns per slice (a multiple of 256); out = C with row stride ldo
+// (one slice) or the slice partials P[z][T][N] (ldo = N).  The weights' decode:
+// a nibble q becomes the fp16 number 1 + q/16 by placing it in the mantissa
+// (0x3C00 | q << 6, both nibbles of a byte from one 24-bit multiply and one
+// v_bitop3 (a & b) | c), and one packed fp16 fma with (16 S, C = -16 S - M)
+// gives 16 S (1 + q/16) + C = S q - M, exact before its one rounding: 1.5 VALU
+// per weight, with the fp16 roundings of 16 S, C and the result (16 d 63 +
+// dmin 63 must stay below 65504).
+template <int NW, int NB, bool GLU>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void k_hgemm_q4k(
+    const uint8_t *__restrict__ W, const _Float16 *__restrict__ X, int T, int N, int K, int nt, int ntile, int kper,
+    float *__restrict__ out, int ldo, const float *__restrict__ xs) {
+    using L = HqLds<NW, NB>;
+    constexpr int ROWS = L::ROWS, TOK = L::TOK;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char hq_lds[];
+    L *st = reinterpret_cast<L *>(hq_lds);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31,
+              lh = lane >> 5;
+    const int tile = hg_tile(ntile);
+    if (tile < 0) return;   // uniform
+    const int n0 = (tile / nt) * ROWS, t0 = (tile % nt) * TOK;
+    const int kb = blockIdx.y * kper, nsb = (min(K, kb + kper) - kb) >> 8;   // super-blocks of this slice
+    const uint32_t rb = (uint32_t)(K >> 8) * 144u;
 
-    // fp16 loaders: segment i of this thread = row tid / SPR + RSTEP i, 8
-    // halves at 8 (tid % SPR)
-    constexpr int SPR = HG_BK / 8, RSTEP = HG_THREADS / SPR;
-    const int lrow = tid / SPR, lcol = 8 * (tid % SPR);
-    const int xbytes = T * K * 2;
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void *)X, (short)0, xbytes, 0x00020000);
-    int xoff[HG_BSEG];
+    // rows of this wave's two 32-row blocks
+    const int F = N >> 1;
+    const int rbase0 = GLU ? (n0 >> 1) + 32 * wave : n0 + 64 * wave;
+    const int rbase1 = GLU ? F + rbase0 : rbase0 + 32;
+    const int rmax0 = GLU ? F - 1 : N - 1, rmax1 = N - 1;
+    // descriptor bases at the (clamped) first rows of each block
+    const int rs0 = min(rbase0, rmax0), rs1 = min(rbase1, rmax1);
+    const dma_rsrc_t w0 = dma_rsrc(W + (long long)rs0 * rb + (long long)(kb >> 8) * 144, 0x7FFFFFFFu);
+    const dma_rsrc_t w1 = dma_rsrc(W + (long long)rs1 * rb + (long long)(kb >> 8) * 144, 0x7FFFFFFFu);
+    const dma_rsrc_t xr = dma_rsrc(X + kb, 0x7FFFFFFFu);
+    // quant copies: 16 rows x 4 segments each; group g of 4 covers rows 16 g .. of the wave's 64
+    uint32_t qv[4], hv;
+    {
 #pragma unroll
-    for (int i = 0; i < HG_BSEG; i++) {
-        const int t = t0 + lrow + RSTEP * i;   // rows past T load zeros (offset beyond the buffer)
-        xoff[i] = t < T ? (t * K + kb + lcol) * 2 : xbytes;
+        for (int g = 0; g < 4; g++) {
+            const int rr = 16 * (g & 1) + (lane >> 2);   // row in its 32-row block
+            const int row = g < 2 ? min(rbase0 + rr, rmax0) - rs0 : min(rbase1 + rr, rmax1) - rs1;
+            qv[g] = (uint32_t)row * rb + 16u + 16u * ((lane & 3) ^ swz4(rr));
+        }
     }
-    // A loader (AF 0: fp16 segments as the B loader; AF 1: row, sub-block of
-    // the step's pair, piece)
-    const _Float16 *Wh = reinterpret_cast<const _Float16 *>(Wv);
-    const uint8_t *Wq = reinterpret_cast<const uint8_t *>(Wv);
-    const long long rbq = (long long)(K / 256) * 144;
-    // weight row of tile row rho (rows past N clamp to the last)
+    // header copy: lane = row (0..31 of block 0, then of block 1), all through block 0's descriptor
+    {
+        const long long row = lane < 32 ? min(rbase0 + li, rmax0) : min(rbase1 + li, rmax1);
+        hv = (uint32_t)((row - rs0) * (long long)rb);
+    }
+    // activation copies: 8 tokens x 8 segments each; the 4 NB copies of a step are dealt to the waves round-robin
+    constexpr int AC = 4 * NB, APW = (AC + NW - 1) / NW;
+    uint32_t av[APW];
+#pragma unroll
+    for (int i = 0; i < APW; i++) {
+        const int tok = 8 * (wave + NW * i) + (lane >> 3);
+        av[i] = (uint32_t)min(t0 + tok, T - 1) * (uint32_t)(K * 2) + 16u * ((lane & 7) ^ swz8(tok));
+    }
+    const uint32_t la = lds_addr(st->act[0]), lq = lds_addr(st->q[0]) + wave * 4096, lhd = lds_addr(st->hdr) + wave * 1024;
+    auto copy_act = [&](int buf, int step) {   // step: 64-column step of the slice
+#pragma unroll
+        for (int i = 0; i < APW; i++) {
+            const int c = wave + NW * i;
+            if (AC % NW == 0 || c < AC) dma16(la + buf * (TOK * 128) + c * 1024, av[i], xr, step * 128);
+        }
+    };
+    auto copy_q = [&](int half, int g, int sb) {   // group g of super-block sb's 128-column half
+        dma16(lq + half * (ROWS * 64) + g * 1024, qv[g], g < 2 ? w0 : w1, (uint32_t)(sb * 144 + half * 64));
+    };
+
+    hg_f32x16 acc[2][NB];
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) acc[b][j] = hg_f32x16{};
+
+    // LDS read offsets
+    const int fq = swz4(li), fa = swz8(li);
+    hg_u32x4 hd[2], q[2];
+    uint32_t mhi[2];
+    float d[2], dm[2];
+    hg_f16x2 S16[2], C[2];
+    hg_f16x8 a[2][2];   // [kk parity][block]
+    const unsigned char *qbase = st->q[0] + (wave * 64 + li) * 64;
+    // raw quants of step s (0..3) of the super-block whose halves are in LDS
+    auto raw = [&](int s) {
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const unsigned char *qrow = qbase + (s >> 1) * (ROWS * 64) + 32 * b * 64;
+            if (s == 0) {
+                hd[b] = *reinterpret_cast<const hg_u32x4 *>(st->hdr + (wave * 64 + 32 * b + li) * 16);
+                mhi[b] = *reinterpret_cast<const uint32_t *>(qrow + 16 * fq);
+            }
+            q[b] = *reinterpret_cast<const hg_u32x4 *>(qrow + 16 * (((s & 1) * 2 + lh) ^ fq));
+        }
+    };
+    // scale and constant of step s
+    auto scales = [&](int s) {
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            if (s == 0) {
+                d[b] = (hd[b].x & 0x7C00u) ? (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[b].x & 0xFFFFu)) : 0.f;
+                dm[b] = (hd[b].x & 0x7C000000u) ? (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[b].x >> 16)) : 0.f;
+            }
+            const uint32_t sw = s < 2 ? hd[b].y : hd[b].w, mw = s < 2 ? hd[b].z : mhi[b];
+            const int jb = 16 * (s & 1) + 8 * lh;
+            const float S = d[b] * (float)((sw >> jb) & 63), M = dm[b] * (float)((mw >> jb) & 63);
+            const _Float16 s16 = (_Float16)(16.f * S), cc = (_Float16)(-(float)s16 - M);
+            S16[b] = hg_f16x2{s16, s16};
+            C[b] = hg_f16x2{cc, cc};
+        }
+    };
+    auto frag = [&](int b, int kk) {
+        unsigned w[4];
+        const unsigned qd = kk == 0 ? q[b].x : kk == 1 ? q[b].y : kk == 2 ? q[b].z : q[b].w;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const unsigned y = (qd >> (8 * i)) & 0xFFu;
+            const unsigned t = __builtin_amdgcn_bitop3_b32(__umul24(y, 0x40040u), 0x03C003C0u, 0x3C003C00u, 0xEA);
+            w[i] = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(hg_f16x2, t), S16[b], C[b]));
+        }
+        return __builtin_bit_cast(hg_f16x8, hg_u32x4{w[0], w[1], w[2], w[3]});
+    };
+
+    copy_act(0, 0);
+    dma16(lhd, hv, w0, 0);
+#pragma unroll
+    for (int g = 0; g < 4; g++) { copy_q(0, g, 0); copy_q(1, g, 0); }
+    dma_wait_barrier();
+    raw(0);
+    scales(0);
+#pragma unroll
+    for (int b = 0; b < 2; b++) a[0][b] = frag(b, 0);
+    for (int sb = 0; sb < nsb; sb++) {
+        const int nx = min(sb + 1, nsb - 1);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            // copies of the next step (past the end: the last again, never read)
+            copy_act((s + 1) & 1, min(4 * sb + s + 1, 4 * nsb - 1));
+            if (s == 0) { copy_q(1, 2, sb); copy_q(1, 3, sb); }
+            if (s == 1) { copy_q(0, 0, nx); copy_q(0, 1, nx); }
+            if (s == 2) { copy_q(0, 2, nx); copy_q(0, 3, nx); dma16(lhd, hv, w0, (uint32_t)(nx * 144)); }
+            if (s == 3) { copy_q(1, 0, nx); copy_q(1, 1, nx); }
+            const unsigned char *ab = st->act[s & 1] + li * 128;
+            hg_f16x8 bf[2][NB];
+#pragma unroll
+            for (int j = 0; j < NB; j++) bf[0][j] = *reinterpret_cast<const hg_f16x8 *>(ab + j * 4096 + 16 * ((4 * lh) ^ fa));
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) {
+                if (kk < 3) {
+#pragma unroll
+                    for (int j = 0; j < NB; j++)
+                        bf[(kk + 1) & 1][j] = *reinterpret_cast<const hg_f16x8 *>(ab + j * 4096 + 16 * ((4 * lh + kk + 1) ^ fa));
+                    if (kk == 2) {
+                        // fragment 3 first: the raw registers are then free
+                        a[1][0] = frag(0, 3);
+                        a[1][1] = frag(1, 3);
+                        raw((s + 1) & 3);
+                    } else {
+                        a[(kk + 1) & 1][0] = frag(0, kk + 1);
+                        a[(kk + 1) & 1][1] = frag(1, kk + 1);
+                    }
+                } else {
+                    scales((s + 1) & 3);
+                    a[0][0] = frag(0, 0);
+                    a[0][1] = frag(1, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < NB; j++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+                        acc[b][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kk & 1][b], bf[kk & 1][j], acc[b][j], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2 * NB; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+                }
+            }
+            dma_wait_barrier();
+        }
+    }
+    hg_store<GLU>(acc, GLU ? rbase0 : n0 + 64 * wave, t0, T, N, out + (long long)blockIdx.y * T * N, ldo, xs);
+}
+
+// The same product for fp16 rows; GLU's 32-row blocks alternate gate and up.
+template <int WN, int WT, int NA, int NB, bool GLU>
+__global__ __launch_bounds__(64 * WN * WT) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_hgemm_f16(
+    const _Float16 *__restrict__ W, const _Float16 *__restrict__ X, int T, int N, int K, int nt, int ntile, int kper,
+    float *__restrict__ out, int ldo, const float *__restrict__ xs) {
+    using L = HfLds<WN, WT, NA, NB>;
+    constexpr int NW = WN * WT, ROWS = L::ROWS, TOK = L::TOK, SB = (ROWS + TOK) * 128;
+    constexpr int NC = (ROWS + TOK) / 8, CPW = NC / NW;   // 1 KiB copies per stage, per wave
+    static_assert(NC % NW == 0 && (ROWS / 8) % NW == 0, "");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char hf_lds[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31,
+              lh = lane >> 5;
+    const int tile = hg_tile(ntile);
+    if (tile < 0) return;   // uniform
+    const int n0 = (tile / nt) * ROWS, t0 = (tile % nt) * TOK;
+    const int kb = blockIdx.y * kper, nst = (min(K, kb + kper) - kb) >> 6;
+    const int F = N >> 1;
     auto wrow = [&](int rho) {
-        if constexpr (GLU) {
-            const int F = N / 2, b = rho >> 5;
-            return min((b & 1 ? F : 0) + (n0 >> 1) + 32 * (b >> 1) + (rho & 31), N - 1);
-        } else {
-            return min(n0 + rho, N - 1);
-        }
+        if constexpr (GLU) return min((rho & 32 ? F : 0) + min((n0 >> 1) + 32 * (rho >> 6) + (rho & 31), F - 1), N - 1);
+        else return min(n0 + rho, N - 1);
     };
-    // Q4_K task tk = tid + HG_THREADS i: row tk / (QPS SUBS), sub-block
-    // (tk / QPS) % SUBS of the step, piece tk % QPS
-    auto qtask = [&](int i, int &row, int &sub, int &pc) {
-        const int tk = tid + HG_THREADS * i;
-        row = tk / (HG_QPS * HG_SUBS);
-        sub = (tk / HG_QPS) % HG_SUBS;
-        pc = tk % HG_QPS;
+    const int base = wrow(0);
+    const dma_rsrc_t wr = dma_rsrc(W + (long long)base * K + kb, 0xFFFFFFFFu), xr = dma_rsrc(X + kb, 0x7FFFFFFFu);
+    const uint32_t l0 = lds_addr(hf_lds);
+    // 8 rows x 8 segments per copy, swizzled as the quant copies
+    uint32_t vo[CPW];
+#pragma unroll
+    for (int i = 0; i < CPW; i++) {
+        const int c = wave + NW * i, r = 8 * c + (lane >> 3);
+        const uint32_t seg = 16u * ((lane & 7) ^ swz8(r));
+        if (i < ROWS / 8 / NW) vo[i] = (uint32_t)(wrow(r) - base) * (uint32_t)(K * 2) + seg;
+        else vo[i] = (uint32_t)min(t0 + r - ROWS, T - 1) * (uint32_t)(K * 2) + seg;
+    }
+    auto copy = [&](int slot, int step) {
+#pragma unroll
+        for (int i = 0; i < CPW; i++)
+            dma16(l0 + slot * SB + (wave + NW * i) * 1024, vo[i], i < ROWS / 8 / NW ? wr : xr, step * 128);
     };
-
-    // One step's operands in registers, between their global loads and
-    // their LDS stores.  Two sets: the loads of step s + 2 are in flight
-    // while step s + 1's are stored.
-    struct Regs {
-        hg_u32x4 xr[HG_BSEG];
-        hg_u32x4 wr[HG_ASEG];
-        Q4Sub wq[HG_QTPT];
-    };
-    auto load = [&](Regs &r, int s) {
-        const int k = kb + s * HG_BK;
+    const int wn = NA * 32 * (wave % WN), wt = NB * 32 * (wave / WN);
+    const int fr = swz8(li);
+    hg_f32x16 acc[NA][NB];
 #pragma unroll
-        for (int i = 0; i < HG_BSEG; i++)
-            r.xr[i] = __builtin_bit_cast(hg_u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                       xrs, xoff[i] < xbytes ? xoff[i] + s * HG_BK * 2 : xbytes, 0, 0));
-        if constexpr (AF == 0) {
+    for (int b = 0; b < NA; b++)
 #pragma unroll
-            for (int i = 0; i < HG_ASEG; i++)
-                r.wr[i] = *reinterpret_cast<const hg_u32x4 *>(Wh + (long long)wrow(lrow + RSTEP * i) * K + k + lcol);
-        } else {
+        for (int j = 0; j < NB; j++) acc[b][j] = hg_f32x16{};
+    const int last = nst - 1;
+    copy(0, 0);
+    dma_wait_barrier();
+    const unsigned char *A = hf_lds + (wn + li) * 128, *B = hf_lds + (ROWS + wt + li) * 128;
+    for (int s0 = 0; s0 < nst; s0 += 2) {
 #pragma unroll
-            for (int i = 0; i < HG_QTPT; i++) {
-                int row, sub, pc;
-                qtask(i, row, sub, pc);
-                q4sub_load(Wq + (long long)wrow(row) * rbq + (long long)(k >> 8) * 144,
-                           ((k & 255) >> 5) + sub, pc, r.wq[i]);
+        for (int s = 0; s < 2; s++) {
+            copy(s ^ 1, min(s0 + s + 1, last));
+            const unsigned char *As = A + s * SB, *Bs = B + s * SB;
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) {
+                const int o = 16 * ((2 * kk + lh) ^ fr);
+                hg_f16x8 a[NA], b[NB];
+#pragma unroll
+                for (int i = 0; i < NA; i++) a[i] = *reinterpret_cast<const hg_f16x8 *>(As + i * 4096 + o);
+#pragma unroll
+                for (int i = 0; i < NB; i++) b[i] = *reinterpret_cast<const hg_f16x8 *>(Bs + i * 4096 + o);
+#pragma unroll
+                for (int j = 0; j < NB; j++)
+#pragma unroll
+                    for (int i = 0; i < NA; i++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[j], acc[i][j], 0, 0, 0);
             }
-        }
-    };
-    auto store = [&](const Regs &r, int buf, int s) {
+            // every read of the next k group goes out behind the first MFMAs of this one
+            __builtin_amdgcn_sched_group_barrier(0x100, NA + NB, 0);
 #pragma unroll
-        for (int i = 0; i < HG_BSEG; i++)
-            *reinterpret_cast<hg_u32x4 *>(&st[buf].b[(lrow + RSTEP * i) * HG_LD + lcol]) = r.xr[i];
-        if constexpr (AF == 0) {
-#pragma unroll
-            for (int i = 0; i < HG_ASEG; i++)
-                *reinterpret_cast<hg_u32x4 *>(&st[buf].a[(lrow + RSTEP * i) * HG_LD + lcol]) = r.wr[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < HG_QTPT; i++) {
-                int row, sub, pc;
-                qtask(i, row, sub, pc);
-                hg_f16x8 o[HG_QD];
-                q4sub_f16(r.wq[i], (((kb + s * HG_BK) & 255) >> 5) + sub, o);
-#pragma unroll
-                for (int c = 0; c < HG_QD; c++)
-                    *reinterpret_cast<hg_f16x8 *>(&st[buf].a[row * HG_LD + 32 * sub + 8 * (HG_QD * pc + c)]) = o[c];
+            for (int i = 0; i < 4 * NA * NB; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
-        }
-    };
-
-    hg_f32x16 acc[HG_WI][HG_WJ];
-#pragma unroll
-    for (int i = 0; i < HG_WI; i++)
-#pragma unroll
-        for (int jx = 0; jx < HG_WJ; jx++) acc[i][jx] = hg_f32x16{};
-#ifndef TBQ_HG_ALLREAD
-#define TBQ_HG_ALLREAD 0
-#endif
-    auto compute = [&](int buf) {
-        const _Float16 *A = st[buf].a + (wn + li) * HG_LD + 8 * lh;
-        const _Float16 *B = st[buf].b + (wt + li) * HG_LD + 8 * lh;
-        if constexpr (TBQ_HG_ALLREAD) {
-            // every operand of the step read first, then the 16 MFMAs back to back
-            hg_f16x8 a[HG_BK / 16][HG_WI], b[HG_BK / 16][HG_WJ];
-#pragma unroll
-            for (int kk = 0; kk < HG_BK / 16; kk++) {
-#pragma unroll
-                for (int i = 0; i < HG_WI; i++) a[kk][i] = *reinterpret_cast<const hg_f16x8 *>(A + 32 * i * HG_LD + 16 * kk);
-#pragma unroll
-                for (int i = 0; i < HG_WJ; i++) b[kk][i] = *reinterpret_cast<const hg_f16x8 *>(B + 32 * i * HG_LD + 16 * kk);
-            }
-#pragma unroll
-            for (int kk = 0; kk < HG_BK / 16; kk++)
-#pragma unroll
-                for (int i = 0; i < HG_WI; i++)
-#pragma unroll
-                    for (int jx = 0; jx < HG_WJ; jx++)
-                        acc[i][jx] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kk][i], b[kk][jx], acc[i][jx], 0, 0, 0);
-            return;
-        }
-#pragma unroll
-        for (int kk = 0; kk < HG_BK / 16; kk++) {
-            hg_f16x8 a[HG_WI], b[HG_WJ];
-#pragma unroll
-            for (int i = 0; i < HG_WI; i++) a[i] = *reinterpret_cast<const hg_f16x8 *>(A + 32 * i * HG_LD + 16 * kk);
-#pragma unroll
-            for (int i = 0; i < HG_WJ; i++) b[i] = *reinterpret_cast<const hg_f16x8 *>(B + 32 * i * HG_LD + 16 * kk);
-#pragma unroll
-            for (int i = 0; i < HG_WI; i++)
-#pragma unroll
-                for (int jx = 0; jx < HG_WJ; jx++)
-                    acc[i][jx] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[jx], acc[i][jx], 0, 0, 0);
-        }
-    };
-    // Loads are unconditional (steps past the end reload the last one, whose
-    // stores land in a stage no later step reads), so every path through a
-    // step issues the same loads and the compiler's wait counts stay exact.
-    const int last = nsteps - 1;
-    // sched_barrier(0) pins the order: each step's global loads go out
-    // before its MFMAs (the scheduler would otherwise sink them next to
-    // their LDS stores and expose their whole latency).
-#ifndef TBQ_HG_DEPTH
-#define TBQ_HG_DEPTH 2
-#endif
-    if constexpr (TBQ_HG_DEPTH == 1) {
-        Regs r;
-        load(r, 0);
-        store(r, 0, 0);
-        __syncthreads();
-        for (int s = 0; s < nsteps; s++) {
-            load(r, min(s + 1, last));
-            __builtin_amdgcn_sched_barrier(0);
-            compute(s & 1);
-            __builtin_amdgcn_sched_barrier(0);
-            store(r, (s + 1) & 1, min(s + 1, last));   // the other stage was last read in step s - 1
-            __syncthreads();
-        }
-    } else {
-        // two register sets: step s + 2's loads are issued at the start of
-        // step s, step s + 1's (issued a step earlier) are stored at its end
-        Regs r0, r1;
-        load(r0, 0);
-        load(r1, min(1, last));
-        store(r0, 0, 0);
-        __syncthreads();
-        for (int s = 0; s < nsteps; s += 2) {
-            load(r0, min(s + 2, last));
-            __builtin_amdgcn_sched_barrier(0);
-            compute(0);
-            __builtin_amdgcn_sched_barrier(0);
-            store(r1, 1, min(s + 1, last));   // stage 1 was last read in step s - 1
-            __syncthreads();
-            if (s + 1 >= nsteps) break;       // uniform
-            load(r1, min(s + 3, last));
-            __builtin_amdgcn_sched_barrier(0);
-            compute(1);
-            __builtin_amdgcn_sched_barrier(0);
-            store(r0, 0, min(s + 2, last));
-            __syncthreads();
+            dma_wait_barrier();
         }
     }
-    // accumulator register r of lane l: weight row 8(r/4) + 4(l/32) + r%4 of
-    // the 32-row block, token l % 32 of the 32-token block
-    if constexpr (GLU) {
-        // outputs 64 blockIdx.x + wn / 2 + 8g + 4(l/32) + r%4 of register r
-#pragma unroll
-        for (int jx = 0; jx < HG_WJ; jx++) {
-            const int t = t0 + wt + 32 * jx + li;
-            if (t >= T) continue;
-            const float sx = xs[t];
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int c = (n0 >> 1) + (wn >> 1) + 8 * g + 4 * lh;
-                if (c >= N / 2) continue;
-                float a[4];
-#pragma unroll
-                for (int r = 0; r < 4; r++) a[r] = pro_swiglu(acc[0][jx][4 * g + r] * sx, acc[1][jx][4 * g + r] * sx);
-                *reinterpret_cast<float4 *>(out + (long long)t * ldo + c) = make_float4(a[0], a[1], a[2], a[3]);
-            }
-        }
-        return;
-    }
-    float *o = out + (long long)blockIdx.z * T * N;   // z > 0 only for partials (ldo = N)
-#pragma unroll
-    for (int jx = 0; jx < HG_WJ; jx++) {
-        const int t = t0 + wt + 32 * jx + li;
-        if (t >= T) continue;
-#pragma unroll
-        for (int i = 0; i < HG_WI; i++)
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int n = n0 + wn + 32 * i + 8 * g + 4 * lh;
-                if (n >= N) continue;   // rows past N (clamped loads) are not stored
-                *reinterpret_cast<float4 *>(o + (long long)t * ldo + n) =
-                    make_float4(acc[i][jx][4 * g], acc[i][jx][4 * g + 1], acc[i][jx][4 * g + 2], acc[i][jx][4 * g + 3]);
-            }
-    }
+    hg_store<GLU>(acc, GLU ? (n0 + wn) >> 1 : n0 + wn, t0 + wt, T, N, out + (long long)blockIdx.y * T * N, ldo, xs);
 }
 
 // C[t][n] (row stride ldc) = sum over the S slices of P[z][t][n], in slice order.
@@ -407,21 +418,111 @@ int hgemm_cus() {
     return c > 0 && c < 256 ? c : 256;
 }
 
-// K slices for a T x N product: enough workgroups for one per CU (two per
-// CU measured slower: the extra partial sums cost more in k_gemm_reduce
-// than the occupancy gains), each slice at least 8 steps.
-int hgemm_slices(int T, int N, int K, int n_cu) {
-    const int tiles = ((N + HG_BN - 1) / HG_BN) * ((T + HG_BT - 1) / HG_BT);
-#ifndef TBQ_HG_SPLIT_WG
-#define TBQ_HG_SPLIT_WG 1
-#endif
-    int s = (TBQ_HG_SPLIT_WG * n_cu + tiles - 1) / tiles;
-    s = std::min(s, std::max(1, K / (8 * HG_BK)));
-    return std::max(1, std::min(s, 8));
+namespace {
+
+// Tile choice.  A launch of W workgroups runs n = ceil(W / CUs) of them on
+// its busiest CU, so its time is about
+//   c0 + steps * (n == 1 ? ke + (k1 - ke) W / CUs : n k2 / 2) + partial sums
+// in us, with steps = 64-column steps per workgroup: ke is a step of one
+// workgroup on an otherwise idle chip, k1 with one on every CU (clock and L2
+// shared), k2 a step of two on every CU.  The constants were fitted to 585
+// measured launches (every tile, T 20..1999, N 2560..19456, K 2560..9728, 1
+// to 8 slices; 4-12% rms), and the launch takes the tile and slice count with
+// the least; partial sums are priced at 0.25 us a MB written plus 0.2 read.
+struct HgTile {
+    int rows, tok;
+    float c0, ke, k1, k2;
+};
+constexpr HgTile HG_Q4K[] = {{256, 128, 3.2f, 0.635f, 1.011f, 1.502f}, {128, 128, 4.0f, 0.577f, 0.709f, 1.116f},
+                             {256, 64, 1.7f, 0.587f, 0.828f, 1.075f}, {128, 64, 3.0f, 0.466f, 0.625f, 0.764f},
+                             {128, 32, 4.1f, 0.381f, 0.451f, 0.544f}};
+constexpr HgTile HG_F16[] = {{256, 256, 2.7f, 1.106f, 1.520f, 3.559f}, {128, 128, 1.1f, 0.551f, 0.776f, 0.973f},
+                             {128, 64, 1.0f, 0.466f, 0.635f, 0.678f}};
+
+struct HgPlan {
+    int tile, S, per;   // index into the table, slices, super-blocks per slice
+};
+
+template <int NT>
+HgPlan hg_plan(const HgTile (&tab)[NT], int T, int N, int K, int n_cu, int max_slices) {
+    HgPlan best{0, 1, K / 256};
+    float bt = 1e30f;
+    for (int i = 0; i < NT; i++) {
+        const long long tiles = (long long)((N + tab[i].rows - 1) / tab[i].rows) * ((T + tab[i].tok - 1) / tab[i].tok);
+        for (int s = 1; s <= std::min(max_slices, K / 256); s++) {
+            const int per = (K / 256 + s - 1) / s, S = (K / 256 + per - 1) / per;
+            if (S != s) continue;
+            const long long W = tiles * S, n = (W + n_cu - 1) / n_cu;
+            const float steps = 4.f * per, mb = (float)T * N * 4e-6f;
+            const float step = n == 1 ? tab[i].ke + (tab[i].k1 - tab[i].ke) * W / n_cu : n * tab[i].k2 * 0.5f;
+            const float t = tab[i].c0 + steps * step + 0.25f * mb * S + (S > 1 ? 0.2f * mb * S : 0.f);
+            if (t < bt) {
+                bt = t;
+                best = {i, S, per};
+            }
+        }
+    }
+    return best;
 }
 
+constexpr int HG_MAX_SLICES = 8;   // the consumers add at most this many
+
+template <int NW, int NB, bool GLU>
+hipError_t go_q4k(const void *W, const _Float16 *X, int T, int N, int K, const HgPlan &p, float *out, int ldo,
+                  const float *xs, hipStream_t st) {
+    using L = HqLds<NW, NB>;
+    // more than 64 KiB of dynamic LDS is opted into once per kernel
+    static const hipError_t a = hipFuncSetAttribute((const void *)k_hgemm_q4k<NW, NB, GLU>,
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(L));
+    if (a != hipSuccess) return a;
+    const int nt = (T + L::TOK - 1) / L::TOK, ntile = nt * ((N + L::ROWS - 1) / L::ROWS);
+    hipLaunchKernelGGL((k_hgemm_q4k<NW, NB, GLU>), dim3((ntile + 7) / 8 * 8, p.S), dim3(64 * NW), sizeof(L), st,
+                       (const uint8_t *)W, X, T, N, K, nt, ntile, p.per * 256, out, ldo, xs);
+    return hipGetLastError();
+}
+
+template <int WN, int WT, int NA, int NB, bool GLU>
+hipError_t go_f16(const void *W, const _Float16 *X, int T, int N, int K, const HgPlan &p, float *out, int ldo,
+                  const float *xs, hipStream_t st) {
+    using L = HfLds<WN, WT, NA, NB>;
+    static const hipError_t a = hipFuncSetAttribute((const void *)k_hgemm_f16<WN, WT, NA, NB, GLU>,
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(L));
+    if (a != hipSuccess) return a;
+    const int nt = (T + L::TOK - 1) / L::TOK, ntile = nt * ((N + L::ROWS - 1) / L::ROWS);
+    hipLaunchKernelGGL((k_hgemm_f16<WN, WT, NA, NB, GLU>), dim3((ntile + 7) / 8 * 8, p.S), dim3(64 * WN * WT),
+                       sizeof(L), st, (const _Float16 *)W, X, T, N, K, nt, ntile, p.per * 256, out, ldo, xs);
+    return hipGetLastError();
+}
+
+template <bool GLU>
+hipError_t go(int wqt, const void *W, const _Float16 *X, int T, int N, int K, const HgPlan &p, float *out, int ldo,
+              const float *xs, hipStream_t st) {
+    if (wqt == QT_F16) {
+        switch (p.tile) {
+        case 0: return go_f16<4, 2, 2, 4, GLU>(W, X, T, N, K, p, out, ldo, xs, st);
+        case 1: return go_f16<2, 2, 2, 2, GLU>(W, X, T, N, K, p, out, ldo, xs, st);
+        default: return go_f16<2, 2, 2, 1, GLU>(W, X, T, N, K, p, out, ldo, xs, st);
+        }
+    }
+    switch (p.tile) {
+    case 0: return go_q4k<4, 4, GLU>(W, X, T, N, K, p, out, ldo, xs, st);
+    case 1: return go_q4k<2, 4, GLU>(W, X, T, N, K, p, out, ldo, xs, st);
+    case 2: return go_q4k<4, 2, GLU>(W, X, T, N, K, p, out, ldo, xs, st);
+    case 3: return go_q4k<2, 2, GLU>(W, X, T, N, K, p, out, ldo, xs, st);
+    default: return go_q4k<2, 1, GLU>(W, X, T, N, K, p, out, ldo, xs, st);
+    }
+}
+
+HgPlan hg_plan_for(int wqt, int T, int N, int K, int n_cu, int max_slices) {
+    return wqt == QT_F16 ? hg_plan(HG_F16, T, N, K, n_cu, max_slices) : hg_plan(HG_Q4K, T, N, K, n_cu, max_slices);
+}
+
+}  // namespace
+
+// Partial sums of a T x N product over K, whichever weight format runs it.
 size_t hgemm_partial_bytes(int T, int N, int K, int n_cu) {
-    const int s = hgemm_slices(T, N, K, n_cu);
+    const int s = std::max(hg_plan_for(QT_F16, T, N, K, n_cu, HG_MAX_SLICES).S,
+                           hg_plan_for(QT_Q4_K, T, N, K, n_cu, HG_MAX_SLICES).S);
     return s > 1 ? (size_t)s * T * N * 4 : 0;
 }
 
@@ -429,29 +530,16 @@ bool hgemm_supported(int wqt, int N, int K) {
     return (wqt == QT_F16 || wqt == QT_Q4_K) && N > 0 && N % 4 == 0 && K > 0 && K % 256 == 0;
 }
 
-// The gate/up product with SwiGLU in the epilogue (k_hgemm GLU mode): W
-// holds 2F rows (gate then up), A[T][F] (row stride lda) = silu(g xs) (u
-// xs).  hipErrorNotSupported where the product would be split over K (the
-// SwiGLU of partial sums is not defined) or F is not a multiple of 64.
+// The gate/up product with SwiGLU in the epilogue: W holds 2F rows (gate then
+// up), A[T][F] (row stride lda) = silu(g xs) (u xs).  K is never split here
+// (the SwiGLU of partial sums is not defined).  hipErrorNotSupported where F
+// is not a multiple of 64.
 hipError_t launch_hgemm_glu(int wqt, const void *W, const _Float16 *X, const float *xs, int T, int F, int K,
                             float *A, int lda, int n_cu, hipStream_t st) {
     const int N = 2 * F;
-    if (!hgemm_supported(wqt, N, K) || F % 64 || T <= 0 || (long long)T * K * 2 >= (1ll << 31) ||
-        hgemm_slices(T, N, K, n_cu) != 1)
+    if (!hgemm_supported(wqt, N, K) || F % 64 || T <= 0 || (long long)T * K * 2 >= (1ll << 31))
         return hipErrorNotSupported;
-    dim3 grid(N / HG_BN, (T + HG_BT - 1) / HG_BT, 1);
-    constexpr size_t lds = 2 * sizeof(HgStage);
-    static const hipError_t a0 =
-        hipFuncSetAttribute((const void *)k_hgemm<0, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    static const hipError_t a1 =
-        hipFuncSetAttribute((const void *)k_hgemm<1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (a0 != hipSuccess) return a0;
-    if (a1 != hipSuccess) return a1;
-    if (wqt == QT_F16)
-        hipLaunchKernelGGL((k_hgemm<0, true>), grid, dim3(HG_THREADS), lds, st, W, X, T, N, K, K, A, lda, xs);
-    else
-        hipLaunchKernelGGL((k_hgemm<1, true>), grid, dim3(HG_THREADS), lds, st, W, X, T, N, K, K, A, lda, xs);
-    return hipGetLastError();
+    return go<true>(wqt, W, X, T, N, K, hg_plan_for(wqt, T, N, K, n_cu, 1), A, lda, xs, st);
 }
 
 // wqt: QT_F16 (IEEE fp16 rows, as k_dequant_f16 writes them) or QT_Q4_K.
@@ -460,33 +548,15 @@ hipError_t launch_hgemm_glu(int wqt, const void *W, const _Float16 *X, const flo
 hipError_t launch_hgemm(int wqt, const void *W, const _Float16 *X, int T, int N, int K, float *C, int ldc,
                         float *part, int n_cu, hipStream_t st, int *nslices) {
     if (!hgemm_supported(wqt, N, K) || T <= 0 || (long long)T * K * 2 >= (1ll << 31)) return hipErrorNotSupported;
-    const int S = hgemm_slices(T, N, K, n_cu);
-    const int steps = K / HG_BK, per = (steps + S - 1) / S;
-    const int Sx = (steps + per - 1) / per;   // slices actually used
-    dim3 grid((N + HG_BN - 1) / HG_BN, (T + HG_BT - 1) / HG_BT, Sx);
-    float *out = Sx > 1 ? part : C;
-    if (Sx > 1 && !part) return hipErrorInvalidValue;
-    if (nslices && Sx > 1 && ldc != N) return hipErrorInvalidValue;   // slices are packed at row stride N
-    // more than 64 KiB of dynamic LDS is opted into once per kernel
-    constexpr size_t lds = 2 * sizeof(HgStage);
-    static const hipError_t a0 =
-        hipFuncSetAttribute((const void *)k_hgemm<0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    static const hipError_t a1 =
-        hipFuncSetAttribute((const void *)k_hgemm<1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (a0 != hipSuccess) return a0;
-    if (a1 != hipSuccess) return a1;
-    if (wqt == QT_F16)
-        hipLaunchKernelGGL(k_hgemm<0>, grid, dim3(HG_THREADS), lds, st, W, X, T, N, K, per * HG_BK, out,
-                           Sx > 1 ? N : ldc);
-    else
-        hipLaunchKernelGGL(k_hgemm<1>, grid, dim3(HG_THREADS), lds, st, W, X, T, N, K, per * HG_BK, out,
-                           Sx > 1 ? N : ldc);
-    hipError_t err = hipGetLastError();
-    if (nslices) *nslices = Sx;
-    if (err != hipSuccess || Sx == 1 || nslices) return err;
+    const HgPlan p = hg_plan_for(wqt, T, N, K, n_cu, HG_MAX_SLICES);
+    if (p.S > 1 && !part) return hipErrorInvalidValue;
+    if (nslices && p.S > 1 && ldc != N) return hipErrorInvalidValue;   // slices are packed at row stride N
+    const hipError_t err = go<false>(wqt, W, X, T, N, K, p, p.S > 1 ? part : C, p.S > 1 ? N : ldc, nullptr, st);
+    if (nslices) *nslices = p.S;
+    if (err != hipSuccess || p.S == 1 || nslices) return err;
     const long long n4 = (long long)T * N / 4;
     const int g = (int)std::min<long long>((n4 + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_gemm_reduce, dim3(g), dim3(256), 0, st, part, Sx, T, N, C, ldc);
+    hipLaunchKernelGGL(k_gemm_reduce, dim3(g), dim3(256), 0, st, part, p.S, T, N, C, ldc);
     return hipGetLastError();
 }
 
