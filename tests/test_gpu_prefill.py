@@ -115,6 +115,36 @@ def test_prefill_long_context_many_splits(oracle, G):
     assert rel_l2(kcg[:, :, P:P + 100], ref.kc[:, :, P:P + 100]) <= PREFILL_TOL
 
 
+@pytest.mark.parametrize("D,G,P,T", [(64, 1, 0, 64), (64, 2, 63, 2), (64, 8, 64, 65), (128, 4, 127, 33), (128, 1, 1, 63),
+                                     (128, 8, 200, 17), (128, 2, 690, 131)])
+def test_prefill_attention_edges(oracle, D, G, P, T):
+    """Query blocks and position chunks on either side of their 64-position
+    edges, one and several splits, after P cached N(0,1) K/V rows: the second
+    layer's K/V rows of every prompt position depend on its own attention."""
+    import torch
+    from oracle.dense import DenseOracle
+    from trailblaze_amd.dense import SyntheticDense
+    cfg = _cfg(n_layers=2, n_heads=8, n_kv_heads=8 // G, head_dim=D, max_ctx=P + T + 5, vocab=256)
+    m = SyntheticDense(cfg, 50, keep_host=True)
+    ref = DenseOracle(oracle, cfg, m.host)
+    rng = np.random.default_rng(P + T)
+    for dev, cache in ((m.k_cache, ref.kc), (m.v_cache, ref.vc)):
+        cache[:, :, :P] = rng.standard_normal(cache[:, :, :P].shape).astype(np.float32)
+        dev.copy_(torch.from_numpy(cache.astype(np.float32)))
+    toks = rng.integers(0, 256, T)
+    logits = torch.empty(cfg.vocab, dtype=torch.float32, device="cuda")
+    print("prefill attention edges", D, G, P, T, flush=True)
+    m.prefill(toks, P, logits)
+    for i, tok in enumerate(toks):
+        want = ref.decode(tok, P + i)
+    assert rel_l2(host(logits), want) <= PREFILL_TOL
+    for dev, cache in ((m.k_cache, ref.kc), (m.v_cache, ref.vc)):
+        got = host(dev).reshape(cache.shape)
+        for p in range(P, P + T):
+            assert rel_l2(got[1, :, p], cache[1, :, p]) <= PREFILL_TOL, p
+        assert np.array_equal(got[:, :, :P], cache[:, :, :P].astype(np.float32)) and not np.any(got[:, :, P + T:])
+
+
 @pytest.mark.parametrize("ql,qe", [(fm.Q8_0, fm.Q6_K), (fm.Q5_K, fm.Q8_0), (fm.GGML | fm.Q4_K, fm.GGML | fm.Q6_K),
                                    (fm.GGML | fm.Q3_K, fm.Q4_K)])
 def test_prefill_other_formats(oracle, ql, qe):

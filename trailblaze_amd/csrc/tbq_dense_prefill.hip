@@ -12,6 +12,7 @@
 //   GEMM             qkv = h16 Wqkv^T             fp16 MFMA, fp32 acc
 //   k_pf_qk          per (token, head): QK-norm + RoPE of q (to qb) and k;
 //                    k and v rows written to the cache at pos0 + t
+//   k_pf_kv16        the layer's cache rows as fp16, V transposed
 //   k_pf_attn        causal GQA attention over cache positions 0 .. pos on
 //                    fp16 MFMA, online softmax, key ranges split over
 //                    workgroups
@@ -34,6 +35,7 @@
 
 #include <algorithm>
 
+#include "tbq_dma.hpp"
 #include "tbq_kernels.h"
 #include "tbq_device.hpp"
 #include "../../include/tbq.h"
@@ -41,7 +43,9 @@
 namespace tbq {
 
 constexpr int PN_THREADS = 256;
-constexpr int PA_KF = 32;     // split sizes are multiples of this many positions
+
+// Slot swizzle of 128-byte LDS rows (eight 16-byte segments).
+__device__ __forceinline__ int pf_swz8(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
 __device__ __forceinline__ float pf_block_sum(float v, float *red) {
     v = group_sum<64>(v);
@@ -188,71 +192,110 @@ __global__ __launch_bounds__(64) void k_pf_rope(int pos0, float theta, int D, fl
     }
 }
 
-// Head vector (one wave; lane l holds elements l and l + 64, or l for
-// D = 64): RMSNorm with the head's weights, then rotate-half RoPE with the
-// position's table row rc (cos | sin).
+// grid = (T, ceil((NQ + NKV) / heads per workgroup)); D / 4 lanes per head,
+// lane l of them holding elements 2l, 2l + 1 and D/2 + 2l, D/2 + 2l + 1 (the
+// rotation's pairs are in one lane), four waves.  qkv row t times rs[t] is the
+// true row.  Head hh < NQ: q head hh of token t, normed, rotated and scaled by
+// log2(e) / sqrt(D) (the attention's softmax is in powers of two) into qb as
+// fp16, the attention's operand; else k head hh - NQ, normed and rotated, and
+// the matching v head, written to the layer's cache rows pos0 + t.  One wave
+// per head in a workgroup of its own was bound by the workgroups' launch: T =
+// 1999, 40 heads of 128: 22.0 -> 16.2 us.
+constexpr int PQ_THREADS = 256;
 template <int D>
-__device__ __forceinline__ void pf_norm_rope(float (&x)[D / 64], const float *__restrict__ w,
-                                             const float *__restrict__ rc, float eps) {
-    const int lane = threadIdx.x & 63;
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < D / 64; i++) ss += x[i] * x[i];
-    ss = group_sum<64>(ss);
-    const float r = 1.0f / sqrtf(ss / (float)D + eps);
-#pragma unroll
-    for (int i = 0; i < D / 64; i++) x[i] = x[i] * r * w[lane + 64 * i];
-    const int j = lane % (D / 2);
-    const float cs = rc[j], sn = rc[D / 2 + j];
-    if constexpr (D == 128) {
-        const float a = x[0], b = x[1];
-        x[0] = a * cs - b * sn;
-        x[1] = a * sn + b * cs;
-    } else {
-        const float other = __shfl_xor(x[0], 32);
-        x[0] = lane < 32 ? x[0] * cs - other * sn : other * sn + x[0] * cs;
-    }
-}
-
-// grid = (T, NQ + NKV), one wave; qkv row t times rs[t] is the true row.
-// Head hh < NQ: q head hh of token t,
-// normed, rotated and scaled by 1/sqrt(D) into qb[t][hh]; else k head
-// hh - NQ, normed and rotated, and the matching v head, written to the
-// layer's cache rows pos0 + t.
-template <int D>
-__global__ __launch_bounds__(64) void k_pf_qk(const float *__restrict__ qkv, int nq, long long qstride,
-                                              const float *__restrict__ rs, const float *__restrict__ qn,
-                                              const float *__restrict__ kn, int NQ, int NKV, int pos0,
-                                              const float *__restrict__ rope, float eps, float *__restrict__ kc,
-                                              float *__restrict__ vc, int max_ctx, float *__restrict__ qb) {
-    const int t = blockIdx.x, hh = blockIdx.y, lane = threadIdx.x;
+__global__ __launch_bounds__(PQ_THREADS) void k_pf_qk(const float *__restrict__ qkv, int nq, long long qstride,
+                                                      const float *__restrict__ rs, const float *__restrict__ qn,
+                                                      const float *__restrict__ kn, int NQ, int NKV, int pos0,
+                                                      const float *__restrict__ rope, float eps, float *__restrict__ kc,
+                                                      float *__restrict__ vc, int max_ctx, _Float16 *__restrict__ qb) {
+    constexpr int LPH = D / 4;
+    const int t = blockIdx.x, l = threadIdx.x % LPH, h0 = blockIdx.y * (PQ_THREADS / LPH) + threadIdx.x / LPH;
+    const bool on = h0 < NQ + NKV;
+    const int hh = on ? h0 : NQ + NKV - 1;   // lanes past the last head repeat it and store nothing
     const int QKVR = (NQ + 2 * NKV) * D, pos = pos0 + t;
     const float sc = rs[t];   // row t of qkv is scaled by 1 / rs[t]
     // qkv may be a GEMM's nq split-K slices (slice z at qkv + z * qstride),
     // added in slice order
     auto elem = [&](long long off) {
-        float a = qkv[off];
-        for (int z = 1; z < nq; z++) a = a + qkv[off + z * qstride];
-        return a;
+        float2 a = *reinterpret_cast<const float2 *>(qkv + off);
+        for (int z = 1; z < nq; z++) {
+            const float2 b = *reinterpret_cast<const float2 *>(qkv + off + z * qstride);
+            a.x = a.x + b.x;
+            a.y = a.y + b.y;
+        }
+        return make_float2(a.x * sc, a.y * sc);
     };
-    const long long src = (long long)t * QKVR + hh * D;
-    float x[D / 64];
-#pragma unroll
-    for (int i = 0; i < D / 64; i++) x[i] = elem(src + lane + 64 * i) * sc;
-    pf_norm_rope<D>(x, hh < NQ ? qn : kn, rope + (long long)t * D, eps);
+    const long long src = (long long)t * QKVR + hh * D + 2 * l;
+    float2 x = elem(src), y = elem(src + D / 2);
+    const float *w = (hh < NQ ? qn : kn) + 2 * l;
+    const float2 cs = *reinterpret_cast<const float2 *>(rope + (long long)t * D + 2 * l);
+    const float2 sn = *reinterpret_cast<const float2 *>(rope + (long long)t * D + D / 2 + 2 * l);
+    const float ss = group_sum<LPH>(x.x * x.x + x.y * x.y + y.x * y.x + y.y * y.y);
+    const float r = 1.0f / sqrtf(ss / (float)D + eps);
+    x.x = x.x * r * w[0];
+    x.y = x.y * r * w[1];
+    y.x = y.x * r * w[D / 2];
+    y.y = y.y * r * w[D / 2 + 1];
+    const float2 a = make_float2(x.x * cs.x - y.x * sn.x, x.y * cs.y - y.y * sn.y);
+    const float2 b = make_float2(x.x * sn.x + y.x * cs.x, x.y * sn.y + y.y * cs.y);
+    if (!on) return;
     if (hh < NQ) {
-        const float scale = 1.0f / sqrtf((float)D);
-#pragma unroll
-        for (int i = 0; i < D / 64; i++) qb[((long long)t * NQ + hh) * D + lane + 64 * i] = x[i] * scale;
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        const float scale = 1.4426950408889634f / sqrtf((float)D);
+        h2 *q = reinterpret_cast<h2 *>(qb + ((long long)t * NQ + hh) * D + 2 * l);
+        q[0] = h2{(_Float16)(a.x * scale), (_Float16)(a.y * scale)};
+        q[D / 4] = h2{(_Float16)(b.x * scale), (_Float16)(b.y * scale)};
     } else {
         const int kvh = hh - NQ;
-        const long long row = ((long long)kvh * max_ctx + pos) * D;
-        const long long vsrc = (long long)t * QKVR + (NQ + NKV + kvh) * D;
+        const long long row = ((long long)kvh * max_ctx + pos) * D + 2 * l;
+        const long long vsrc = (long long)t * QKVR + (NQ + NKV + kvh) * D + 2 * l;
+        *reinterpret_cast<float2 *>(kc + row) = a;
+        *reinterpret_cast<float2 *>(kc + row + D / 2) = b;
+        *reinterpret_cast<float2 *>(vc + row) = elem(vsrc);
+        *reinterpret_cast<float2 *>(vc + row + D / 2) = elem(vsrc + D / 2);
+    }
+}
+
+// The layer's cache rows 0 .. kmax - 1 as the attention's fp16 operands, once
+// per layer instead of once per query block: k16[kvh][pos][D], and vt[kvh][D]
+// [pos], V transposed, its positions inside each group of 16 in the order 0-3,
+// 8-11, 4-7, 12-15 (the order in which the probabilities sit in the
+// accumulators).  Both have cp positions per head; rows past kmax up to the
+// next multiple of 64 are zeros (their probabilities are 0, and 0 times a
+// stale infinity is not).  grid = (NKV, ceil(kmax / 64)).
+constexpr int PC_KC = 64;
+template <int D>
+__global__ __launch_bounds__(256) void k_pf_kv16(const float *__restrict__ kc, const float *__restrict__ vc,
+                                                 int max_ctx, int kmax, int cp, _Float16 *__restrict__ k16,
+                                                 _Float16 *__restrict__ vt) {
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    const int kvh = blockIdx.x, c0 = blockIdx.y * PC_KC, tid = threadIdx.x;
+    const float *kb = kc + (long long)kvh * max_ctx * D, *vb = vc + (long long)kvh * max_ctx * D;
 #pragma unroll
-        for (int i = 0; i < D / 64; i++) {
-            kc[row + lane + 64 * i] = x[i];
-            vc[row + lane + 64 * i] = elem(vsrc + lane + 64 * i) * sc;
-        }
+    for (int i = 0; i < PC_KC * D / 4 / 256; i++) {
+        const int f = tid + 256 * i, key = f / (D / 4), c4 = f % (D / 4), p = c0 + key;
+        float4 v = *reinterpret_cast<const float4 *>(kb + (long long)min(p, kmax - 1) * D + 4 * c4);
+        if (p >= kmax) v = make_float4(0.f, 0.f, 0.f, 0.f);
+        *reinterpret_cast<h4 *>(k16 + ((long long)kvh * cp + p) * D + 4 * c4) =
+            h4{(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+    }
+    // thread = dim tid % D of NP positions
+    constexpr int NP = PC_KC * D / 256;
+    const int d = tid % D, p0 = c0 + NP * (tid / D);
+    float v[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        v[i] = vb[(long long)min(p0 + i, kmax - 1) * D + d];
+        if (p0 + i >= kmax) v[i] = 0.f;
+    }
+    _Float16 *dst = vt + ((long long)kvh * D + d) * cp + p0;
+#pragma unroll
+    for (int i = 0; i < NP / 8; i++) {
+        h8 o;
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = (_Float16)v[16 * (i / 2) + 8 * (e / 4) + 4 * (i % 2) + e % 4];
+        *reinterpret_cast<h8 *>(dst + 8 * i) = o;
     }
 }
 
@@ -317,124 +360,163 @@ __global__ __launch_bounds__(256) void k_pf_scale_row(const float *__restrict__ 
 }
 
 // Causal attention on MFMA (v_mfma_f32_32x32x16_f16, fp16 operands, fp32
-// accumulate).  grid = (NKV, ceil(T / QB), nsplit), 4 waves: the workgroup
-// owns QB = 128 / G tokens x the G query heads of kv head kvh = 128 query
-// columns, 32 per wave (query c of a wave: token c / G, head c % G).  Cache
-// positions pass through LDS 32 at a time in fp16: K as [position][dim],
-// V transposed as [dim][position].  Per chunk a wave forms S^T = K Q^T (32
-// positions x its 32 queries), so a lane holds 16 scores of one query:
-// lane l, register r: query l % 32, position 8(r/4) + 4(l/32) + r%4.  The
-// query's max and denominator need one exchange with lane l ^ 32.  The
-// probabilities, rounded to fp16, are already the B operand of
-// O^T += V^T P^T when the 16 positions of a step are taken in the order
-// k-slot 8h + i <-> position 8(i/4) + 4h + i%4 (h = l / 32), which V^T's A
-// operand follows; O^T's accumulators hold dims 32j + 8(r/4) + 4h + r%4
-// of the lane's query.  Online softmax over chunks; positions past a
-// query's own are masked.
+// accumulate).  grid = (NKV, ceil(T / QB), nsplit), WV waves: the workgroup
+// owns QB = 32 WV / G tokens x the G query heads of kv head kvh = 32 WV query
+// columns, 32 per wave (query c of a wave: token c / G, head c % G).  K and V
+// pass through LDS 64 positions at a time in fp16 (k_pf_kv16's form), copied
+// directly from global memory a chunk ahead into one of two stages; the
+// 16-byte segments of a row are XOR-swizzled by the copies' source addresses.
+// Per chunk a wave forms S^T = K Q^T (64 positions x its 32 queries), so a
+// lane holds 32 scores of one query: lane l, block b, register r: query l %
+// 32, position 32 b + 8(r/4) + 4(l/32) + r%4.  The query's max needs one
+// exchange with lane l ^ 32.  The probabilities, rounded to fp16, are already
+// the B operand of O^T += V^T P^T when the 16 positions of a step are taken in
+// the order k-slot 8h + i <-> position 8(i/4) + 4h + i%4 (h = l / 32), in which
+// vt stores them; O^T's accumulators hold dims 32j + 8(r/4) + 4h + r%4 of the
+// lane's query.
+//
+// Online softmax in powers of two.  The running max m is raised, and the
+// output rescaled, only when some query of the wave exceeds its m by more than
+// 8: probabilities stay below 2^8 and the rescaling (half of the chunk's VALU
+// work at D = 128) is rare after the first chunks.  Only chunks that reach past
+// a query's own position are masked.  m starts at a large negative number
+// rather than -inf, so a chunk without a visible position gives p = 0.
+//
+// Workgroup i runs on XCD i % 8: with kv heads along x an XCD's L2 holds the K
+// and V of NKV / 8 heads.  The query blocks that see most positions start
+// first.
 //
 // Key splits: split z takes positions [z ks, (z + 1) ks) (ks a multiple of
-// PA_KF), so the heavy blocks of a causal prompt (whose queries see every
-// earlier position) spread over several workgroups.  With nsplit > 1 each
-// writes its queries' unnormalised output, running max and denominator to
-// the record part[(row * nsplit + z) * pf_rec(D)] (D outputs, max,
-// denominator, two floats of padding so that every record starts 16-byte
-// aligned for the float4 stores), and k_pf_attn_rows merges the splits a
-// row reaches.
-constexpr int PM_THREADS = 256, PM_Q = 128, PM_KC = 32;
+// 64), so the heavy blocks of a causal prompt (whose queries see every earlier
+// position) spread over several workgroups.  With nsplit > 1 each writes its
+// queries' unnormalised output, running max and denominator to the record
+// part[(row * nsplit + z) * pf_rec(D)] (D outputs, max, denominator, two
+// floats of padding so that every record starts 16-byte aligned for the float4
+// stores), and k_pf_attn_rows merges the splits a row reaches.
+//
+// Bound by the softmax's VALU work beside the MFMAs.  T = 1999 after 1024
+// cached positions, 32 / 8 heads of 128: 293 -> 93 us (0.7 PFLOP/s), T = 512
+// from position 0: 25.2 -> 14.6 us, against converting the fp32 cache rows in
+// every query block, 32 positions at a time between two barriers (and 5 to 11
+// us of k_pf_kv16, which that form did without).  Two workgroups of 4 waves
+// per CU; 8 waves (half the copies, one workgroup per CU) were 1% slower on the
+// whole prefill.
+constexpr int PM_KC = PC_KC;
 __host__ __device__ constexpr int pf_rec(int D) { return D + 4; }
 typedef _Float16 pm_h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 pm_h4 __attribute__((ext_vector_type(4)));
 typedef float pm_f16 __attribute__((ext_vector_type(16)));
 
-template <int D, int G>
-__global__ __launch_bounds__(PM_THREADS) void k_pf_attn(const float *__restrict__ qb, const float *__restrict__ kc,
-                                                        const float *__restrict__ vc, int T, int pos0, int NQ,
-                                                        int max_ctx, int ks, int nsplit, float *__restrict__ part,
-                                                        float *__restrict__ out) {
-    constexpr int QB = PM_Q / G, KLD = D + 8, VLD = PM_KC + 8, NT = D / 32, NS = D / 16;
-    __shared__ __attribute__((aligned(16))) _Float16 Ks[PM_KC * KLD];
-    __shared__ __attribute__((aligned(16))) _Float16 Vt[D * VLD];
-    const int kvh = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, h = lane >> 5;
+template <int D>
+struct PmLds {
+    unsigned char k[2][PM_KC * D * 2];   // [position][dim]
+    unsigned char v[2][D * PM_KC * 2];   // [dim][position]
+};
+
+template <int D, int G, int WV>
+__global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_pf_attn(
+    const _Float16 *__restrict__ qb, const _Float16 *__restrict__ k16, const _Float16 *__restrict__ vt, int T, int pos0,
+    int NQ, int cp, int ks, int nsplit, float *__restrict__ part, float *__restrict__ out) {
+    constexpr int QB = 32 * WV / G, NT = D / 32, NS = D / 16, KSEG = D / 8;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char pm_lds[];
+    PmLds<D> *st = reinterpret_cast<PmLds<D> *>(pm_lds);
+    const int kvh = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63,
+              li = lane & 31, h = lane >> 5;
+    const int yb = gridDim.y - 1 - blockIdx.y;
     const int qc = wave * 32 + li, g = qc % G;
-    const int t = blockIdx.y * QB + qc / G;
-    const int tt = t < T ? t : T - 1;
-    const int qpos = pos0 + tt;
-    const int tend = min(T, (int)(blockIdx.y + 1) * QB);
-    const int k0 = blockIdx.z * ks;                  // this split's positions k0 .. kend - 1
-    const int kend = min(pos0 + tend, k0 + ks);
+    const int t = yb * QB + qc / G;
+    const int tt = min(t, T - 1), qpos = pos0 + tt;
+    const int k0 = blockIdx.z * ks;                              // this split's positions k0 .. kend - 1
+    const int kend = min(pos0 + min(T, (yb + 1) * QB), k0 + ks);
     if (k0 >= kend) return;   // no position of the split is seen by the block (uniform)
+    // the wave's first and last query positions
+    const int qlo = pos0 + min(yb * QB + wave * 32 / G, T - 1), qhi = pos0 + min(yb * QB + (wave * 32 + 31) / G, T - 1);
     // Q^T's B fragments: dim step s, lane half h supplies dims 16s + 8h .. + 8
     pm_h8 qf[NS];
-    const float *qsrc = qb + ((long long)tt * NQ + kvh * G + g) * D;
+    const _Float16 *qsrc = qb + ((long long)tt * NQ + kvh * G + g) * D + 8 * h;
 #pragma unroll
-    for (int s = 0; s < NS; s++)
+    for (int s = 0; s < NS; s++) qf[s] = *reinterpret_cast<const pm_h8 *>(qsrc + 16 * s);
+    // copies: KC of K rows (KSEG segments), VC of V rows (8 segments), dealt to the waves
+    constexpr int NC = PM_KC * KSEG / 64, CPW = NC / WV;
+    static_assert(NC % WV == 0 && D * 8 / 64 == NC, "K and V take the same number of copies");
+    const dma_rsrc_t kr = dma_rsrc(k16 + (long long)kvh * cp * D, (uint32_t)((long long)cp * D * 2));
+    const dma_rsrc_t vr = dma_rsrc(vt + (long long)kvh * cp * D, (uint32_t)((long long)cp * D * 2));
+    auto kswz = [](int row) { return KSEG == 16 ? row & 15 : pf_swz8(row); };
+    uint32_t ko[CPW], vo[CPW];
 #pragma unroll
-        for (int c = 0; c < 8; c++) qf[s][c] = (_Float16)qsrc[16 * s + 8 * h + c];
+    for (int i = 0; i < CPW; i++) {
+        const int c = wave + WV * i;
+        const int kr_ = c * (64 / KSEG) + lane / KSEG, vr_ = 8 * c + (lane >> 3);
+        ko[i] = (uint32_t)(kr_ * D * 2 + 16 * ((lane % KSEG) ^ kswz(kr_)));
+        vo[i] = (uint32_t)vr_ * (uint32_t)(cp * 2) + 16u * ((lane & 7) ^ pf_swz8(vr_));
+    }
+    const uint32_t lk = lds_addr(st->k[0]), lv = lds_addr(st->v[0]);
+    auto copy = [&](int buf, int c0) {
+#pragma unroll
+        for (int i = 0; i < CPW; i++) {
+            dma16(lk + buf * (PM_KC * D * 2) + (wave + WV * i) * 1024, ko[i], kr, (uint32_t)c0 * (D * 2));
+            dma16(lv + buf * (PM_KC * D * 2) + (wave + WV * i) * 1024, vo[i], vr, (uint32_t)c0 * 2);
+        }
+    };
     pm_f16 o[NT];
 #pragma unroll
     for (int j = 0; j < NT; j++) o[j] = pm_f16{};
-    float m = -__builtin_huge_valf(), l = 0.f;
-    const float *kb = kc + (long long)kvh * max_ctx * D;
-    const float *vb = vc + (long long)kvh * max_ctx * D;
-    for (int c0 = k0; c0 < kend; c0 += PM_KC) {
-        __syncthreads();   // the previous chunk is no longer read
-        for (int f = tid; f < PM_KC * D / 4; f += PM_THREADS) {
-            const int key = f / (D / 4), c4 = f % (D / 4);
-            const long long p = min(c0 + key, kend - 1);
-            const float4 kv = *reinterpret_cast<const float4 *>(kb + p * D + 4 * c4);
-            const float4 vv = *reinterpret_cast<const float4 *>(vb + p * D + 4 * c4);
-            *reinterpret_cast<pm_h4 *>(&Ks[key * KLD + 4 * c4]) =
-                pm_h4{(_Float16)kv.x, (_Float16)kv.y, (_Float16)kv.z, (_Float16)kv.w};
-            Vt[(4 * c4) * VLD + key] = (_Float16)vv.x;
-            Vt[(4 * c4 + 1) * VLD + key] = (_Float16)vv.y;
-            Vt[(4 * c4 + 2) * VLD + key] = (_Float16)vv.z;
-            Vt[(4 * c4 + 3) * VLD + key] = (_Float16)vv.w;
-        }
-        __syncthreads();
-        pm_f16 sc = pm_f16{};
+    float m = -1e30f, l = 0.f;
+    const int ksw = kswz(li), vsw = pf_swz8(li);
+    copy(0, k0);
+    dma_wait_barrier();
+    int buf = 0;
+    for (int c0 = k0; c0 < kend; c0 += PM_KC, buf ^= 1) {
+        copy(buf ^ 1, c0 + PM_KC < kend ? c0 + PM_KC : c0);   // the last chunk copies itself again, never read
+        if (c0 <= qhi) {   // uniform per wave
+            const unsigned char *Kb = st->k[buf] + li * (D * 2), *Vb = st->v[buf] + li * (PM_KC * 2);
+            pm_f16 sc[2] = {pm_f16{}, pm_f16{}};
 #pragma unroll
-        for (int s = 0; s < NS; s++) {
-            const pm_h8 a = *reinterpret_cast<const pm_h8 *>(&Ks[li * KLD + 16 * s + 8 * h]);
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[s], sc, 0, 0, 0);
-        }
-        float mx = -__builtin_huge_valf();
+            for (int s = 0; s < NS; s++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int key = c0 + 8 * (r / 4) + 4 * h + r % 4;
-            const float v = key <= qpos ? sc[r] : -__builtin_huge_valf();
-            sc[r] = v;
-            mx = fmaxf(mx, v);
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        // a query that has seen no position yet keeps m = -inf, l = 0, o = 0
-        const float mn = fmaxf(m, mx);
-        const float corr = m == -__builtin_huge_valf() ? 0.f : __expf(m - mn);
-        float ls = 0.f;
+                for (int b = 0; b < 2; b++) {
+                    const pm_h8 a = *reinterpret_cast<const pm_h8 *>(Kb + b * (32 * D * 2) + 16 * ((2 * s + h) ^ ksw));
+                    sc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[s], sc[b], 0, 0, 0);
+                }
+            if (c0 + PM_KC - 1 > qlo) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const float p = sc[r] == -__builtin_huge_valf() ? 0.f : __expf(sc[r] - mn);
-            sc[r] = p;
-            ls += p;
-        }
-        ls += __shfl_xor(ls, 32);
-        l = l * corr + ls;
-        m = mn;
-        pm_h8 pb[2];
+                for (int b = 0; b < 2; b++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) pb[r / 8][r % 8] = (_Float16)sc[r];
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            o[j] *= corr;
-#pragma unroll
-            for (int k = 0; k < 2; k++) {
-                const _Float16 *vr = &Vt[(32 * j + li) * VLD + 16 * k + 4 * h];
-                const pm_h4 lo = *reinterpret_cast<const pm_h4 *>(vr);
-                const pm_h4 hi = *reinterpret_cast<const pm_h4 *>(vr + 8);
-                const pm_h8 a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[k], o[j], 0, 0, 0);
+                    for (int r = 0; r < 16; r++) {
+                        const int key = c0 + 32 * b + 8 * (r / 4) + 4 * h + r % 4;
+                        sc[b][r] = key <= qpos ? sc[b][r] : -__builtin_huge_valf();
+                    }
             }
+            float mx = sc[0][0];
+#pragma unroll
+            for (int r = 1; r < 32; r++) mx = fmaxf(mx, sc[r / 16][r % 16]);
+            mx = swap32_max(mx);
+            if (__builtin_amdgcn_ballot_w64(mx > m + 8.f)) {
+                const float mn = fmaxf(m, mx), corr = __builtin_amdgcn_exp2f(m - mn);
+                m = mn;
+                l *= corr;
+#pragma unroll
+                for (int j = 0; j < NT; j++) o[j] *= corr;
+            }
+            pm_h8 pb[4];
+            float ls = 0.f;
+#pragma unroll
+            for (int r = 0; r < 32; r++) {
+                const float p = __builtin_amdgcn_exp2f(sc[r / 16][r % 16] - m);
+                ls += p;
+                pb[r / 8][r % 8] = (_Float16)p;
+            }
+            l += ls;   // this half's positions; the halves are added at the end
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const pm_h8 a = *reinterpret_cast<const pm_h8 *>(Vb + j * (32 * PM_KC * 2) + 16 * ((2 * u + h) ^ vsw));
+                    o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[u], o[j], 0, 0, 0);
+                }
         }
+        dma_wait_barrier();
     }
+    l = swap32_sum(l);
     if (t >= T) return;
     const long long row = (long long)t * NQ + kvh * G + g;
     const float inv = nsplit == 1 ? 1.0f / l : 1.f;
@@ -453,14 +535,14 @@ __global__ __launch_bounds__(PM_THREADS) void k_pf_attn(const float *__restrict_
 
 // Attention rows to the o GEMM's operand in one pass: row t (all NQ heads,
 // QD = NQ * D floats) is the attention output -- att[t] itself when the
-// keys were not split, else the merge of the splits z <= (pos0 + t) / ks
-// with e^(m_z - M) weights and fmaf sums in z order -- and is written as fp16 scaled by
+// keys were not split, else the merge of the splits z <= (pos0 + t) / ks (at
+// most NZ) with 2^(m_z - M) weights and fmaf sums in z order -- and is written as fp16 scaled by
 // the power of two that puts its max |value| in [2^14, 2^15), with
 // hinv[t] = the inverse scale (k_rows_f16's arithmetic).  grid = T,
 // PN_THREADS threads, up to PR_V float4 of the row per thread (QD <= 8192).
 constexpr int PR_V = 8;
-constexpr int PA_PREF_KS = 128, PA_MAX_SPLIT = 8;   // preferred split size, most splits
-template <int D>
+constexpr int PA_MIN_KS = 128, PA_MAX_SPLIT = 8;   // smallest split size, most splits
+template <int D, int NZ>
 __global__ __launch_bounds__(PN_THREADS) void k_pf_attn_rows(const float *__restrict__ part,
                                                              const float *__restrict__ att, int NQ, int pos0, int ks,
                                                              int nsplit, _Float16 *__restrict__ h16,
@@ -477,16 +559,16 @@ __global__ __launch_bounds__(PN_THREADS) void k_pf_attn_rows(const float *__rest
         if (j >= n4) continue;
         const int hh = 4 * j / D, d = 4 * j % D;
         const long long row = (long long)t * NQ + hh;
-        if (nsplit == 1) {
+        if constexpr (NZ == 1) {
             v[i] = *reinterpret_cast<const float4 *>(att + row * D + d);
         } else {
             // every split's record loaded at once (splits past nz re-read the
             // last one and are skipped), then merged in z order
             const float *p = part + row * nsplit * RS;
-            float ml[PA_MAX_SPLIT], ll[PA_MAX_SPLIT];
-            float4 o[PA_MAX_SPLIT];
+            float ml[NZ], ll[NZ];
+            float4 o[NZ];
 #pragma unroll
-            for (int z = 0; z < PA_MAX_SPLIT; z++) {
+            for (int z = 0; z < NZ; z++) {
                 const float *r = p + min(z, nz - 1) * RS;
                 ml[z] = r[D];
                 ll[z] = r[D + 1];
@@ -494,13 +576,13 @@ __global__ __launch_bounds__(PN_THREADS) void k_pf_attn_rows(const float *__rest
             }
             float M = -__builtin_huge_valf();
 #pragma unroll
-            for (int z = 0; z < PA_MAX_SPLIT; z++)
+            for (int z = 0; z < NZ; z++)
                 if (z < nz) M = fmaxf(M, ml[z]);
             float n0 = 0.f, n1 = 0.f, n2 = 0.f, n3 = 0.f, den = 0.f;
 #pragma unroll
-            for (int z = 0; z < PA_MAX_SPLIT; z++) {
+            for (int z = 0; z < NZ; z++) {
                 if (z < nz) {
-                    const float f = __expf(ml[z] - M);
+                    const float f = __builtin_amdgcn_exp2f(ml[z] - M);
                     n0 = fmaf(f, o[z].x, n0);
                     n1 = fmaf(f, o[z].y, n1);
                     n2 = fmaf(f, o[z].z, n2);
@@ -530,32 +612,53 @@ __global__ __launch_bounds__(PN_THREADS) void k_pf_attn_rows(const float *__rest
     if (tid == 0) hinv[t] = ldexpf(1.f, -sh);
 }
 
-// Split size: PA_PREF_KS positions, larger for long contexts so that at
-// most PA_MAX_SPLIT splits exist (a multiple of PA_KF either way).
-static int pf_split_size(int kmax) {
-    int ks = PA_PREF_KS;
-    if ((kmax + ks - 1) / ks > PA_MAX_SPLIT) ks = ((kmax + PA_MAX_SPLIT - 1) / PA_MAX_SPLIT + PA_KF - 1) / PA_KF * PA_KF;
-    return ks;
+// Splits of the positions: as few as give every CU about two workgroups' worth
+// of waves (the partial records are written and read once per split), of at
+// least PA_MIN_KS positions, a multiple of the chunk.
+static int pf_split_size(int kmax, int wgs, int n_cu) {
+    int n = std::max(1, std::min(PA_MAX_SPLIT, (2 * n_cu + wgs - 1) / wgs));
+    n = std::min(n, (kmax + PA_MIN_KS - 1) / PA_MIN_KS);
+    return ((kmax + n - 1) / n + PM_KC - 1) / PM_KC * PM_KC;
 }
 
+template <int D, int G, int WV>
+static hipError_t launch_pf_attn_g(const _Float16 *qb, const _Float16 *k16, const _Float16 *vt, int T, int pos0, int NQ,
+                                   int NKV, int cp, int ks, int nsplit, float *part, float *out, hipStream_t st) {
+    constexpr int QB = 32 * WV / G;
+    static const hipError_t a = hipFuncSetAttribute((const void *)k_pf_attn<D, G, WV>,
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(PmLds<D>));
+    if (a != hipSuccess) return a;
+    hipLaunchKernelGGL((k_pf_attn<D, G, WV>), dim3(NKV, (T + QB - 1) / QB, nsplit), dim3(64 * WV), sizeof(PmLds<D>), st,
+                       qb, k16, vt, T, pos0, NQ, cp, ks, nsplit, part, out);
+    return hipGetLastError();
+}
+
+constexpr int PA_WV = 4;   // waves per attention workgroup
 template <int D>
-static hipError_t launch_pf_attn(int G, const float *qb, const float *kc, const float *vc, int T, int pos0, int NQ,
-                                 int NKV, int max_ctx, float *part, float *out, _Float16 *h16, float *hinv,
-                                 hipStream_t st) {
-    const int ks = pf_split_size(pos0 + T), nsplit = (pos0 + T + ks - 1) / ks;
-#define TBQ_PFA(GG)                                                                                                \
-    case GG:                                                                                                       \
-        hipLaunchKernelGGL((k_pf_attn<D, GG>), dim3(NKV, (T + PM_Q / GG - 1) / (PM_Q / GG), nsplit),               \
-                           dim3(PM_THREADS), 0, st, qb, kc, vc, T, pos0, NQ, max_ctx, ks, nsplit, part, out);      \
-        break;
+static hipError_t launch_pf_attn(int G, const _Float16 *qb, const float *kc, const float *vc, int T, int pos0, int NQ,
+                                 int NKV, int max_ctx, _Float16 *k16, _Float16 *vt, int cp, float *part, float *out,
+                                 _Float16 *h16, float *hinv, int n_cu, hipStream_t st) {
+    const int kmax = pos0 + T, qb_tokens = 32 * PA_WV / G;
+    hipLaunchKernelGGL(k_pf_kv16<D>, dim3(NKV, (kmax + PC_KC - 1) / PC_KC), dim3(256), 0, st, kc, vc, max_ctx, kmax, cp,
+                       k16, vt);
+    const int ks = pf_split_size(kmax, NKV * ((T + qb_tokens - 1) / qb_tokens), n_cu), nsplit = (kmax + ks - 1) / ks;
+    hipError_t err;
     switch (G) {
-        TBQ_PFA(1) TBQ_PFA(2) TBQ_PFA(4) TBQ_PFA(8)
-    default:
-        return hipErrorNotSupported;
+    case 1: err = launch_pf_attn_g<D, 1, PA_WV>(qb, k16, vt, T, pos0, NQ, NKV, cp, ks, nsplit, part, out, st); break;
+    case 2: err = launch_pf_attn_g<D, 2, PA_WV>(qb, k16, vt, T, pos0, NQ, NKV, cp, ks, nsplit, part, out, st); break;
+    case 4: err = launch_pf_attn_g<D, 4, PA_WV>(qb, k16, vt, T, pos0, NQ, NKV, cp, ks, nsplit, part, out, st); break;
+    case 8: err = launch_pf_attn_g<D, 8, PA_WV>(qb, k16, vt, T, pos0, NQ, NKV, cp, ks, nsplit, part, out, st); break;
+    default: return hipErrorNotSupported;
     }
-#undef TBQ_PFA
-    hipLaunchKernelGGL(k_pf_attn_rows<D>, dim3(T), dim3(PN_THREADS), 0, st, part, out, NQ, pos0, ks, nsplit, h16,
-                       hinv);
+    if (err != hipSuccess) return err;
+#define TBQ_PFR(NZ)                                                                                                 \
+    hipLaunchKernelGGL((k_pf_attn_rows<D, NZ>), dim3(T), dim3(PN_THREADS), 0, st, part, out, NQ, pos0, ks, nsplit, \
+                       h16, hinv)
+    if (nsplit == 1) TBQ_PFR(1);
+    else if (nsplit == 2) TBQ_PFR(2);
+    else if (nsplit <= 4) TBQ_PFR(4);
+    else TBQ_PFR(8);
+#undef TBQ_PFR
     return hipGetLastError();
 }
 
@@ -575,8 +678,9 @@ bool dense_prefill_batched(const tbq_dense_model *m) {
 }
 
 struct PfWs {
-    float *x, *y, *qkv, *qb, *att, *gu, *sa, *sb, *part, *rope, *gpart;
-    _Float16 *h16, *wh;
+    float *x, *y, *qkv, *att, *gu, *sa, *sb, *part, *rope, *gpart;
+    _Float16 *h16, *wh, *qb, *k16, *vt;
+    int cp;   // positions per head of k16 and vt
     int *tok;
     void *dec;
 };
@@ -600,7 +704,11 @@ static PfWs pf_ws(const tbq_dense_model *m, int T, void *ws, size_t *total) {
         w.x = (float *)take((size_t)T * H * 4);
         w.y = (float *)take((size_t)T * H * 4);
         w.qkv = (float *)take((size_t)T * QKVR * 4);
-        w.qb = (float *)take((size_t)T * QD * 4);
+        w.qb = (_Float16 *)take((size_t)T * QD * 2);
+        // fp16 K and V of one layer (a prefill reaches position kmax - 1 < max_ctx)
+        w.cp = (m->max_ctx + PC_KC - 1) / PC_KC * PC_KC;
+        w.k16 = (_Float16 *)take((size_t)m->n_kv_heads * w.cp * m->head_dim * 2);
+        w.vt = (_Float16 *)take((size_t)m->n_kv_heads * w.cp * m->head_dim * 2);
         w.att = (float *)take((size_t)T * QD * 4);
         w.gu = (float *)take((size_t)T * 2 * F * 4);
         w.h16 = (_Float16 *)take((size_t)T * wide * 2);
@@ -618,8 +726,8 @@ static PfWs pf_ws(const tbq_dense_model *m, int T, void *ws, size_t *total) {
         w.gpart = gp ? (float *)take(gp) : nullptr;
         w.rope = (float *)take((size_t)T * m->head_dim * 4);
         // attention split partials: a prefill reaching position kmax - 1 uses
-        // min(PA_MAX_SPLIT, ceil(kmax / PA_PREF_KS)) splits, and kmax <= max_ctx
-        const int ns = std::min(PA_MAX_SPLIT, (m->max_ctx + PA_PREF_KS - 1) / PA_PREF_KS);
+        // at most min(PA_MAX_SPLIT, ceil(kmax / PA_MIN_KS)) splits, and kmax <= max_ctx
+        const int ns = std::min(PA_MAX_SPLIT, (m->max_ctx + PA_MIN_KS - 1) / PA_MIN_KS);
         w.part = ns > 1 ? (float *)take((size_t)T * m->n_heads * ns * pf_rec(m->head_dim) * 4) : nullptr;
     }
     if (total) *total = off;
@@ -671,13 +779,17 @@ static hipError_t pf_batched(const tbq_dense_model *m, const PfWs &w, int T, int
         if (err != hipSuccess) break;
         const float *qsrc = qns > 1 ? w.gpart : w.qkv;
         if (D == 128) {
-            hipLaunchKernelGGL(k_pf_qk<128>, dim3(T, NQ + NKV), dim3(64), 0, st, qsrc, qns, (long long)T * QKVR, w.sa,
-                               L.q_norm, L.k_norm, NQ, NKV, pos0, w.rope, m->norm_eps, kc, vc, m->max_ctx, w.qb);
-            err = launch_pf_attn<128>(G, w.qb, kc, vc, T, pos0, NQ, NKV, m->max_ctx, w.part, w.att, w.h16, w.sb, st);
+            hipLaunchKernelGGL(k_pf_qk<128>, dim3(T, (NQ + NKV + 7) / 8), dim3(PQ_THREADS), 0, st, qsrc, qns,
+                               (long long)T * QKVR, w.sa, L.q_norm, L.k_norm, NQ, NKV, pos0, w.rope, m->norm_eps, kc,
+                               vc, m->max_ctx, w.qb);
+            err = launch_pf_attn<128>(G, w.qb, kc, vc, T, pos0, NQ, NKV, m->max_ctx, w.k16, w.vt, w.cp, w.part, w.att,
+                                     w.h16, w.sb, cu, st);
         } else {
-            hipLaunchKernelGGL(k_pf_qk<64>, dim3(T, NQ + NKV), dim3(64), 0, st, qsrc, qns, (long long)T * QKVR, w.sa,
-                               L.q_norm, L.k_norm, NQ, NKV, pos0, w.rope, m->norm_eps, kc, vc, m->max_ctx, w.qb);
-            err = launch_pf_attn<64>(G, w.qb, kc, vc, T, pos0, NQ, NKV, m->max_ctx, w.part, w.att, w.h16, w.sb, st);
+            hipLaunchKernelGGL(k_pf_qk<64>, dim3(T, (NQ + NKV + 15) / 16), dim3(PQ_THREADS), 0, st, qsrc, qns,
+                               (long long)T * QKVR, w.sa, L.q_norm, L.k_norm, NQ, NKV, pos0, w.rope, m->norm_eps, kc,
+                               vc, m->max_ctx, w.qb);
+            err = launch_pf_attn<64>(G, w.qb, kc, vc, T, pos0, NQ, NKV, m->max_ctx, w.k16, w.vt, w.cp, w.part, w.att,
+                                     w.h16, w.sb, cu, st);
         }
         if (err != hipSuccess) break;
         if ((err = gemm(qt_of(L.qt_o), L.wo, H, QD, w.y, H, &yns)) != hipSuccess) break;
