@@ -42,11 +42,29 @@ __device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, dma_rsrc_t rs
                  : "memory");
 }
 
+// 256 bytes: lane i copies the 4 bytes at voff to LDS byte lds + 4 i.
+__device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, dma_rsrc_t rsrc) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc)
+                 : "memory");
+}
+
+// dma16 from a 64-bit address per lane.
+__device__ __forceinline__ void dma16_ptr(uint32_t lds, const void *p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+
 // Every outstanding copy of this wave has landed and every LDS read it has
 // issued has returned, then the workgroup's barrier: what the other waves
 // copied is visible, and what this wave read may be overwritten.
 __device__ __forceinline__ void dma_wait_barrier() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The same with the N memory operations issued last left in flight (they
+// complete in issue order, so all copies before them have landed).
+template <int N>
+__device__ __forceinline__ void dma_wait_barrier_n() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 }  // namespace tbq

@@ -87,7 +87,7 @@ hipError_t launch_combine(const MoeArgs &a, hipStream_t st);
 hipError_t launch_router(const float *xn, const float *router, const float *bias, int T, int H, int E, int top_k,
                          float *logits, unsigned *counters, int *sel_idx, float *sel_w, hipStream_t st,
                          _Float16 *x16 = nullptr, float *xinv = nullptr, bool *x16_done = nullptr,
-                         const MoeArgs *group = nullptr, bool *grouped = nullptr);
+                         const MoeArgs *group = nullptr, bool *grouped = nullptr, bool x16_swap = false);
 // Decode expert kernels for Q4_K tensors (tbq_moe_q4k.hip).  A batch runs in
 // expert order when moe_decode_grouped(a): launch_group writes a.grp first.
 bool moe_decode_grouped(const MoeArgs &a);
@@ -106,11 +106,12 @@ hipError_t launch_moe_down_kq(const MoeArgs &a, bool grouped, hipStream_t st);
 size_t prefill_workspace_bytes(int T, int k, int E, int H, int F);
 bool gemm_k_supported(int K);
 // rows of n floats to fp16 with per-row power-of-two scales (inv = 1 / scale)
-hipError_t launch_rows_f16(const float *in, int rows, int n, _Float16 *out, float *inv, hipStream_t st);
+// (swap: every four elements in the order 0, 2, 1, 3)
+hipError_t launch_rows_f16(const float *in, int rows, int n, _Float16 *out, float *inv, hipStream_t st, bool swap = false);
 hipError_t launch_moe_prefill_q4k(const MoeArgs &a, void *scratch, hipStream_t st, bool x16_done = false);
 // Where the prefill scratch keeps the tokens' fp16 rows and their inverse
-// scales (so the router can write them).
-void prefill_x16(const MoeArgs &a, void *scratch, _Float16 **x16, float **xinv);
+// scales (so the router can write them), and whether the rows are swapped.
+void prefill_x16(const MoeArgs &a, void *scratch, _Float16 **x16, float **xinv, bool *swap);
 hipError_t launch_moe_bf16(const MoeArgs &a, void *scratch, hipStream_t st);
 // int8 MFMA prefill (TBQ_MOE_I8): Q8_K activations against the Q4_K nibbles
 size_t prefill_i8_workspace_bytes(int T, int k, int E, int H, int F);

@@ -461,9 +461,11 @@ static hipError_t launch_moe_bf16_chunk(const MoeArgs &a, void *scratch, hipStre
     _Float16 *x16 = nullptr;
     float *xinv = nullptr;
     bool x16_done = false;
-    prefill_x16(a, scratch, &x16, &xinv);
+    bool swap = false;
+    prefill_x16(a, scratch, &x16, &xinv, &swap);
     hipError_t err = launch_router(a.xn, a.router, a.bias, a.T, a.H, a.E, a.top_k, a.logits,
-                                   a.T >= 32 ? nullptr : a.counters, a.sel_idx, a.sel_w, st, x16, xinv, &x16_done);
+                                   a.T >= 32 ? nullptr : a.counters, a.sel_idx, a.sel_w, st, x16, xinv, &x16_done,
+                                   nullptr, nullptr, swap);
     if (err == hipErrorNotSupported)
         err = launch_route(a.xn, a.router, a.bias, a.T, a.H, a.E, a.top_k, a.sel_idx, a.sel_w, st);
     if (err != hipSuccess) return err;

@@ -11,24 +11,15 @@
 //                     power of two that puts its max |value| in [2^14, 2^15)
 //                     (exact, undone in the GEMM epilogues): x for gate/up,
 //                     the SwiGLU activations for down.
-//   k_moe_f16<0,NS>   act[p] = swiglu(x_t . W_gate[e], x_t . W_up[e]) for a
+//   k_moe_f16<0>      act[p] = swiglu(x_t . W_gate[e], x_t . W_up[e]) for a
 //                     tile of <= 128 pairs x 128 columns (256 weight rows:
 //                     128 gate and 128 up rows), K = H, fp32 out.
-//   k_moe_f16<1,NS>   y[p] = act[p] . W_down[e] for <= 128 pairs x 256 rows,
+//   k_moe_f16<1>      y[p] = act[p] . W_down[e] for <= 128 pairs x 256 rows,
 //                     K = F.
 //   (k_combine)       out = resid + sum over slots in slot order (tbq_moe.hip).
 //
-// Weights never pass through LDS.  Each lane dequantises its own MFMA A
-// operands in registers: in v_mfma_f32_32x32x16_f16, lane l supplies row
-// l % 32 and eight consecutive k of the 16 per step, the half h = l / 32
-// choosing which eight.  Within a 128-column chunk the k order is permuted
-// (the products are summed over k, so any order shared by both operands
-// gives the same sum): step ks, half h covers chunk columns 64h + 8ks .. +8,
-// so a lane's 64 weights per chunk are two whole Q4_K sub-blocks -- 32
-// contiguous quant bytes and one scale/min pair each.  Only the activation
-// tile is shared by the workgroup's 8 waves: it is staged in LDS, double
-// buffered, one barrier per chunk.  Weight loads run two chunks ahead,
-// activation loads one.
+// Weights never pass through LDS as fp16: their packed bytes are staged and
+// each lane dequantises its own MFMA A operands in registers.
 //
 // Dequantisation to fp16.  A nibble q becomes the fp16 number 1 + q/16 by
 // placing q in the mantissa (0x3C00 | q << 6), for two weights per dword:
@@ -43,6 +34,7 @@
 // Accuracy: fp16 weights and activations (11-bit mantissa), fp32
 // accumulation; outputs land within 1e-2 relative L2 of the fp32 reference.
 // The weights' fp16 form needs 16 * 63 * d + 63 * dmin below 65504.
+#include "tbq_dma.hpp"
 #include "tbq_kernels.h"
 #include "tbq_kquant.hpp"
 
@@ -64,14 +56,12 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int PF_MT = 128;         // pairs per tile (four 32-pair MFMA sub-tiles)
 constexpr int PF_KC = 128;         // K columns per chunk (half a Q4_K super-block)
-constexpr int PF_LD = PF_KC + 8;   // LDS row stride in halves (padding breaks bank aliasing)
 #ifndef PF_WAVES
 #define PF_WAVES 8
 #endif
 constexpr int PF_THREADS = 64 * PF_WAVES;   // 32 weight rows per wave
 constexpr int PF_ROWS = 32 * PF_WAVES;      // weight rows per workgroup
 constexpr int PF_COLS = PF_ROWS / 2;        // gate/up columns per workgroup
-constexpr size_t PF_LDS_BYTES = (size_t)2 * PF_MT * PF_LD * 2 + PF_MT * 8;   // two activation tiles, pair ids, scales
 
 struct PfTile {
     int e, n;
@@ -223,13 +213,14 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_i
 // ---------------------------------------------------------------------------
 // Rows of n floats to fp16: one workgroup per row; s = 2^(15 - e) with
 // max |row| = f * 2^e (f in [0.5, 1)), so |row| * s < 2^15; inv[row] = 1/s.
-// n a multiple of 4.
+// n a multiple of 4.  swap: every four elements are stored in the order 0, 2,
+// 1, 3 (the k order of the ggml layout's fragments).
 // ---------------------------------------------------------------------------
 // RV > 0: the row is held in registers (n <= 1024 RV), read once with
 // every load issued before the max; RV = 0: two passes over the row.
 template <int RV>
 __global__ __launch_bounds__(256) void k_rows_f16(const float *__restrict__ in, int n, _Float16 *__restrict__ out,
-                                                  float *__restrict__ inv) {
+                                                  float *__restrict__ inv, bool swap) {
     __shared__ float part[4];
     const int row = blockIdx.x, tid = threadIdx.x, n4 = n / 4;
     const float4 *r = reinterpret_cast<const float4 *>(in + (long long)row * n);
@@ -259,8 +250,8 @@ __global__ __launch_bounds__(256) void k_rows_f16(const float *__restrict__ in, 
     const float s = ldexpf(1.f, sh);
     uint2 *o = reinterpret_cast<uint2 *>(out + (long long)row * n);
     auto put = [&](int i, float4 w) {
-        const f16x2 a = {(_Float16)(w.x * s), (_Float16)(w.y * s)};
-        const f16x2 b = {(_Float16)(w.z * s), (_Float16)(w.w * s)};
+        const f16x2 a = {(_Float16)(w.x * s), (_Float16)((swap ? w.z : w.y) * s)};
+        const f16x2 b = {(_Float16)((swap ? w.y : w.z) * s), (_Float16)(w.w * s)};
         o[i] = make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
     };
     if constexpr (RV > 0) {
@@ -273,329 +264,340 @@ __global__ __launch_bounds__(256) void k_rows_f16(const float *__restrict__ in, 
     if (tid == 0) inv[row] = ldexpf(1.f, -sh);
 }
 
-// ---------------------------------------------------------------------------
-// Weight staging.
-// ---------------------------------------------------------------------------
-// One lane's loads for a 128-column chunk: the 64 weights of sub-blocks j0
-// and j0 + 1 of a row's Q4_K super-block (j0 even), and 16 header bytes.
-// The header the two chunks of a super-block need is bytes 0..19: d/dmin
-// (0..3), the scale and min dwords of sub-blocks 0..3 (4..7, 8..11), the
-// scale dword of 4..7 (12..15) and their min dword (16..19, which are quant
-// bytes 0..3, layer4/tb_gguf.c:163-168).  The even chunk (j0 < 4) loads
-// bytes 0..15 and passes d/dmin and the scale dword of 4..7 on to the odd
-// chunk, which loads bytes 16..31 for the min dword: one 16-byte load per
-// chunk instead of a dword and a dword pair (weight loads are issued per
-// lane, each to its own row's cache lines, and their count is what the
-// memory pipeline pays for).
-struct Q4Pair {
-    u32x4 h, q0, q1;
-};
-
-template <bool GG>
-__device__ __forceinline__ void q4pair_load(const uint8_t *sb, int j0, Q4Pair &r) {
-    // ggml's scales and mins of all eight sub-blocks are in bytes 4..15
-    r.h = *reinterpret_cast<const u32x4 *>(sb + (GG || j0 < 4 ? 0 : 16));
-    r.q0 = *reinterpret_cast<const u32x4 *>(sb + 16 + 16 * j0);
-    r.q1 = *reinterpret_cast<const u32x4 *>(sb + 32 + 16 * j0);
-}
-
 __device__ __forceinline__ float h2f(unsigned bits) {
     return (float)__builtin_bit_cast(_Float16, (unsigned short)(bits & 0xFFFFu));
 }
 
-// Four quant bytes -> eight fp16 weights S q - Mn (low nibble first, the
-// reference's order), as one MFMA operand.
-__device__ __forceinline__ f16x8 q4dword_f16(unsigned q, f16x2 S16, f16x2 C) {
-    unsigned o[4];
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        // quant byte (hi << 4 | lo) -> halves (1 + lo/16, 1 + hi/16)
-        const unsigned y = (q >> (8 * b)) & 0xFFu;
-        const unsigned t = __builtin_amdgcn_bitop3_b32(__umul24(y, 0x40040u), 0x03C003C0u, 0x3C003C00u, 0xEA);   // (a & b) | c
-        o[b] = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, t), S16, C));
-    }
-    return __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
-}
-
-// The lane's four A operands of sub-block j0 + u (steps 4u .. 4u + 3 of the
-// chunk use its quant dwords 0..3).
-// dd = d/dmin, sw and mw = the scale and min dwords of j0's half.
-__device__ __forceinline__ void q4pair_frags(const Q4Pair &r, unsigned dd, unsigned sw, unsigned mw, int j0, int u,
-                                             f16x8 *a) {
-    const int sh = 8 * ((j0 + u) & 3);
-    const float S = h2f(dd) * (float)((sw >> sh) & 63), Mn = h2f(dd >> 16) * (float)((mw >> sh) & 63);
-    const _Float16 s16 = (_Float16)(16.f * S), c = (_Float16)(-(float)s16 - Mn);
-    const f16x2 S16 = {s16, s16}, C = {c, c};
-    const u32x4 q = u ? r.q1 : r.q0;
-    a[0] = q4dword_f16(q.x, S16, C);
-    a[1] = q4dword_f16(q.y, S16, C);
-    a[2] = q4dword_f16(q.z, S16, C);
-    a[3] = q4dword_f16(q.w, S16, C);
-}
-
-// ggml's layout (QT_GQ4_K): the 32 quant bytes of sub-blocks j0, j0 + 1 (j0
-// even) hold sub-block j0's element i in the low nibble of byte i and
-// sub-block j0 + 1's in the high nibble; the scale and min of sub-block j
-// follow ggml's get_scale_min_k4 over scale bytes 4..15; d and dmin are IEEE
-// halves.  Two quant dwords (bytes 8ks .. 8ks + 7) -> the eight fp16 weights
-// S q - Mn of step ks: a byte pair's two nibbles are spread into the two
-// halves by one 24-bit multiply (bits 6..9 and 22..25 of y * 0x4040, y the
-// pair's nibbles at bits 0..3 and 8..11) and one v_bitop3, then the packed
-// fma as in the reference's layout.
-__device__ __forceinline__ f16x8 gq4dwords_f16(unsigned d0, unsigned d1, bool hi, f16x2 S16, f16x2 C) {
-    const unsigned m0 = (hi ? d0 >> 4 : d0) & 0x0F0F0F0Fu, m1 = (hi ? d1 >> 4 : d1) & 0x0F0F0F0Fu;
-    const unsigned y[4] = {m0 & 0xFFFFu, m0 >> 16, m1 & 0xFFFFu, m1 >> 16};
-    unsigned o[4];
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        const unsigned t = __builtin_amdgcn_bitop3_b32(__umul24(y[b], 0x4040u), 0x03C003C0u, 0x3C003C00u, 0xEA);
-        o[b] = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, t), S16, C));
-    }
-    return __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
-}
-
-__device__ __forceinline__ void gq4pair_frags(const Q4Pair &r, int j0, int u, f16x8 *a) {
-    const int jj = j0 + u, k = jj & 3;
-    const bool hi = jj >= 4;
-    const unsigned y = r.h.y >> (8 * k), z = r.h.z >> (8 * k), w = r.h.w >> (8 * k);
-    const int sc = hi ? (int)((w & 15u) | (((y >> 6) & 3u) << 4)) : (int)(y & 63u);
-    const int mn = hi ? (int)(((w >> 4) & 15u) | (((z >> 6) & 3u) << 4)) : (int)(z & 63u);
-    const float S = h2f(r.h.x) * (float)sc, Mn = h2f(r.h.x >> 16) * (float)mn;
-    const _Float16 s16 = (_Float16)(16.f * S), c = (_Float16)(-(float)s16 - Mn);
-    const f16x2 S16 = {s16, s16}, C = {c, c};
-    a[0] = gq4dwords_f16(r.q0.x, r.q0.y, u, S16, C);
-    a[1] = gq4dwords_f16(r.q0.z, r.q0.w, u, S16, C);
-    a[2] = gq4dwords_f16(r.q1.x, r.q1.y, u, S16, C);
-    a[3] = gq4dwords_f16(r.q1.z, r.q1.w, u, S16, C);
-}
-
 // ---------------------------------------------------------------------------
-// Expert tile GEMM.  Work items are (tile, row block) pairs, tile-major
-// (ncb = F/PF_COLS row blocks for MODE 0, H/PF_ROWS for MODE 1), the tiles
-// heaviest first; K = NS * 128.  The grid is persistent (one workgroup
-// per CU): workgroup b starts with item b, then takes tickets from the
+// Expert tile GEMM.  Work items are (tile, row block) pairs, tile-major (ncb =
+// F/128 row blocks of 128 columns for MODE 0, H/256 of 256 rows for MODE 1),
+// the tiles heaviest first.  The grid is persistent (two workgroups of four
+// waves per CU): workgroup b starts with item b, then takes tickets from the
 // counter ntiles[1 + MODE] (zeroed by k_dispatch): item grid + ticket, the
-// ticket taken two chunks before the end of the current item.  Items thus
-// go out heaviest first to whichever workgroup is about to be free (greedy
-// list scheduling); a fixed stride over the items left the workgroups that
-// drew heavy items 30% busier than the mean.
-//   MODE 0: wave w, lane row i = l % 32 is gate (i < 16) or up (i >= 16)
-//   column PF_COLS*cb + 16w + i % 16, so a lane's accumulator registers r
-//   and r + 8 hold gate and up of the same (column, pair) and SwiGLU needs
-//   no data exchange; X rows are tokens (ttok) of x.
-//   MODE 1: lane row i is down row PF_ROWS*cb + 32w + i; X rows are pairs
-//   (tpair) of act.  xinv[X row] undoes the row's fp16 scaling.
-// Activation staging per chunk: segments tid + 512m (m < 4) = (pair it/16,
-// 8 halves at 8*(it%16)).  Every global load is unconditional (indices
-// clamped, results selected), so the compiler's wait counts stay exact.
+// ticket taken two steps before the end of the current item (taken an item
+// ahead, with the next item's lists copied to LDS meanwhile, T = 512 was 9%
+// slower: with little more than one item per workgroup the second ones then go
+// to the workgroups with the heaviest first).  Items thus go out heaviest first
+// to whichever workgroup is about to be free (greedy list scheduling); a fixed stride over the items left the workgroups that drew
+// heavy items 30% busier than the mean.
+//
+// Wave w owns 64 weight rows in two 32-row blocks: MODE 0 gate and up of the
+// columns 128 cb + 32 w .. + 31 (so SwiGLU pairs the two blocks' accumulators),
+// MODE 1 the down rows 256 cb + 64 w .. + 63; and all of the tile's pairs, in
+// NB 32-pair sub-tiles.  X rows are tokens (ttok) of x in MODE 0, pairs (tpair)
+// of act in MODE 1; xinv[X row] undoes the row's fp16 scaling.
+//
+// K advances 64 columns (two Q4_K sub-blocks) a step.  Packed quants (32 bytes
+// a row), headers and activation rows are copied directly to LDS (tbq_dma.hpp)
+// into rings of D steps, with counted waits: a tile of few pairs is bound by
+// the weights' latency, and D = 5 at one sub-tile keeps four steps (32 KiB) of
+// weights in flight per workgroup; D = 3 where four sub-tiles' activations
+// need the room.  Quants run one step ahead of the activations, so a lane reads
+// its rows' bytes during the step before and its first MFMA finds the fragment
+// made.  Each lane dequantises its own rows' fragments between the MFMAs
+// of the fragments before (half h = lane / 32 covers columns 32 h .. + 31 of a
+// step, one sub-block; the k order inside a step is the same for both
+// operands).  LDS rows are swizzled by the copies' source addresses: slot seg
+// ^ swizzle(row), so column reads spread over all banks.
+//
+// Against one 8-wave workgroup per CU whose lanes loaded their own rows' bytes
+// (32 rows per wave, so twice the LDS reads per MFMA), Qwen3-30B-A3B layer: T =
+// 512 Zipf-skewed gate/up 87.5 -> 72 us and down 46.6 -> 55 us (its 12 steps
+// are short against an item's start), 1999 tokens of ggml's layout 330 -> 267
+// us for the two.  Left: 512 tokens read 204 + 153 MB (39 + 29 us at the copy
+// rate) while the heaviest experts' tiles, which set the end, wait for the same
+// memory; without copies the two take 88 us, without the dequantisation as
+// well 71.
 // ---------------------------------------------------------------------------
-template <int MODE, int NS, bool GG>
-__global__ __launch_bounds__(PF_THREADS) void k_moe_f16(const uint8_t *__restrict__ W0, const uint8_t *__restrict__ W1,
-                                                        const _Float16 *__restrict__ X, int x_rows,
-                                                        const float *__restrict__ xinv, const int *__restrict__ tpair,
-                                                        const int *__restrict__ ttok, const PfTile *__restrict__ tiles,
-                                                        int *__restrict__ ntiles, int ncb, int H, int F,
-                                                        float *__restrict__ out) {
-    constexpr int K = NS * PF_KC;
-    constexpr int XPT = PF_MT * PF_KC / 8 / PF_THREADS;   // 16-byte activation segments per thread per chunk
-    extern __shared__ __attribute__((aligned(16))) _Float16 pf_lds[];   // [2][PF_MT][PF_LD]
-    const int nitems = *ntiles * ncb;
-    __shared__ int next_item;
-    for (int item = blockIdx.x; item < nitems;) {
-    // item -> (tile, row block).  The tile record and its row lists are
-    // loaded together.
-    const int tix = item / ncb, cb = item % ncb;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, lh = lane >> 5;
-    const int *xrows = (MODE == 0 ? ttok : tpair) + tix * PF_MT;
-    int px[XPT];
-#pragma unroll
-    for (int m = 0; m < XPT; m++) px[m] = xrows[(tid + PF_THREADS * m) >> 4];
-    const int po = tid < PF_MT ? tpair[tix * PF_MT + tid] : -1;
-    const int pxo = tid < PF_MT ? xrows[tid] : -1;
-    const PfTile tl = tiles[tix];
-    const long long rb = (long long)(K / 256) * 144;
+constexpr int MF_WAVES = 4, MF_ROWS = 64 * MF_WAVES;
+constexpr int mf_depth(int nb) { return nb == 1 ? 5 : nb == 2 ? 4 : 3; }
+// header slots: at D = 5 the next super-block's copy is issued in the step that
+// reads the current one's, at D <= 4 after it
+constexpr int mf_hdrs(int nb) { return mf_depth(nb) > 4 ? 2 : 1; }
+constexpr int mf_lds(int nb) { return mf_hdrs(nb) * MF_ROWS * 16 + mf_depth(nb) * (MF_ROWS * 32 + nb * 32 * 128); }
+// behind the rings: this item's pair ids and row scales, and the next item
+struct MfLists {
+    int tp[PF_MT];
+    float xsc[PF_MT];
+    int next, pad[3];
+};
+constexpr int MF_RING = mf_lds(4) > mf_lds(1) ? mf_lds(4) : mf_lds(1);
+constexpr int MF_LDS = MF_RING + (int)sizeof(MfLists);
+static_assert(mf_lds(2) <= MF_RING && mf_lds(3) <= MF_RING && 2 * MF_LDS <= 160 * 1024, "two workgroups per CU");
 
-    const uint8_t *wrow;
-    if (MODE == 0) {
-        const int col = cb * PF_COLS + 16 * wave + (li & 15);
-        wrow = (li < 16 ? W0 : W1) + ((long long)tl.e * F + col) * rb;
-    } else {
-        wrow = W0 + ((long long)tl.e * H + cb * PF_ROWS + 32 * wave + li) * rb;
-    }
-    auto wload = [&](Q4Pair &w, int s) { q4pair_load<GG>(wrow + (long long)(s >> 1) * 144, 4 * (s & 1) + 2 * lh, w); };
-    Q4Pair w0, w1, w2;
+__device__ __forceinline__ int mf_swz8(int r) { return (r & 7) ^ ((r >> 3) & 1); }    // 128-byte rows
+__device__ __forceinline__ int mf_swz2(int r) { return ((r >> 2) ^ (r >> 3)) & 1; }   // 32-byte rows
 
-    // activation rows through a range-checked buffer descriptor: rows past
-    // the tile's pair count (id -1) get an offset beyond the buffer, which
-    // loads zeros without a memory access
-    const int xbytes = x_rows * K * 2;
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void *)X, (short)0, xbytes, 0x00020000);
-    int xoff[XPT];
+// One item for a compile-time count of sub-tiles.  w0, w1: the wave's blocks'
+// rows (32 rows of rb bytes each); xrows: the tile's X rows; tp, xsc: its pair
+// ids and X row scales in LDS.
+template <int MODE, bool GG, int NB>
+__device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, const uint8_t *w1, uint32_t rb, int K,
+                                        const _Float16 *X, uint32_t xbytes, const int *xrows, const int *tp,
+                                        const float *xsc, int n, int col, int ldo, float *out, int *ticket, int &nxt) {
+    constexpr int D = mf_depth(NB), HD = mf_hdrs(NB), XS = NB * 32 * 128, QS = MF_ROWS * 32;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31,
+              lh = lane >> 5;
+    unsigned char *const lh_p = lds, *const lq_p = lds + HD * MF_ROWS * 16, *const lx_p = lq_p + D * QS;
+    const int nst = K >> 6;
+    // activation copies: 8 rows x 8 segments each, NB per wave and step; rows
+    // past the tile's pairs (id -1) copy row 0, whose results are not stored
+    uint32_t xv[NB];
 #pragma unroll
-    for (int m = 0; m < XPT; m++) {
-        const int it = tid + PF_THREADS * m;
-        xoff[m] = px[m] >= 0 ? (px[m] * K + 8 * (it & 15)) * 2 : xbytes;
+    for (int i = 0; i < NB; i++) {
+        const int r = 8 * (wave + MF_WAVES * i) + (lane >> 3);
+        xv[i] = (uint32_t)max(xrows[r], 0) * (uint32_t)(K * 2) + 16u * ((lane & 7) ^ mf_swz8(r));
     }
-    u32x4 xr[XPT];
-    auto xload = [&](int s) {
+    const dma_rsrc_t xr = dma_rsrc(X, xbytes);
+    const dma_rsrc_t r0 = dma_rsrc(w0, 32 * rb), r1 = dma_rsrc(w1, 32 * rb);
+    // quant copies: 32 rows x 2 segments each, one per block and step
+    const uint32_t qv = (uint32_t)(lane >> 1) * rb + 16u + 16u * ((lane & 1) ^ mf_swz2(lane >> 1));
+    // header copy: lane = row of block 0, then of block 1
+    const uint8_t *hp = (lane < 32 ? w0 : w1) + (uint32_t)li * rb;
+    const uint32_t ax = lds_addr(lx_p) + wave * 1024, aq = lds_addr(lq_p) + wave * 2048, ah = lds_addr(lh_p) + wave * 1024;
+    auto copy_x = [&](int slot, int step) {
 #pragma unroll
-        for (int m = 0; m < XPT; m++)
-            xr[m] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xoff[m] < xbytes ? xoff[m] + s * PF_KC * 2 : xbytes, 0, 0);
+        for (int i = 0; i < NB; i++) dma16(ax + slot * XS + MF_WAVES * i * 1024, xv[i], xr, min(step, nst - 1) * 128);
     };
-    auto xstore = [&](int buf) {
+    auto copy_q = [&](int slot, int step) {   // steps past the end: empty descriptors, no memory access
+        const uint32_t so = (min(step, nst - 1) >> 2) * 144 + (step & 3) * 32;
+        dma16(aq + slot * QS, qv, r0, so);
+        dma16(aq + slot * QS + 1024, qv, r1, so);
+    };
+    auto copy_h = [&](int sb) { dma16_ptr(ah + sb % HD * (MF_ROWS * 16), hp + min(sb, (nst >> 2) - 1) * 144); };
+
+    f32x16 acc[2][NB];
 #pragma unroll
-        for (int m = 0; m < XPT; m++) {
-            const int it = tid + PF_THREADS * m;
-            *reinterpret_cast<u32x4 *>(pf_lds + (buf * PF_MT + (it >> 4)) * PF_LD + 8 * (it & 15)) = xr[m];
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int t = 0; t < NB; t++) acc[b][t] = f32x16{};
+
+    constexpr int QR = GG ? 2 : 1;   // 16-byte quant reads per lane and step
+    u32x4 hd[2], q[2][QR];
+    uint32_t mhi[2];
+    f16x2 S16[2], C[2];
+    f16x8 a[2][2];
+    const int wrow = wave * 64 + li, qsw = mf_swz2(li);
+    // the raw bytes of step s (of its super-block), whose quants sit in slot
+    auto raw = [&](int s, int slot, int sb) {
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const unsigned char *qrow = lq_p + slot * QS + (wrow + 32 * b) * 32;
+            if (s == 0) {
+                hd[b] = *reinterpret_cast<const u32x4 *>(lh_p + sb % HD * (MF_ROWS * 16) + (wrow + 32 * b) * 16);
+                // the reference's mins of sub-blocks 4..7 are quant bytes 0..3 (layer4/tb_gguf.c:163-168)
+                if constexpr (!GG) mhi[b] = *reinterpret_cast<const uint32_t *>(qrow + 16 * qsw);
+            }
+            if constexpr (GG) {
+                q[b][0] = *reinterpret_cast<const u32x4 *>(qrow + 16 * qsw);
+                q[b][QR - 1] = *reinterpret_cast<const u32x4 *>(qrow + 16 * (qsw ^ 1));
+            } else {
+                q[b][0] = *reinterpret_cast<const u32x4 *>(qrow + 16 * (lh ^ qsw));
+            }
         }
     };
-    // Issue order: chunk 0's activations and the rows' scales, then the
-    // weights of chunks 0 and 1, so that staging the activations and
-    // storing the scales wait for their own loads only (the wait counter
-    // counts loads in issue order); the weights arrive behind them.
-    xload(0);
-    const float sc = tid < PF_MT && pxo >= 0 ? xinv[pxo] : 0.f;
-    wload(w0, 0);
-    wload(w1, min(1, NS - 1));
-    // the tile's pair ids and activation-row scales, for the epilogue, in
-    // LDS behind the two activation buffers
-    int *po_s = reinterpret_cast<int *>(pf_lds + 2 * PF_MT * PF_LD);
-    float *sc_s = reinterpret_cast<float *>(po_s + PF_MT);
-    xstore(0);
-    if (tid < PF_MT) {
-        po_s[tid] = po;
-        sc_s[tid] = sc;
-    }
-    xload(min(1, NS - 1));
-    __syncthreads();
-
-    const _Float16 *xfrag = pf_lds + li * PF_LD + 64 * lh;
-    // the workgroup's next item: a ticket taken two chunks before the end of
-    // this one (its latency hidden behind them), so items go to workgroups
-    // in the order they finish work, heaviest items first
-    int nxt = 0;
-    // d/dmin and the scale dword of sub-blocks 4..7, from the even chunk's
-    // header for the odd chunk of the same super-block
-    unsigned kdd = 0, ksw = 0;
-    // The chunk loop and the epilogue for a compile-time count of 32-pair
-    // sub-tiles (1..4, uniform over the workgroup): one copy per count, so
-    // no branch splits a chunk's LDS reads from its MFMAs and the compiler
-    // can issue the next operands' reads while the current MFMAs run.
-    auto body = [&](auto nsub_c) {
-        constexpr int NSUB = decltype(nsub_c)::value;
-        f32x16 acc[NSUB];
+    // 16 S and C = -16 S - M of the lane's sub-block 2 s + lh
+    auto scales = [&](int s) {
 #pragma unroll
-        for (int t = 0; t < NSUB; t++) acc[t] = f32x16{};
-        // steps 4u .. 4u + 3 of a chunk for every sub-tile
-        auto mma = [&](const f16x8 *a, const _Float16 *xb, int u) {
-#pragma unroll
-            for (int t = 0; t < NSUB; t++) {
-                f16x8 bv[4];
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++)
-                    bv[ks] = *reinterpret_cast<const f16x8 *>(xb + 32 * t * PF_LD + 8 * (4 * u + ks));
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++)
-                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks], bv[ks], acc[t], 0, 0, 0);
+        for (int b = 0; b < 2; b++) {
+            const int jb = 16 * (s & 1) + 8 * lh;
+            uint32_t sc, mn;
+            if constexpr (GG) {   // ggml's get_scale_min_k4
+                const uint32_t y = hd[b].y >> jb, z = hd[b].z >> jb, w = hd[b].w >> jb;
+                sc = s < 2 ? y & 63 : (w & 15) | ((y >> 2) & 48);
+                mn = s < 2 ? z & 63 : ((w >> 4) & 15) | ((z >> 2) & 48);
+            } else {
+                sc = ((s < 2 ? hd[b].y : hd[b].w) >> jb) & 63;
+                mn = ((s < 2 ? hd[b].z : mhi[b]) >> jb) & 63;
             }
-        };
-        // chunk s: weights of chunk s + 2 into wn (ring of three named
-        // slots, so the loop need not be unrolled to keep them in
-        // registers), activations of chunk s + 2 into registers after
-        // staging chunk s + 1's into LDS.  Chunks past the end reload the
-        // last one and skip the work.  Every path through a chunk issues the
-        // same global loads (the compiler merges wait counts over paths, and
-        // a path with fewer loads would make it wait for the prefetches too).
-        auto chunk = [&](int s, const Q4Pair &wc, Q4Pair &wn) {
-            wload(wn, min(s + 2, NS - 1));
-            if (s == NS - 2 && tid == 0) nxt = atomicAdd(ntiles + 1 + MODE, 1) + (int)gridDim.x;
-            if (s < NS) {
-                const int j0 = 4 * (s & 1) + 2 * lh;
-                const _Float16 *xb = xfrag + (s & 1) * PF_MT * PF_LD;
-                if constexpr (GG) {
+            const float S = h2f(hd[b].x) * (float)sc, M = h2f(hd[b].x >> 16) * (float)mn;
+            const _Float16 s16 = (_Float16)(16.f * S), cc = (_Float16)(-(float)s16 - M);
+            S16[b] = f16x2{s16, s16};
+            C[b] = f16x2{cc, cc};
+        }
+    };
+    const int gsh0 = 6 - 4 * lh, gsh1 = 2 + 4 * lh;   // ggml: nibble lh of bytes 0, 2 and of bytes 1, 3 to bit 6
+    // fragment kk: the weights of columns 32 lh + 8 kk .. + 7 of the step.
+    // Reference layout: weights 2i, 2i + 1 in the nibbles of quant byte i, a
+    // byte spread into the two halves by one 24-bit multiply.  ggml's: weight i
+    // of sub-block lh in nibble lh of byte i; one shift and one v_bitop3 take
+    // bytes 0 and 2 (then 1 and 3) of a dword, so k runs 0, 2, 1, 3 in every
+    // four columns, an order in which the activation rows are stored
+    // (launch_rows_f16).
+    auto frag = [&](int b, int kk) {
+        unsigned w[4];
+        if constexpr (GG) {
+            const u32x4 v = q[b][kk >> 1 & (QR - 1)];
 #pragma unroll
-                    for (int u = 0; u < 2; u++) {
-                        f16x8 a[4];
-                        gq4pair_frags(wc, j0, u, a);
-                        mma(a, xb, u);
-                    }
-                } else {
-                    const bool odd = s & 1;
-                    const unsigned dd = odd ? kdd : wc.h.x, sw = odd ? ksw : wc.h.y, mw = odd ? wc.h.x : wc.h.z;
-                    kdd = dd;
-                    ksw = odd ? ksw : wc.h.w;
-#pragma unroll
-                    for (int u = 0; u < 2; u++) {
-                        f16x8 a[4];
-                        q4pair_frags(wc, dd, sw, mw, j0, u, a);
-                        mma(a, xb, u);
-                    }
-                }
-                // buffer last read in chunk s - 1, before the previous barrier
-                if (s + 1 < NS) xstore((s + 1) & 1);
-            }
-            xload(min(s + 2, NS - 1));
-            if (s < NS) __syncthreads();
-        };
-        if constexpr (NS == 4 || (GG && NS <= 8)) {
-            // two or three trips, not unrolled: unrolled, the compiler
-            // overlaps the trips past what the register file holds (spills)
-#pragma nounroll
-            for (int s = 0; s < NS; s += 3) {
-                chunk(s, w0, w2);
-                chunk(s + 1, w1, w0);
-                chunk(s + 2, w2, w1);
+            for (int i = 0; i < 4; i++) {
+                const unsigned d = i < 2 ? (kk & 1 ? v.z : v.x) : (kk & 1 ? v.w : v.y);
+                // nibble lh of bytes 0 and 2 (i even) or 1 and 3 to bits 6..9 and 22..25
+                const unsigned y = i & 1 ? d >> gsh1 : d << gsh0;
+                const unsigned t = __builtin_amdgcn_bitop3_b32(y, 0x03C003C0u, 0x3C003C00u, 0xEA);
+                w[i] = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, t), S16[b], C[b]));
             }
         } else {
-            for (int s = 0; s < NS; s += 3) {
-                chunk(s, w0, w2);
-                chunk(s + 1, w1, w0);
-                chunk(s + 2, w2, w1);
+            const u32x4 v = q[b][0];
+            const unsigned qd = kk == 0 ? v.x : kk == 1 ? v.y : kk == 2 ? v.z : v.w;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const unsigned y = (qd >> (8 * i)) & 0xFFu;
+                const unsigned t = __builtin_amdgcn_bitop3_b32(__umul24(y, 0x40040u), 0x03C003C0u, 0x3C003C00u, 0xEA);   // (a & b) | c
+                w[i] = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, t), S16[b], C[b]));
             }
         }
-        // accumulator register r of lane l: row 8(r/4) + 4(l/32) + r%4 of
-        // the wave's 32, pair 32t + l%32 of the tile
+        return __builtin_bit_cast(f16x8, u32x4{w[0], w[1], w[2], w[3]});
+    };
+
+    // Step i issues the activations of step i + D - 1 and the quants (and at a
+    // super-block's first step the header) of step i + D.  Before step s the
+    // activations of step s and the quants of step s + 1 must have landed:
+    // everything issued up to step s - D + 1, so the D - 2 steps issued after
+    // it may stay in flight (any other memory operation in between only makes
+    // the wait longer).
+    copy_x(0, 0);
+    copy_q(0, 0);
+    copy_h(0);
+    copy_q(1, 1);
 #pragma unroll
-        for (int t = 0; t < NSUB; t++) {
-            const int pr = 32 * t + li;
-            if (pr < tl.n) {
-                const int p = po_s[pr];
-                const float sc = sc_s[pr];
-                if (MODE == 0) {
+    for (int i = 1; i <= D - 2; i++) {
+        copy_x(i, i);
+        copy_q(i + 1, i + 1);
+        if (i + 1 == 4) copy_h(1);
+    }
+    dma_wait_barrier_n<(D - 2) * (NB + 2) + (D >= 5 ? 1 : 0)>();
+    raw(0, 0, 0);
+    scales(0);
+    a[0][0] = frag(0, 0);
+    a[0][1] = frag(1, 0);
+    int xs = 0, qs = 0;   // slots of this step's activations and quants
+    const unsigned char *const xb0 = lx_p + li * 128;
+    const int xsw = mf_swz8(li);
+    for (int s0 = 0; s0 < nst; s0 += 4) {
 #pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        float a[4];
+        for (int s = 0; s < 4; s++) {
+            copy_x(xs == 0 ? D - 1 : xs - 1, s0 + s + D - 1);
+            copy_q(qs, s0 + s + D);
+            if ((s + D) % 4 == 0) copy_h((s0 + s + D) >> 2);
+            const int qn = qs == D - 1 ? 0 : qs + 1;
+            if (s == 2 && s0 + 4 >= nst && tid == 0) nxt = atomicAdd(ticket, 1) + (int)gridDim.x;
+            const unsigned char *xb = xb0 + xs * XS;
+            f16x8 bf[2][NB];
 #pragma unroll
-                        for (int c = 0; c < 4; c++) {
-                            const int r = 4 * h + c;
-                            const float g = acc[t][r] * sc, u = acc[t][r + 8] * sc;
-                            a[c] = g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
-                        }
-                        const int col = cb * PF_COLS + 16 * wave + 8 * h + 4 * lh;
-                        *reinterpret_cast<float4 *>(out + (long long)p * F + col) = make_float4(a[0], a[1], a[2], a[3]);
-                    }
+            for (int t = 0; t < NB; t++) bf[0][t] = *reinterpret_cast<const f16x8 *>(xb + t * 4096 + 16 * ((4 * lh) ^ xsw));
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) {
+                if (kk < 3) {
+#pragma unroll
+                    for (int t = 0; t < NB; t++)
+                        bf[(kk + 1) & 1][t] = *reinterpret_cast<const f16x8 *>(xb + t * 4096 + 16 * ((4 * lh + kk + 1) ^ xsw));
+                    a[(kk + 1) & 1][0] = frag(0, kk + 1);
+                    a[(kk + 1) & 1][1] = frag(1, kk + 1);
+                    if (kk == 2) raw((s + 1) & 3, qn, (s0 + s + 1) >> 2);
                 } else {
+                    scales((s + 1) & 3);
+                    a[0][0] = frag(0, 0);
+                    a[0][1] = frag(1, 0);
+                }
 #pragma unroll
-                    for (int h = 0; h < 4; h++) {
-                        const int row = cb * PF_ROWS + 32 * wave + 8 * h + 4 * lh;
-                        *reinterpret_cast<float4 *>(out + (long long)p * H + row) =
-                            make_float4(acc[t][4 * h] * sc, acc[t][4 * h + 1] * sc, acc[t][4 * h + 2] * sc,
-                                        acc[t][4 * h + 3] * sc);
+                for (int t = 0; t < NB; t++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+                        acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kk & 1][b], bf[kk & 1][t], acc[b][t], 0, 0, 0);
+                if constexpr (!GG && NB >= 3) {   // keep the decode between the MFMAs: run ahead, it spills
+#pragma unroll
+                    for (int i = 0; i < 2 * NB; i++) {
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, 7, 0);
                     }
                 }
             }
+            // steps s - D + 3 .. s (of the unrolled four) stay in flight
+            constexpr int base = (D - 2) * (NB + 2);
+            bool hdr = false;
+#pragma unroll
+            for (int i = 0; i < D - 2; i++) hdr = hdr || (s - i + D + 4) % 4 == 0;
+            if (hdr) dma_wait_barrier_n<base + 1>();
+            else dma_wait_barrier_n<base>();
+            xs = xs == D - 1 ? 0 : xs + 1;
+            qs = qn;
         }
-    };
-    switch ((tl.n + 31) / 32) {
-    case 1: body(PfSub<1>{}); break;
-    case 2: body(PfSub<2>{}); break;
-    case 3: body(PfSub<3>{}); break;
-    default: body(PfSub<4>{}); break;
     }
-    // the next item rewrites the activation buffers and the pair lists
-    if (tid == 0) next_item = nxt;
-    __syncthreads();
-    item = next_item;
+    // accumulator register r of lane l: row 8(r/4) + 4(l/32) + r%4 of the
+    // 32-row block, pair 32 t + l % 32 of the tile
+#pragma unroll
+    for (int t = 0; t < NB; t++) {
+        if (32 * t + li >= n) continue;
+        const float sc = xsc[32 * t + li];
+        float *o = out + (long long)tp[32 * t + li] * ldo + col + 4 * lh;
+        if constexpr (MODE == 0) {
+#pragma unroll
+            for (int g4 = 0; g4 < 4; g4++) {
+                float v[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const float g = acc[0][t][4 * g4 + c] * sc, u = acc[1][t][4 * g4 + c] * sc;
+                    v[c] = g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
+                }
+                *reinterpret_cast<float4 *>(o + 8 * g4) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+        } else {
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int g4 = 0; g4 < 4; g4++)
+                    *reinterpret_cast<float4 *>(o + 32 * b + 8 * g4) =
+                        make_float4(acc[b][t][4 * g4] * sc, acc[b][t][4 * g4 + 1] * sc, acc[b][t][4 * g4 + 2] * sc,
+                                    acc[b][t][4 * g4 + 3] * sc);
+        }
+    }
+}
+
+template <int MODE, bool GG>
+__global__ __launch_bounds__(64 * MF_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_moe_f16(
+    const uint8_t *__restrict__ W0, const uint8_t *__restrict__ W1, const _Float16 *__restrict__ X, int x_rows,
+    const float *__restrict__ xinv, const int *__restrict__ tpair, const int *__restrict__ ttok,
+    const PfTile *__restrict__ tiles, int *__restrict__ ntiles, int ncb, int H, int F, float *__restrict__ out) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char mf_lds_p[];
+    const int K = MODE == 0 ? H : F, nitems = *ntiles * ncb;
+    const uint32_t rb = (uint32_t)(K >> 8) * 144u;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    MfLists &ml = *reinterpret_cast<MfLists *>(mf_lds_p + MF_RING);
+    const dma_rsrc_t sr = dma_rsrc(xinv, (uint32_t)x_rows * 4u);
+    const int lane = threadIdx.x & 63;
+    for (int item = blockIdx.x; item < nitems;) {
+        const int tix = item / ncb, cb = item % ncb;
+        const PfTile tl = tiles[tix];
+        const int *xrows = (MODE == 0 ? ttok : tpair) + (long long)tix * PF_MT;
+        // the tile's pair ids and row scales to LDS for the epilogue (rows
+        // past its pairs: row 0's scale, not used)
+        if (wave < 2) {
+            const uint32_t r = (uint32_t)max(xrows[64 * wave + lane], 0);
+            dma4(lds_addr(ml.tp) + 256 * wave, 4u * (64 * wave + lane), dma_rsrc(tpair + (long long)tix * PF_MT, PF_MT * 4));
+            dma4(lds_addr(ml.xsc) + 256 * wave, 4u * r, sr);
+        }
+        const int e = __builtin_amdgcn_readfirstlane(tl.e), n = __builtin_amdgcn_readfirstlane(tl.n);
+        const int col = MODE == 0 ? cb * (MF_ROWS / 2) + 32 * wave : cb * MF_ROWS + 64 * wave;
+        const uint8_t *w0 = W0 + ((long long)e * (MODE == 0 ? F : H) + col) * rb;
+        const uint8_t *w1 = MODE == 0 ? W1 + ((long long)e * F + col) * rb : w0 + 32ll * rb;
+        int nxt = 0;
+        auto body = [&](auto nb) {
+            mf_item<MODE, GG, decltype(nb)::value>(mf_lds_p, w0, w1, rb, K, X, (uint32_t)x_rows * (uint32_t)(K * 2),
+                                                   xrows, ml.tp, ml.xsc, n, col, MODE == 0 ? F : H, out,
+                                                   ntiles + 1 + MODE, nxt);
+        };
+        switch ((n + 31) / 32) {   // uniform
+        case 1: body(PfSub<1>{}); break;
+        case 2: body(PfSub<2>{}); break;
+        case 3: body(PfSub<3>{}); break;
+        default: body(PfSub<4>{}); break;
+        }
+        // every wave is past its last read of the rings and lists when all
+        // have passed this barrier
+        if (threadIdx.x == 0) ml.next = nxt;
+        dma_wait_barrier();
+        item = __builtin_amdgcn_readfirstlane(ml.next);
     }
 }
 
@@ -634,10 +636,10 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_f16(const uint8_t *__restric
 // exchange per flush) and to 16 pairs, whose block scales are staged in LDS
 // per item.
 //
-// Items: (tile, 32-pair sub-tile, row block), otherwise the layout of
-// k_moe_f16 (8 waves x 32 weight rows, MODE 0 gate/up interleaved per wave,
-// activation tile double-buffered in LDS, one barrier per chunk); SwiGLU
-// takes a gate row's up partner from lane li + 16.
+// Items: (tile, 32-pair sub-tile, row block), on an 8-wave workgroup (32 weight
+// rows per wave, MODE 0 rows i < 16 gate and i >= 16 up of column 16 w + i %
+// 16, activation tile double-buffered in LDS, one barrier per chunk of 128
+// columns); SwiGLU takes a gate row's up partner from lane li + 16.
 // ---------------------------------------------------------------------------
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
@@ -979,26 +981,16 @@ static unsigned pf_grid(unsigned max_items) {
 }
 
 template <int MODE, bool GG>
-static hipError_t launch_moe_f16(int ns, unsigned nwg, hipStream_t st, const uint8_t *W0, const uint8_t *W1,
+static hipError_t launch_moe_f16(unsigned max_items, hipStream_t st, const uint8_t *W0, const uint8_t *W1,
                                  const _Float16 *X, int x_rows, const float *xinv, const int *tpair, const int *ttok,
                                  const PfTile *tiles, int *ntiles, int ncb, int H, int F, float *out) {
     // more than 64 KiB of dynamic LDS is opted into once per kernel
-#define TBQ_NS(N)                                                                                                  \
-    case N: {                                                                                                      \
-        static const hipError_t attr = hipFuncSetAttribute((const void *)k_moe_f16<MODE, N, GG>,                   \
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize,             \
-                                                           (int)PF_LDS_BYTES);                                     \
-        if (attr != hipSuccess) return attr;                                                                       \
-        hipLaunchKernelGGL((k_moe_f16<MODE, N, GG>), dim3(nwg), dim3(PF_THREADS), PF_LDS_BYTES, st, W0, W1, X,     \
-                           x_rows, xinv, tpair, ttok, tiles, ntiles, ncb, H, F, out);                              \
-        break;                                                                                                     \
-    }
-    switch (ns) {
-        TBQ_NS(2) TBQ_NS(4) TBQ_NS(6) TBQ_NS(8) TBQ_NS(12) TBQ_NS(16) TBQ_NS(24) TBQ_NS(32)
-    default:
-        return hipErrorNotSupported;
-    }
-#undef TBQ_NS
+    static const hipError_t attr =
+        hipFuncSetAttribute((const void *)k_moe_f16<MODE, GG>, hipFuncAttributeMaxDynamicSharedMemorySize, MF_LDS);
+    if (attr != hipSuccess) return attr;
+    const unsigned g = 2u * (unsigned)(tbq_cu_count() > 0 ? tbq_cu_count() : 256);   // two workgroups per CU
+    hipLaunchKernelGGL((k_moe_f16<MODE, GG>), dim3(max_items < g ? max_items : g), dim3(64 * MF_WAVES), MF_LDS, st, W0,
+                       W1, X, x_rows, xinv, tpair, ttok, tiles, ntiles, ncb, H, F, out);
     return hipGetLastError();
 }
 
@@ -1078,7 +1070,7 @@ hipError_t launch_moe_prefill_q4k_i8(const MoeArgs &a, void *scratch, hipStream_
 // same scale and conversion as k_rows_f16.
 template <int RW>
 __global__ __launch_bounds__(256) void k_rows_f16_wave(const float *__restrict__ in, int rows, int n,
-                                                       _Float16 *__restrict__ out, float *__restrict__ inv) {
+                                                       _Float16 *__restrict__ out, float *__restrict__ inv, bool swap) {
     const int lane = threadIdx.x & 63;
     const int row = min((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), rows - 1);   // past the end: redo the last
     const bool store = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6) < rows;
@@ -1103,33 +1095,33 @@ __global__ __launch_bounds__(256) void k_rows_f16_wave(const float *__restrict__
 #pragma unroll
     for (int i = 0; i < RW; i++) {
         if (lane + 64 * i < n4) {
-            const f16x2 a = {(_Float16)(v[i].x * s), (_Float16)(v[i].y * s)};
-            const f16x2 b = {(_Float16)(v[i].z * s), (_Float16)(v[i].w * s)};
+            const f16x2 a = {(_Float16)(v[i].x * s), (_Float16)((swap ? v[i].z : v[i].y) * s)};
+            const f16x2 b = {(_Float16)((swap ? v[i].y : v[i].z) * s), (_Float16)(v[i].w * s)};
             o[lane + 64 * i] = make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
         }
     }
     if (lane == 0) inv[row] = ldexpf(1.f, -sh);
 }
 
-hipError_t launch_rows_f16(const float *in, int rows, int n, _Float16 *out, float *inv, hipStream_t st) {
+hipError_t launch_rows_f16(const float *in, int rows, int n, _Float16 *out, float *inv, hipStream_t st, bool swap) {
     const int rw = (n / 4 + 63) / 64;   // float4 per lane with a wave per row
     const unsigned wgs = (unsigned)((rows + 3) / 4);
     if (rw <= 4) {
-        if (rw <= 1) hipLaunchKernelGGL(k_rows_f16_wave<1>, dim3(wgs), dim3(256), 0, st, in, rows, n, out, inv);
-        else if (rw <= 2) hipLaunchKernelGGL(k_rows_f16_wave<2>, dim3(wgs), dim3(256), 0, st, in, rows, n, out, inv);
-        else if (rw <= 3) hipLaunchKernelGGL(k_rows_f16_wave<3>, dim3(wgs), dim3(256), 0, st, in, rows, n, out, inv);
-        else hipLaunchKernelGGL(k_rows_f16_wave<4>, dim3(wgs), dim3(256), 0, st, in, rows, n, out, inv);
+        if (rw <= 1) hipLaunchKernelGGL(k_rows_f16_wave<1>, dim3(wgs), dim3(256), 0, st, in, rows, n, out, inv, swap);
+        else if (rw <= 2) hipLaunchKernelGGL(k_rows_f16_wave<2>, dim3(wgs), dim3(256), 0, st, in, rows, n, out, inv, swap);
+        else if (rw <= 3) hipLaunchKernelGGL(k_rows_f16_wave<3>, dim3(wgs), dim3(256), 0, st, in, rows, n, out, inv, swap);
+        else hipLaunchKernelGGL(k_rows_f16_wave<4>, dim3(wgs), dim3(256), 0, st, in, rows, n, out, inv, swap);
         return hipGetLastError();
     }
     const int rv = (n / 4 + 255) / 256;
     switch (rv) {
-    case 1: hipLaunchKernelGGL(k_rows_f16<1>, dim3(rows), dim3(256), 0, st, in, n, out, inv); break;
-    case 2: hipLaunchKernelGGL(k_rows_f16<2>, dim3(rows), dim3(256), 0, st, in, n, out, inv); break;
-    case 3: case 4: hipLaunchKernelGGL(k_rows_f16<4>, dim3(rows), dim3(256), 0, st, in, n, out, inv); break;
-    case 5: case 6: case 7: case 8: hipLaunchKernelGGL(k_rows_f16<8>, dim3(rows), dim3(256), 0, st, in, n, out, inv); break;
-    case 9: case 10: case 11: case 12: hipLaunchKernelGGL(k_rows_f16<12>, dim3(rows), dim3(256), 0, st, in, n, out, inv); break;
-    case 13: case 14: case 15: case 16: hipLaunchKernelGGL(k_rows_f16<16>, dim3(rows), dim3(256), 0, st, in, n, out, inv); break;
-    default: hipLaunchKernelGGL(k_rows_f16<0>, dim3(rows), dim3(256), 0, st, in, n, out, inv); break;
+    case 1: hipLaunchKernelGGL(k_rows_f16<1>, dim3(rows), dim3(256), 0, st, in, n, out, inv, swap); break;
+    case 2: hipLaunchKernelGGL(k_rows_f16<2>, dim3(rows), dim3(256), 0, st, in, n, out, inv, swap); break;
+    case 3: case 4: hipLaunchKernelGGL(k_rows_f16<4>, dim3(rows), dim3(256), 0, st, in, n, out, inv, swap); break;
+    case 5: case 6: case 7: case 8: hipLaunchKernelGGL(k_rows_f16<8>, dim3(rows), dim3(256), 0, st, in, n, out, inv, swap); break;
+    case 9: case 10: case 11: case 12: hipLaunchKernelGGL(k_rows_f16<12>, dim3(rows), dim3(256), 0, st, in, n, out, inv, swap); break;
+    case 13: case 14: case 15: case 16: hipLaunchKernelGGL(k_rows_f16<16>, dim3(rows), dim3(256), 0, st, in, n, out, inv, swap); break;
+    default: hipLaunchKernelGGL(k_rows_f16<0>, dim3(rows), dim3(256), 0, st, in, n, out, inv, swap); break;
     }
     return hipGetLastError();
 }
@@ -1138,7 +1130,8 @@ hipError_t launch_rows_f16(const float *in, int rows, int n, _Float16 *out, floa
 // Uses a.act (pairs x F fp32), a.y (pairs x H fp32) and `scratch`
 // (prefill_workspace_bytes).  H and F must be 256, 512, 768, 1024, 1536,
 // 2048, 3072 or 4096, H a multiple of PF_ROWS and F of PF_COLS; T <= 65536.
-void prefill_x16(const MoeArgs &a, void *scratch, _Float16 **x16, float **xinv) {
+void prefill_x16(const MoeArgs &a, void *scratch, _Float16 **x16, float **xinv, bool *swap) {
+    *swap = prefill_gq4k_layer(a);
     const size_t P = (size_t)a.T * a.k;
     const size_t max_tiles = (P + PF_MT - 1) / PF_MT + a.E;
     auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
@@ -1150,12 +1143,8 @@ void prefill_x16(const MoeArgs &a, void *scratch, _Float16 **x16, float **xinv) 
 }
 
 hipError_t launch_moe_prefill_q4k(const MoeArgs &a, void *scratch, hipStream_t st, bool x16_done) {
-    auto ok_k = [](int K) {
-        const int n = K / PF_KC;
-        return K % 256 == 0 && gemm_k_supported(K);
-    };
     const bool gg = prefill_gq4k_layer(a);
-    if (!(prefill_q4k_layer(a) || gg) || !ok_k(a.H) || !ok_k(a.F) || a.H % PF_ROWS || a.F % PF_COLS ||
+    if (!(prefill_q4k_layer(a) || gg) || !gemm_k_supported(a.H) || !gemm_k_supported(a.F) || a.H % MF_ROWS || a.F % (MF_ROWS / 2) ||
         a.T > 65536 || a.E > 256)
         return hipErrorNotSupported;
     const size_t P = (size_t)a.T * a.k;
@@ -1172,27 +1161,26 @@ hipError_t launch_moe_prefill_q4k(const MoeArgs &a, void *scratch, hipStream_t s
     float *ainv = (float *)w; w += up(P * 4);
     float *xinv = (float *)w;
     if (!x16_done) {
-        const hipError_t e = launch_rows_f16(a.xn, a.T, a.H, x16, xinv, st);
+        const hipError_t e = launch_rows_f16(a.xn, a.T, a.H, x16, xinv, st, gg);
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k_dispatch, dim3(1), dim3(1024), 0, st, a.sel_idx, a.T, a.k, a.E, perm, tiles, ntiles, tpair,
                        ttok);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    const int ncb0 = a.F / PF_COLS, ncb1 = a.H / PF_ROWS;
-    const unsigned g0 = pf_grid((unsigned)(max_tiles * ncb0)), g1 = pf_grid((unsigned)(max_tiles * ncb1));
+    const int ncb0 = a.F / (MF_ROWS / 2), ncb1 = a.H / MF_ROWS;
+    const unsigned m0 = (unsigned)(max_tiles * ncb0), m1 = (unsigned)(max_tiles * ncb1);
     const uint8_t *wg = (const uint8_t *)a.gate, *wu = (const uint8_t *)a.up, *wd = (const uint8_t *)a.down;
-    err = gg ? launch_moe_f16<0, true>(a.H / PF_KC, g0, st, wg, wu, x16, a.T, xinv, tpair, ttok, tiles, ntiles, ncb0,
-                                       a.H, a.F, a.act)
-             : launch_moe_f16<0, false>(a.H / PF_KC, g0, st, wg, wu, x16, a.T, xinv, tpair, ttok, tiles, ntiles,
-                                        ncb0, a.H, a.F, a.act);
+    err = gg ? launch_moe_f16<0, true>(m0, st, wg, wu, x16, a.T, xinv, tpair, ttok, tiles, ntiles, ncb0, a.H, a.F, a.act)
+             : launch_moe_f16<0, false>(m0, st, wg, wu, x16, a.T, xinv, tpair, ttok, tiles, ntiles, ncb0, a.H, a.F,
+                                        a.act);
     if (err != hipSuccess) return err;
-    err = launch_rows_f16(a.act, (int)P, a.F, act16, ainv, st);
+    err = launch_rows_f16(a.act, (int)P, a.F, act16, ainv, st, gg);
     if (err != hipSuccess) return err;
-    return gg ? launch_moe_f16<1, true>(a.F / PF_KC, g1, st, wd, nullptr, act16, (int)P, ainv, tpair, ttok, tiles,
-                                        ntiles, ncb1, a.H, a.F, a.y)
-              : launch_moe_f16<1, false>(a.F / PF_KC, g1, st, wd, nullptr, act16, (int)P, ainv, tpair, ttok, tiles,
-                                         ntiles, ncb1, a.H, a.F, a.y);
+    return gg ? launch_moe_f16<1, true>(m1, st, wd, nullptr, act16, (int)P, ainv, tpair, ttok, tiles, ntiles, ncb1, a.H,
+                                        a.F, a.y)
+              : launch_moe_f16<1, false>(m1, st, wd, nullptr, act16, (int)P, ainv, tpair, ttok, tiles, ntiles, ncb1,
+                                         a.H, a.F, a.y);
 }
 
 }  // namespace tbq

@@ -786,9 +786,9 @@ __device__ __forceinline__ void rb_store(const rb_f4 (&wr)[RB_WPT], const rb_f4 
 
 // One row of x to fp16 by one wave, scaled by the power of two that puts
 // its max |value| in [2^14, 2^15); xinv = the inverse scale.  The same
-// arithmetic as the prefill's k_rows_f16.  H a multiple of 256, <= 8192.
+// arithmetic (and swap) as the prefill's k_rows_f16.  H a multiple of 256, <= 8192.
 __device__ __forceinline__ void rb_row_f16(const float *__restrict__ x, int H, _Float16 *__restrict__ o,
-                                           float *__restrict__ inv) {
+                                           float *__restrict__ inv, bool swap) {
     const int lane = threadIdx.x & 63;
     const rb_f4 *r = reinterpret_cast<const rb_f4 *>(x);
     rb_f4 v[32];   // H / 256 float4 per lane
@@ -811,8 +811,8 @@ __device__ __forceinline__ void rb_row_f16(const float *__restrict__ x, int H, _
     for (int i = 0; i < 32; i++) {
         if (256 * i < H) {
             typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-            const h2 a = {(_Float16)(v[i].x * sc), (_Float16)(v[i].y * sc)};
-            const h2 b = {(_Float16)(v[i].z * sc), (_Float16)(v[i].w * sc)};
+            const h2 a = {(_Float16)(v[i].x * sc), (_Float16)((swap ? v[i].z : v[i].y) * sc)};
+            const h2 b = {(_Float16)((swap ? v[i].y : v[i].z) * sc), (_Float16)(v[i].w * sc)};
             out[lane + 64 * i] = make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
         }
     }
@@ -825,10 +825,10 @@ __device__ __forceinline__ void rb_row_f16(const float *__restrict__ x, int H, _
 __global__ __launch_bounds__(RB_THREADS) void k_router_batch(const float *__restrict__ xn, const float *__restrict__ Wr,
                                                              const float *__restrict__ bias, int T, int H, int E,
                                                              float *__restrict__ logits, _Float16 *__restrict__ x16,
-                                                             float *__restrict__ xinv) {
+                                                             float *__restrict__ xinv, bool swap) {
     if (x16 && blockIdx.y == gridDim.y - 1) {   // uniform
         const int t = blockIdx.x * RB_TOK + (int)(threadIdx.x >> 6);
-        if (t < T) rb_row_f16(xn + (long long)t * H, H, x16 + (long long)t * H, xinv + t);
+        if (t < T) rb_row_f16(xn + (long long)t * H, H, x16 + (long long)t * H, xinv + t, swap);
         return;
     }
     extern __shared__ rb_f4 rb_lds[];
@@ -895,11 +895,11 @@ struct RtlShared {
 __global__ __launch_bounds__(RTL_THREADS) void k_router_tile(const float *__restrict__ xn, const float *__restrict__ Wr,
                                                              const float *__restrict__ bias, int T, int H, int E,
                                                              float *__restrict__ logits, _Float16 *__restrict__ x16,
-                                                             float *__restrict__ xinv) {
+                                                             float *__restrict__ xinv, bool swap) {
     if (x16 && blockIdx.y == gridDim.y - 1) {   // uniform: the fp16 rows of this workgroup's 16 tokens
         for (int i = (int)(threadIdx.x >> 6); i < RTL_T; i += RTL_THREADS / 64) {
             const int t = blockIdx.x * RTL_T + i;
-            if (t < T) rb_row_f16(xn + (long long)t * H, H, x16 + (long long)t * H, xinv + t);
+            if (t < T) rb_row_f16(xn + (long long)t * H, H, x16 + (long long)t * H, xinv + t, swap);
         }
         return;
     }
@@ -1040,7 +1040,7 @@ static hipError_t launch_router_dpp(const float *xn, const float *router, const 
 // a top-k kernel.  hipErrorNotSupported when H does not fit either tiling.
 hipError_t launch_router(const float *xn, const float *router, const float *bias, int T, int H, int E, int top_k,
                          float *logits, unsigned *counters, int *sel_idx, float *sel_w, hipStream_t st,
-                         _Float16 *x16, float *xinv, bool *x16_done, const MoeArgs *group, bool *grouped) {
+                         _Float16 *x16, float *xinv, bool *x16_done, const MoeArgs *group, bool *grouped, bool x16_swap) {
     if (x16_done) *x16_done = false;
     if (grouped) *grouped = false;
     if (counters && T < 32 && (H == 2048 || H == 1024 || H == 512)) {
@@ -1063,7 +1063,7 @@ hipError_t launch_router(const float *xn, const float *router, const float *bias
         const bool rows = x16 && xinv && H <= 8192;
         hipLaunchKernelGGL(k_router_tile, dim3((T + RTL_T - 1) / RTL_T, E / RTL_E + (rows ? 1 : 0)),
                            dim3(RTL_THREADS), sizeof(RtlShared), st, xn, router, bias, T, H, E, logits,
-                           rows ? x16 : nullptr, xinv);
+                           rows ? x16 : nullptr, xinv, x16_swap);
         hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
         if (x16_done) *x16_done = rows;
@@ -1073,7 +1073,7 @@ hipError_t launch_router(const float *xn, const float *router, const float *bias
         const bool rows = x16 && xinv && H <= 8192;
         hipLaunchKernelGGL(k_router_batch, dim3((T + RB_TOK - 1) / RB_TOK, (E + 63) / 64 + (rows ? 1 : 0)),
                            dim3(RB_THREADS), sizeof(RbShared), st, xn, router, bias, T, H, E, logits,
-                           rows ? x16 : nullptr, xinv);
+                           rows ? x16 : nullptr, xinv, x16_swap);
         hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
         if (x16_done) *x16_done = rows;
