@@ -1006,7 +1006,7 @@ __global__ __launch_bounds__(S * G * 64) void k_mv_kq(const uint8_t *__restrict_
     constexpr int RL = GLU ? 1 : R;   // output rows per lane group and pass
     constexpr int RP = GLU ? 2 : R;   // weight rows per lane group and pass
     constexpr int NT = S * G * 64, RPP = 64 / LPR, RW = RL * RPP, RWG = G * RW, RWP = RP * RPP;
-    constexpr int MAXT = (16 * 64 * S + NT - 1) / NT;   // U <= 64 * S
+    constexpr int MAXT = (16 * LPR * S + NT - 1) / NT;   // U <= LPR * S
     extern __shared__ uint32_t smem[];
     const int U = K / 64;
     uint32_t *xd = smem;
@@ -1313,8 +1313,21 @@ static hipError_t launch_kq_q(const void *W, int M, int K, const float *x, float
             return launch_kq_seg<QT, KQ_SEG_NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
     if (U <= 4) return launch_kq_shape<QT, 4, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
     if (U <= 8) return launch_kq_shape<QT, 8, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
-    if (U <= 16) return launch_kq_shape<QT, 16, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
-    if (U <= 32) return launch_kq_shape<QT, 32, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
+    // Short matrices: where 16-wave workgroups of one pass would sit on at most
+    // half of the CUs, 4-wave ones spread the rows over four times as many
+    // (Q8_0, 256 CUs, K = 1024: gate|up with SwiGLU 2 x 3072 rows on 48
+    // workgroups, spilling under 128 registers, 12.4 -> 4.5 us; 2048 rows 5.1 ->
+    // 3.4; 1024 rows with the residual 5.0 -> 3.2; 1024x3072 5.0 -> 3.6); with
+    // more workgroups than that each CU stages x four times over for nothing
+    auto few = [&](int rows) { return 2 * (((long long)M + rows - 1) / rows) <= n_cu; };
+    if (U <= 16) {
+        if (few(NW * 4)) return launch_kq_shape<QT, 16, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
+        return launch_kq_shape<QT, 16, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
+    }
+    if (U <= 32) {
+        if (few(NW * 2)) return launch_kq_shape<QT, 32, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
+        return launch_kq_shape<QT, 32, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
+    }
     // Tall matrices of 64-unit rows: the segmented mapping, 16 rows per
     // workgroup pass (151936x4096: Q5_K 82.0 -> 79.5 us, Q2_K 59.4 -> 56.1,
     // Q8_0 65536x4096 52.5 -> 51.0; up to 24576 rows the row slices are as
@@ -1333,7 +1346,10 @@ static hipError_t launch_kq_q(const void *W, int M, int K, const float *x, float
     // 8.47 us at 9728x2560)
     if constexpr (QT != QT_Q8_0 && QT != QT_GQ8_0)
         if (U < 64 && (U & (U - 1)) != 0) return launch_kq_seg<QT, KQ_SEG_NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
-    if (U <= 64) return launch_kq_shape<QT, 64, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
+    if (U <= 64) {
+        if (few(NW)) return launch_kq_shape<QT, 64, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
+        return launch_kq_shape<QT, 64, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
+    }
     if (U <= 128) return launch_kq_shape<QT, 64, 2, NW / 2, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
     if (U <= 192) {
         // three slices: 5 row groups when that takes fewer passes than G3
