@@ -459,3 +459,42 @@ def test_moe_prefill_i8_small_batches(oracle, H, F, E, k):
         ref, ridx, rw = oracle.moe(xn, resid, router, gate, up, down, F=F, top_k=k, qtype=fm.Q4_K)
         assert np.array_equal(idx, ridx)
         assert rel_l2(out - resid, ref - resid) <= PREFILL_TOL
+
+
+# Every token takes the same k experts (a zero router under distinct biases), so
+# each expert's tile holds exactly T pairs: both sides of the 32-pair sub-tiles
+# and of the 128-pair tile, one super-block rows (the shortest ring), and the
+# shapes whose items take one and two row blocks per wave in either GEMM.
+@pytest.mark.parametrize("qt", [fm.Q4_K, fm.GGML | fm.Q4_K])
+@pytest.mark.parametrize("T,H,F,E,k", [
+    (1, 256, 512, 2, 1), (31, 512, 256, 3, 2), (33, 256, 256, 4, 2), (64, 768, 512, 2, 2), (65, 256, 768, 4, 1),
+    (97, 512, 256, 2, 1), (128, 256, 256, 3, 1), (129, 512, 256, 2, 2),
+    (33, 256, 4096, 64, 8), (129, 256, 4096, 64, 8), (97, 4096, 256, 128, 8),
+])
+def test_moe_prefill_tile_edges(oracle, qt, T, H, F, E, k):
+    import torch
+    _, gate, up, down = synth.moe_layer(H, F, E, qt, seed=T + H)
+    router = np.zeros((E, H), np.float32)
+    rng = np.random.default_rng(T * 3 + F)
+    bias = rng.permutation(E).astype(np.float32) * np.float32(0.25)
+    xn = synth.activations((T, H), rng)
+    resid = synth.activations((T, H), rng)
+    L = tb.moe_layer(H, F, E, k, qt, dev(router), dev(gate), dev(up), dev(down), dev(bias))
+    out, idx, w = empty((T + 1) * H, torch.float32), empty(T * 8, torch.int32), empty(T * 8, torch.float32)
+    out.fill_(7.0)
+    ws = torch.zeros(tb.moe_workspace_size(L, T, tb.TBQ_MOE_BF16), dtype=torch.uint8, device="cuda")
+    print("moe prefill tile edges", T, H, F, E, k, qt, flush=True)
+    for _ in range(2):   # the second call on the first one's workspace
+        tb.moe_forward(L, T, dev(xn), dev(resid), out, idx, w, workspace=ws, mode=tb.TBQ_MOE_BF16)
+    ref, ridx, rw = oracle.moe(xn, resid, router, gate, up, down, F=F, top_k=k, qtype=qt, bias=bias)
+    assert np.array_equal(host(idx).reshape(T, 8), ridx)
+    assert bits_equal(host(w).reshape(T, 8), rw)
+    got = host(out).reshape(T + 1, H)
+    assert np.all(got[T] == 7.0)
+    # The mode's bound over the layer, and the same per token against the tokens'
+    # typical size: fp16 operands err by 2^-11 of the sum of |w||x|, which tokens
+    # share, and these weights' nonzero mean makes some tokens' sums cancel to a
+    # fraction of it.  A token in a wrong slot would be off by its whole size.
+    d, r = got[:T] - ref, ref - resid
+    assert np.linalg.norm(d) <= 1e-2 * np.linalg.norm(r)
+    assert np.linalg.norm(d, axis=1).max() <= 3e-2 * np.sqrt(np.mean(np.sum(r * r, axis=1)))

@@ -83,9 +83,10 @@ struct PfSub {
 // ---------------------------------------------------------------------------
 constexpr int PF_MAX_TILES = 65536 * 8 / PF_MT + 256;
 // up to this many pairs, k_dispatch keeps the expert indices in registers
-// (read once) and the permutation in LDS: a permutation in global memory is
-// read back, after its own stores, by a loop of dependent round trips
-constexpr int PF_LDS_PAIRS = 8192;
+// (read once) and the permutation in LDS (16 bits a pair): a permutation in
+// global memory is read back, after its own stores, by a loop of dependent
+// round trips (15992 pairs: 31 -> 19.5 us)
+constexpr int PF_LDS_PAIRS = 16384, PF_LDS_TILES = PF_LDS_PAIRS / PF_MT + 256;
 
 __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_idx, int T, int k, int E,
                                                    int *__restrict__ perm, PfTile *__restrict__ tiles,
@@ -95,11 +96,14 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_i
     static_assert(PF_MT == 128 && NQ == 4, "tile classes");
     __shared__ int hist[256], off[257], cur[256], wsum[4];
     __shared__ int qcnt[NQ + 1], qbase[NQ + 2];
-    __shared__ int t_e[PF_MAX_TILES], t_start[PF_MAX_TILES];
-    __shared__ int perm_s[PF_LDS_PAIRS];
+    // the tile list, and where the pairs fit the permutation behind it
+    constexpr int SMALL = 2 * PF_LDS_TILES + PF_LDS_PAIRS / 2;
+    __shared__ int lists[SMALL > 2 * PF_MAX_TILES ? SMALL : 2 * PF_MAX_TILES];
     constexpr int NE = PF_LDS_PAIRS / 1024;   // expert indices per thread
     const int tid = threadIdx.x, P = T * k;
     const bool small = P <= PF_LDS_PAIRS;   // uniform
+    int *t_e = lists, *t_start = lists + (small ? PF_LDS_TILES : PF_MAX_TILES);
+    unsigned short *perm_s = reinterpret_cast<unsigned short *>(lists + 2 * PF_LDS_TILES);
     if (tid < 256) { hist[tid] = 0; cur[tid] = 0; }
     if (tid <= NQ) qcnt[tid] = 0;
     int es[NE];
@@ -188,7 +192,7 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_i
 #pragma unroll
         for (int m = 0; m < NE; m++) {
             const int e = es[m];
-            if ((unsigned)e < (unsigned)E) perm_s[off[e] + atomicAdd(&cur[e], 1)] = tid + 1024 * m;
+            if ((unsigned)e < (unsigned)E) perm_s[off[e] + atomicAdd(&cur[e], 1)] = (unsigned short)(tid + 1024 * m);
         }
     } else {
         for (int p = tid; p < P; p += 1024) {
@@ -270,7 +274,7 @@ __device__ __forceinline__ float h2f(unsigned bits) {
 
 // ---------------------------------------------------------------------------
 // Expert tile GEMM.  Work items are (tile, row block) pairs, tile-major (ncb =
-// F/128 row blocks of 128 columns for MODE 0, H/256 of 256 rows for MODE 1),
+// F / (64 NA) row blocks of columns for MODE 0, H / (128 NA) of rows for MODE 1),
 // the tiles heaviest first.  The grid is persistent (two workgroups of four
 // waves per CU): workgroup b starts with item b, then takes tickets from the
 // counter ntiles[1 + MODE] (zeroed by k_dispatch): item grid + ticket, the
@@ -281,11 +285,12 @@ __device__ __forceinline__ float h2f(unsigned bits) {
 // to whichever workgroup is about to be free (greedy list scheduling); a fixed stride over the items left the workgroups that drew
 // heavy items 30% busier than the mean.
 //
-// Wave w owns 64 weight rows in two 32-row blocks: MODE 0 gate and up of the
-// columns 128 cb + 32 w .. + 31 (so SwiGLU pairs the two blocks' accumulators),
-// MODE 1 the down rows 256 cb + 64 w .. + 63; and all of the tile's pairs, in
-// NB 32-pair sub-tiles.  X rows are tokens (ttok) of x in MODE 0, pairs (tpair)
-// of act in MODE 1; xinv[X row] undoes the row's fp16 scaling.
+// Wave w owns NA 32-row blocks of weight rows and all of the tile's pairs, in NB
+// 32-pair sub-tiles.  MODE 0: NA = 2 gate and up of 32 columns, one block each;
+// NA = 1 gate (rows 0..15) and up (16..31) of 16 columns; either way SwiGLU pairs
+// accumulators of one lane.  MODE 1: 32 NA down rows.  X rows are tokens (ttok)
+// of x in MODE 0, pairs (tpair) of act in MODE 1; xinv[X row] undoes the row's
+// fp16 scaling.
 //
 // K advances 64 columns (two Q4_K sub-blocks) a step.  Packed quants (32 bytes
 // a row), headers and activation rows are copied directly to LDS (tbq_dma.hpp)
@@ -301,15 +306,14 @@ __device__ __forceinline__ float h2f(unsigned bits) {
 // ^ swizzle(row), so column reads spread over all banks.
 //
 // Against one 8-wave workgroup per CU whose lanes loaded their own rows' bytes
-// (32 rows per wave, so twice the LDS reads per MFMA), Qwen3-30B-A3B layer: T =
-// 512 Zipf-skewed gate/up 87.5 -> 72 us and down 46.6 -> 55 us (its 12 steps
-// are short against an item's start), 1999 tokens of ggml's layout 330 -> 267
-// us for the two.  Left: 512 tokens read 204 + 153 MB (39 + 29 us at the copy
-// rate) while the heaviest experts' tiles, which set the end, wait for the same
-// memory; without copies the two take 88 us, without the dequantisation as
-// well 71.
+// (a cache line per lane and load), whole layer: 60 tokens of 32 experts 55.3 ->
+// 43.7 us, 300 of 128 91.1 -> 79.5, Qwen3-30B-A3B with 512 Zipf-skewed tokens
+// 176.4 -> 166.6, 1999 of ggml's layout 433 -> 391.  Left at 512 tokens: 204 +
+// 153 MB read (39 + 29 us at the copy rate) while the heaviest experts' tiles,
+// which set the end, wait for the same memory; at NA = 2 the two GEMMs take 127
+// us, without copies 88, without the dequantisation as well 71.
 // ---------------------------------------------------------------------------
-constexpr int MF_WAVES = 4, MF_ROWS = 64 * MF_WAVES;
+constexpr int MF_WAVES = 4, MF_ROWS = 64 * MF_WAVES;   // rows at two blocks per wave
 constexpr int mf_depth(int nb) { return nb == 1 ? 5 : nb == 2 ? 4 : 3; }
 // header slots: at D = 5 the next super-block's copy is issued in the step that
 // reads the current one's, at D <= 4 after it
@@ -331,11 +335,11 @@ __device__ __forceinline__ int mf_swz2(int r) { return ((r >> 2) ^ (r >> 3)) & 1
 // One item for a compile-time count of sub-tiles.  w0, w1: the wave's blocks'
 // rows (32 rows of rb bytes each); xrows: the tile's X rows; tp, xsc: its pair
 // ids and X row scales in LDS.
-template <int MODE, bool GG, int NB>
+template <int MODE, bool GG, int NA, int NB>
 __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, const uint8_t *w1, uint32_t rb, int K,
                                         const _Float16 *X, uint32_t xbytes, const int *xrows, const int *tp,
                                         const float *xsc, int n, int col, int ldo, float *out, int *ticket, int &nxt) {
-    constexpr int D = mf_depth(NB), HD = mf_hdrs(NB), XS = NB * 32 * 128, QS = MF_ROWS * 32;
+    constexpr int D = mf_depth(NB), HD = mf_hdrs(NB), XS = NB * 32 * 128, QS = MF_WAVES * NA * 32 * 32;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31,
               lh = lane >> 5;
     unsigned char *const lh_p = lds, *const lq_p = lds + HD * MF_ROWS * 16, *const lx_p = lq_p + D * QS;
@@ -352,39 +356,44 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
     const dma_rsrc_t r0 = dma_rsrc(w0, 32 * rb), r1 = dma_rsrc(w1, 32 * rb);
     // quant copies: 32 rows x 2 segments each, one per block and step
     const uint32_t qv = (uint32_t)(lane >> 1) * rb + 16u + 16u * ((lane & 1) ^ mf_swz2(lane >> 1));
-    // header copy: lane = row of block 0, then of block 1
-    const uint8_t *hp = (lane < 32 ? w0 : w1) + (uint32_t)li * rb;
-    const uint32_t ax = lds_addr(lx_p) + wave * 1024, aq = lds_addr(lq_p) + wave * 2048, ah = lds_addr(lh_p) + wave * 1024;
+    // header copy: lane = row of block 0, then of block 1 (NA = 1: of the one
+    // block again).  NA = 1, MODE 0: the block's rows are 16 of w0, then 16 of w1
+    constexpr bool MIX = NA == 1 && MODE == 0;
+    const uint8_t *hp = MIX ? (li < 16 ? w0 : w1) + (uint32_t)(li & 15) * rb
+                            : (lane < 32 || NA == 1 ? w0 : w1) + (uint32_t)li * rb;
+    const uint8_t *qp = (lane < 32 ? w0 : w1) + (uint32_t)((lane >> 1) & 15) * rb + 16 + 16 * ((lane & 1) ^ mf_swz2(lane >> 1));
+    const uint32_t ax = lds_addr(lx_p) + wave * 1024, aq = lds_addr(lq_p) + wave * (NA * 1024), ah = lds_addr(lh_p) + wave * 1024;
     auto copy_x = [&](int slot, int step) {
 #pragma unroll
         for (int i = 0; i < NB; i++) dma16(ax + slot * XS + MF_WAVES * i * 1024, xv[i], xr, min(step, nst - 1) * 128);
     };
     auto copy_q = [&](int slot, int step) {   // steps past the end: empty descriptors, no memory access
         const uint32_t so = (min(step, nst - 1) >> 2) * 144 + (step & 3) * 32;
-        dma16(aq + slot * QS, qv, r0, so);
-        dma16(aq + slot * QS + 1024, qv, r1, so);
+        if constexpr (MIX) dma16_ptr(aq + slot * QS, qp + so);
+        else dma16(aq + slot * QS, qv, r0, so);
+        if constexpr (NA == 2) dma16(aq + slot * QS + 1024, qv, r1, so);
     };
     auto copy_h = [&](int sb) { dma16_ptr(ah + sb % HD * (MF_ROWS * 16), hp + min(sb, (nst >> 2) - 1) * 144); };
 
-    f32x16 acc[2][NB];
+    f32x16 acc[NA][NB];
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+    for (int b = 0; b < NA; b++)
 #pragma unroll
         for (int t = 0; t < NB; t++) acc[b][t] = f32x16{};
 
     constexpr int QR = GG ? 2 : 1;   // 16-byte quant reads per lane and step
-    u32x4 hd[2], q[2][QR];
-    uint32_t mhi[2];
-    f16x2 S16[2], C[2];
-    f16x8 a[2][2];
-    const int wrow = wave * 64 + li, qsw = mf_swz2(li);
+    u32x4 hd[NA], q[NA][QR];
+    uint32_t mhi[NA];
+    f16x2 S16[NA], C[NA];
+    f16x8 a[2][NA];
+    const int wrow = wave * (32 * NA) + li, qsw = mf_swz2(li);
     // the raw bytes of step s (of its super-block), whose quants sit in slot
     auto raw = [&](int s, int slot, int sb) {
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
+        for (int b = 0; b < NA; b++) {
             const unsigned char *qrow = lq_p + slot * QS + (wrow + 32 * b) * 32;
             if (s == 0) {
-                hd[b] = *reinterpret_cast<const u32x4 *>(lh_p + sb % HD * (MF_ROWS * 16) + (wrow + 32 * b) * 16);
+                hd[b] = *reinterpret_cast<const u32x4 *>(lh_p + sb % HD * (MF_ROWS * 16) + (wave * 64 + 32 * b + li) * 16);
                 // the reference's mins of sub-blocks 4..7 are quant bytes 0..3 (layer4/tb_gguf.c:163-168)
                 if constexpr (!GG) mhi[b] = *reinterpret_cast<const uint32_t *>(qrow + 16 * qsw);
             }
@@ -399,7 +408,7 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
     // 16 S and C = -16 S - M of the lane's sub-block 2 s + lh
     auto scales = [&](int s) {
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
+        for (int b = 0; b < NA; b++) {
             const int jb = 16 * (s & 1) + 8 * lh;
             uint32_t sc, mn;
             if constexpr (GG) {   // ggml's get_scale_min_k4
@@ -465,11 +474,11 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
         copy_q(i + 1, i + 1);
         if (i + 1 == 4) copy_h(1);
     }
-    dma_wait_barrier_n<(D - 2) * (NB + 2) + (D >= 5 ? 1 : 0)>();
+    dma_wait_barrier_n<(D - 2) * (NB + NA) + (D >= 5 ? 1 : 0)>();
     raw(0, 0, 0);
     scales(0);
-    a[0][0] = frag(0, 0);
-    a[0][1] = frag(1, 0);
+#pragma unroll
+    for (int b = 0; b < NA; b++) a[0][b] = frag(b, 0);
     int xs = 0, qs = 0;   // slots of this step's activations and quants
     const unsigned char *const xb0 = lx_p + li * 128;
     const int xsw = mf_swz8(li);
@@ -491,22 +500,22 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
 #pragma unroll
                     for (int t = 0; t < NB; t++)
                         bf[(kk + 1) & 1][t] = *reinterpret_cast<const f16x8 *>(xb + t * 4096 + 16 * ((4 * lh + kk + 1) ^ xsw));
-                    a[(kk + 1) & 1][0] = frag(0, kk + 1);
-                    a[(kk + 1) & 1][1] = frag(1, kk + 1);
+#pragma unroll
+                    for (int b = 0; b < NA; b++) a[(kk + 1) & 1][b] = frag(b, kk + 1);
                     if (kk == 2) raw((s + 1) & 3, qn, (s0 + s + 1) >> 2);
                 } else {
                     scales((s + 1) & 3);
-                    a[0][0] = frag(0, 0);
-                    a[0][1] = frag(1, 0);
+#pragma unroll
+                    for (int b = 0; b < NA; b++) a[0][b] = frag(b, 0);
                 }
 #pragma unroll
                 for (int t = 0; t < NB; t++)
 #pragma unroll
-                    for (int b = 0; b < 2; b++)
+                    for (int b = 0; b < NA; b++)
                         acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kk & 1][b], bf[kk & 1][t], acc[b][t], 0, 0, 0);
-                if constexpr (!GG && NB >= 3) {   // keep the decode between the MFMAs: run ahead, it spills
+                if constexpr (!GG && NA == 2 && NB >= 3) {   // keep the decode between the MFMAs: run ahead, it spills
 #pragma unroll
-                    for (int i = 0; i < 2 * NB; i++) {
+                    for (int i = 0; i < NA * NB; i++) {
                         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
                         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                         __builtin_amdgcn_sched_group_barrier(0x2, 7, 0);
@@ -514,7 +523,7 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
                 }
             }
             // steps s - D + 3 .. s (of the unrolled four) stay in flight
-            constexpr int base = (D - 2) * (NB + 2);
+            constexpr int base = (D - 2) * (NB + NA);
             bool hdr = false;
 #pragma unroll
             for (int i = 0; i < D - 2; i++) hdr = hdr || (s - i + D + 4) % 4 == 0;
@@ -533,18 +542,18 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
         float *o = out + (long long)tp[32 * t + li] * ldo + col + 4 * lh;
         if constexpr (MODE == 0) {
 #pragma unroll
-            for (int g4 = 0; g4 < 4; g4++) {
+            for (int g4 = 0; g4 < 2 * NA; g4++) {   // NA = 1: the up rows are the block's second half
                 float v[4];
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    const float g = acc[0][t][4 * g4 + c] * sc, u = acc[1][t][4 * g4 + c] * sc;
+                    const float g = acc[0][t][4 * g4 + c] * sc, u = acc[NA - 1][t][4 * g4 + c + (NA == 1 ? 8 : 0)] * sc;
                     v[c] = g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
                 }
                 *reinterpret_cast<float4 *>(o + 8 * g4) = make_float4(v[0], v[1], v[2], v[3]);
             }
         } else {
 #pragma unroll
-            for (int b = 0; b < 2; b++)
+            for (int b = 0; b < NA; b++)
 #pragma unroll
                 for (int g4 = 0; g4 < 4; g4++)
                     *reinterpret_cast<float4 *>(o + 32 * b + 8 * g4) =
@@ -554,7 +563,7 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
     }
 }
 
-template <int MODE, bool GG>
+template <int MODE, bool GG, int NA>
 __global__ __launch_bounds__(64 * MF_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_moe_f16(
     const uint8_t *__restrict__ W0, const uint8_t *__restrict__ W1, const _Float16 *__restrict__ X, int x_rows,
     const float *__restrict__ xinv, const int *__restrict__ tpair, const int *__restrict__ ttok,
@@ -578,12 +587,12 @@ __global__ __launch_bounds__(64 * MF_WAVES) __attribute__((amdgpu_waves_per_eu(2
             dma4(lds_addr(ml.xsc) + 256 * wave, 4u * r, sr);
         }
         const int e = __builtin_amdgcn_readfirstlane(tl.e), n = __builtin_amdgcn_readfirstlane(tl.n);
-        const int col = MODE == 0 ? cb * (MF_ROWS / 2) + 32 * wave : cb * MF_ROWS + 64 * wave;
+        const int col = (cb * MF_WAVES + wave) * (MODE == 0 ? 16 : 32) * NA;
         const uint8_t *w0 = W0 + ((long long)e * (MODE == 0 ? F : H) + col) * rb;
         const uint8_t *w1 = MODE == 0 ? W1 + ((long long)e * F + col) * rb : w0 + 32ll * rb;
         int nxt = 0;
         auto body = [&](auto nb) {
-            mf_item<MODE, GG, decltype(nb)::value>(mf_lds_p, w0, w1, rb, K, X, (uint32_t)x_rows * (uint32_t)(K * 2),
+            mf_item<MODE, GG, NA, decltype(nb)::value>(mf_lds_p, w0, w1, rb, K, X, (uint32_t)x_rows * (uint32_t)(K * 2),
                                                    xrows, ml.tp, ml.xsc, n, col, MODE == 0 ? F : H, out,
                                                    ntiles + 1 + MODE, nxt);
         };
@@ -980,18 +989,38 @@ static unsigned pf_grid(unsigned max_items) {
     return max_items < g ? max_items : g;
 }
 
-template <int MODE, bool GG>
-static hipError_t launch_moe_f16(unsigned max_items, hipStream_t st, const uint8_t *W0, const uint8_t *W1,
+template <int MODE, bool GG, int NA>
+static hipError_t launch_moe_f16_na(unsigned max_items, hipStream_t st, const uint8_t *W0, const uint8_t *W1,
                                  const _Float16 *X, int x_rows, const float *xinv, const int *tpair, const int *ttok,
                                  const PfTile *tiles, int *ntiles, int ncb, int H, int F, float *out) {
     // more than 64 KiB of dynamic LDS is opted into once per kernel
     static const hipError_t attr =
-        hipFuncSetAttribute((const void *)k_moe_f16<MODE, GG>, hipFuncAttributeMaxDynamicSharedMemorySize, MF_LDS);
+        hipFuncSetAttribute((const void *)k_moe_f16<MODE, GG, NA>, hipFuncAttributeMaxDynamicSharedMemorySize, MF_LDS);
     if (attr != hipSuccess) return attr;
     const unsigned g = 2u * (unsigned)(tbq_cu_count() > 0 ? tbq_cu_count() : 256);   // two workgroups per CU
-    hipLaunchKernelGGL((k_moe_f16<MODE, GG>), dim3(max_items < g ? max_items : g), dim3(64 * MF_WAVES), MF_LDS, st, W0,
+    hipLaunchKernelGGL((k_moe_f16<MODE, GG, NA>), dim3(max_items < g ? max_items : g), dim3(64 * MF_WAVES), MF_LDS, st, W0,
                        W1, X, x_rows, xinv, tpair, ttok, tiles, ntiles, ncb, H, F, out);
     return hipGetLastError();
+}
+
+template <int MODE, bool GG>
+static hipError_t launch_moe_f16(const MoeArgs &a, int max_tiles, hipStream_t st, const uint8_t *W0, const uint8_t *W1, const _Float16 *X,
+                                 int x_rows, const float *xinv, const int *tpair, const int *ttok, const PfTile *tiles,
+                                 int *ntiles, int H, int F, float *out) {
+    const int n2 = MODE == 0 ? F / (MF_ROWS / 2) : H / MF_ROWS;   // row blocks at NA = 2
+    // Row blocks per wave.  One is better while the items (about P / 128 + E / 2
+    // tiles) are fewer than two rounds of the 512 workgroup slots: twice the
+    // items of half the length fill the chip and hide a step's latencies (60
+    // tokens, 32 experts 52.7 -> 43.7 us a layer, 128 tokens 63.9 -> 50.8, 512
+    // Zipf-skewed of 128 experts 173 -> 166.6); two read the activations half as
+    // often and decode between twice the MFMAs (1999 tokens of 128 experts 401
+    // against 391 us with one; 1500 of 64 the same).
+    const long long P = (long long)a.T * a.k, tiles_est = P / PF_MT + (P < a.E ? P : a.E) / 2;
+    if (tiles_est * n2 <= 1024)
+        return launch_moe_f16_na<MODE, GG, 1>((unsigned)(2 * max_tiles * n2), st, W0, W1, X, x_rows, xinv, tpair, ttok,
+                                              tiles, ntiles, 2 * n2, H, F, out);
+    return launch_moe_f16_na<MODE, GG, 2>((unsigned)(max_tiles * n2), st, W0, W1, X, x_rows, xinv, tpair, ttok, tiles,
+                                          ntiles, n2, H, F, out);
 }
 
 // K values the MFMA kernel is instantiated for (K = 128 * NS).
@@ -1168,19 +1197,14 @@ hipError_t launch_moe_prefill_q4k(const MoeArgs &a, void *scratch, hipStream_t s
                        ttok);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    const int ncb0 = a.F / (MF_ROWS / 2), ncb1 = a.H / MF_ROWS;
-    const unsigned m0 = (unsigned)(max_tiles * ncb0), m1 = (unsigned)(max_tiles * ncb1);
     const uint8_t *wg = (const uint8_t *)a.gate, *wu = (const uint8_t *)a.up, *wd = (const uint8_t *)a.down;
-    err = gg ? launch_moe_f16<0, true>(m0, st, wg, wu, x16, a.T, xinv, tpair, ttok, tiles, ntiles, ncb0, a.H, a.F, a.act)
-             : launch_moe_f16<0, false>(m0, st, wg, wu, x16, a.T, xinv, tpair, ttok, tiles, ntiles, ncb0, a.H, a.F,
-                                        a.act);
+    err = gg ? launch_moe_f16<0, true>(a, max_tiles, st, wg, wu, x16, a.T, xinv, tpair, ttok, tiles, ntiles, a.H, a.F, a.act)
+             : launch_moe_f16<0, false>(a, max_tiles, st, wg, wu, x16, a.T, xinv, tpair, ttok, tiles, ntiles, a.H, a.F, a.act);
     if (err != hipSuccess) return err;
     err = launch_rows_f16(a.act, (int)P, a.F, act16, ainv, st, gg);
     if (err != hipSuccess) return err;
-    return gg ? launch_moe_f16<1, true>(m1, st, wd, nullptr, act16, (int)P, ainv, tpair, ttok, tiles, ntiles, ncb1, a.H,
-                                        a.F, a.y)
-              : launch_moe_f16<1, false>(m1, st, wd, nullptr, act16, (int)P, ainv, tpair, ttok, tiles, ntiles, ncb1,
-                                         a.H, a.F, a.y);
+    return gg ? launch_moe_f16<1, true>(a, max_tiles, st, wd, nullptr, act16, (int)P, ainv, tpair, ttok, tiles, ntiles, a.H, a.F, a.y)
+              : launch_moe_f16<1, false>(a, max_tiles, st, wd, nullptr, act16, (int)P, ainv, tpair, ttok, tiles, ntiles, a.H, a.F, a.y);
 }
 
 }  // namespace tbq
