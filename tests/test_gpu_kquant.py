@@ -147,6 +147,19 @@ def test_matvec_kq_kernel(oracle, qt, M, K):
     assert rel_l2(gpu_matvec(W, qt, M, K, x, tb.TBQ_MV_KQ), oracle.matvec(W, qt, M, K, x)) <= MATVEC_TOL
 
 
+@pytest.mark.parametrize("qt", [fm.Q3_K, fm.Q4_K, fm.Q6_K, fm.Q8_0, fm.GGML | fm.Q4_K])
+@pytest.mark.parametrize("M,K", [(63, 1024), (8192, 1024), (8193, 1024), (4096, 2048), (4097, 2048), (17, 4096),
+                                 (2048, 4096), (2049, 4096)])
+def test_matvec_kq_short_matrices(oracle, qt, M, K):
+    """Rows of 16, 32 and 64 units on both sides of the row count where
+    workgroups of 16 waves would leave half the compute units without one
+    (256 units of 64, 32 and 16 rows), where 4-wave workgroups take over."""
+    rng = np.random.default_rng(M * 17 + K + 3 * (qt & 255))
+    W = synth.kquant_matrix(qt, M, K, rng)
+    x = synth.activations(K, rng)
+    assert rel_l2(gpu_matvec(W, qt, M, K, x, tb.TBQ_MV_KQ), oracle.matvec(W, qt, M, K, x)) <= MATVEC_TOL
+
+
 @pytest.mark.parametrize("qt", KQ_FORMATS)
 @pytest.mark.parametrize("M,K", [(5, 2560), (26, 2304), (777, 3072), (2000, 3840), (6144, 2560), (300, 1280),
                                  (8960, 1536), (43, 1792)])

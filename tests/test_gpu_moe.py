@@ -498,3 +498,28 @@ def test_moe_prefill_tile_edges(oracle, qt, T, H, F, E, k):
     d, r = got[:T] - ref, ref - resid
     assert np.linalg.norm(d) <= 1e-2 * np.linalg.norm(r)
     assert np.linalg.norm(d, axis=1).max() <= 3e-2 * np.sqrt(np.mean(np.sum(r * r, axis=1)))
+
+
+# Experts of very different loads, so the int8 items of one launch come from
+# tiles of all four sub-tile counts: full tiles, remainders on both sides of a
+# sub-tile, and experts with no pair at all.
+@pytest.mark.parametrize("T,H,F,E,k,spread", [(37, 256, 256, 16, 2, 4.0), (150, 512, 256, 24, 3, 3.0),
+                                              (400, 256, 512, 16, 2, 3.0)])
+def test_moe_prefill_int8_mixed_tiles(oracle, T, H, F, E, k, spread):
+    import torch
+    router, gate, up, down = synth.moe_layer(H, F, E, fm.Q4_K, seed=T + E)
+    rng = np.random.default_rng(T + 5 * E)
+    xn, resid = synth.activations((T, H), rng), synth.activations((T, H), rng)
+    bias = (np.linspace(-spread, spread, E) * np.std(xn @ router.T)).astype(np.float32)
+    ref, ridx, rw = oracle.moe(xn, resid, router, gate, up, down, F=F, top_k=k, qtype=fm.Q4_K, bias=bias)
+    n = np.bincount(ridx[:, :k].ravel(), minlength=E)
+    classes = {(int(c) % 128 + 31) // 32 for c in n if c % 128} | {4 for c in n if c >= 128}
+    assert n.min() == 0 and len(classes) >= min(T // 50, 4)
+    L = tb.moe_layer(H, F, E, k, fm.Q4_K, dev(router), dev(gate), dev(up), dev(down), dev(bias))
+    out, idx, w = empty(T * H, torch.float32), empty(T * 8, torch.int32), empty(T * 8, torch.float32)
+    ws = torch.zeros(tb.moe_workspace_size(L, T, tb.TBQ_MOE_I8), dtype=torch.uint8, device="cuda")
+    print("moe int8 mixed tiles", T, H, F, E, k, sorted(n), flush=True)
+    for _ in range(2):
+        tb.moe_forward(L, T, dev(xn), dev(resid), out, idx, w, workspace=ws, mode=tb.TBQ_MOE_I8)
+    assert np.array_equal(host(idx).reshape(T, 8)[:, :k], ridx[:, :k])
+    assert rel_l2(host(out).reshape(T, H) - resid, ref - resid) <= PREFILL_TOL

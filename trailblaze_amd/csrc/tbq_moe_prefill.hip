@@ -170,6 +170,7 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_i
         for (int q = NQ; q >= 1; q--) {
             qbase[q] = b;
             b += qcnt[q];
+            ntiles[3 + NQ - q] = qcnt[q];   // tiles of NQ, NQ - 1 .. 1 sub-tiles (k_moe_i8's items)
             qcnt[q] = 0;
         }
         *ntiles = b;
@@ -767,7 +768,8 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict
                                                        int ncb, int H, int F, float *__restrict__ out) {
     constexpr int K = NS * PF_KC;
     constexpr int NSB = K / 256;
-    constexpr int NQ = PF_MT / I8_MT;   // sub-tiles per tile
+    constexpr int NQ = PF_MT / I8_MT;   // sub-tiles per tile, as k_dispatch counts them
+    static_assert(I8_MT == 32, "sub-tile classes");
     // weight chunks loaded ahead: 3 for long rows (two spill at K = 768)
     constexpr int AH = NS >= 8 ? I8_AHEAD : 2;
     extern __shared__ __attribute__((aligned(16))) int8_t i8_lds[];   // [2][I8_MT][2][I8_LD]
@@ -780,12 +782,35 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict
     const long long rb = (long long)(K / 256) * 144;
     const int xbytes = x_rows * 2 * K;
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void *)X, (short)0, xbytes, 0x00020000);
-    const int nitems = *ntiles * NQ * ncb;
+    // Items are the sub-tiles that exist, tiles in their heaviest-first order (c[i]
+    // tiles of NQ - i sub-tiles each): with NQ item slots per tile, the stride
+    // over mostly empty slots left some workgroups twice the mean's items.  E = 128,
+    // k = 8, H = 2048, F = 768 (layer): 512 tokens, Zipf routing 370 -> 279 us; 40
+    // tokens 329 -> 187; 1999 tokens, tiles nearly full, 814 -> 750.
+    int c[NQ], nsub = 0;
+#pragma unroll
+    for (int i = 0; i < NQ; i++) {
+        c[i] = ntiles[3 + i];
+        nsub += (NQ - i) * c[i];
+    }
+    const int nitems = nsub * ncb;
     for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
-        const int tix = item / (NQ * ncb), qt = (item / ncb) % NQ, cb = item % ncb;
+        const int cb = item % ncb;
+        int s = item / ncb, tix = 0, qt = 0;
+        bool found = false;
+#pragma unroll
+        for (int i = 0; i < NQ; i++) {
+            if (!found && s < (NQ - i) * c[i]) {
+                tix += s / (NQ - i);
+                qt = s % (NQ - i);
+                found = true;
+            } else if (!found) {
+                tix += c[i];
+                s -= (NQ - i) * c[i];
+            }
+        }
         const PfTile tl = tiles[tix];
-        const int n = min(tl.n - I8_MT * qt, I8_MT);   // pairs of this sub-tile (uniform)
-        if (n <= 0) continue;                         // uniform: no barrier skipped by part of the group
+        const int n = min(tl.n - I8_MT * qt, I8_MT);   // pairs of this sub-tile (uniform, > 0)
         const int *xrows = (MODE == 0 ? ttok : tpair) + tix * PF_MT + I8_MT * qt;
         // activation staging: thread -> (pair slot tid >> 4, level (tid >> 3) & 1, 16 bytes at 16 (tid & 7))
         const int xr = xrows[tid >> 4];
