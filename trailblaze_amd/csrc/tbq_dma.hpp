@@ -7,7 +7,7 @@
 // choose what goes there (the XOR swizzles below are made this way).  The
 // copy is written as asm because the compiler's wait-count pass waits for
 // every outstanding copy before any LDS read it cannot prove unrelated; here
-// the kernels wait themselves (dma_wait), once per step, for copies issued a
+// the kernels wait themselves (dma_wait_barrier), once per step, for copies issued a
 // whole step earlier.  The asm has no register output: nothing lands in a
 // register the compiler could reuse early.
 #pragma once

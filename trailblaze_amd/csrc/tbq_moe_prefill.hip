@@ -648,22 +648,23 @@ __global__ __launch_bounds__(64 * MF_WAVES) __attribute__((amdgpu_waves_per_eu(2
 //
 // Items: (tile, 32-pair sub-tile, row block), on an 8-wave workgroup (32 weight
 // rows per wave, MODE 0 rows i < 16 gate and i >= 16 up of column 16 w + i %
-// 16, activation tile double-buffered in LDS, one barrier per chunk of 128
-// columns); SwiGLU takes a gate row's up partner from lane li + 16.
+// 16); SwiGLU takes a gate row's up partner from lane li + 16.  Packed rows and
+// activations are copied directly to LDS (tbq_dma.hpp), a super-block a step:
+// weights two steps ahead into the wave's own rows of a stage (one ahead where
+// K > 2048 leaves room for two stages only), activations one ahead, one barrier
+// a step.  Lanes that loaded their own rows' bytes touched a cache line per lane
+// and load, five loads per 128 columns.  At 512 Zipf-skewed tokens of E = 128, k
+// = 8, H = 2048, F = 768 the gate/up launch went 168 -> 146 us and the down
+// launch 82 -> 76, at 1999 tokens the layer 750 -> 701.  The rest is the SIMDs'
+// own time: two 8-bit levels times two scale parts make four integer MFMAs per
+// fragment, their operands some 330 vector instructions per super-block, at two
+// waves per SIMD.
 // ---------------------------------------------------------------------------
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int I8_MT = 32;                 // pairs per item
-#ifndef I8_AHEAD
-#define I8_AHEAD 3                        // weight chunks in flight ahead of the one in use (2 or 3)
-#endif
-constexpr int I8_LD = PF_KC + 16;         // LDS row stride in bytes (one activation level)
-// two activation tiles, the pair and row ids, the pairs' block scales (up
-// to 16 super-blocks: K <= 4096), the pairs' 16-element sums of both levels
-// (K / 8 halves per pair)
-constexpr size_t I8_LDS_BYTES = (size_t)2 * I8_MT * 2 * I8_LD + I8_MT * 8 + 16 * I8_MT * 4 + I8_MT * 4096 / 4;
 
 // Position of element e (< 16) of a 16-element group in the stored order.
 __device__ __forceinline__ int q8_pos(int e) {
@@ -736,29 +737,6 @@ __global__ __launch_bounds__(256) void k_rows_q8(const float *__restrict__ in, i
     }
 }
 
-// One lane's Q4_K data for a 128-column chunk c of its row: d/dmin, the
-// chunk's four scale bytes, the four mins of its half of the super-block
-// (for the min MFMA), and 8 quant bytes of each of the chunk's four
-// sub-blocks (elements 16 lh .. 16 lh + 15 of sub-block 4 (c & 1) + ks).
-// A lane's share of chunk c (half c & 1 of a super-block, sub-blocks
-// 4(c & 1) .. +3): half lh of the k range, as two whole sub-blocks, lh and
-// 2 + lh of the chunk (two 16-byte loads; MFMA step ks takes sub-block
-// 2(ks >> 1) + lh, bytes 8(ks & 1) .. +7, and the activations' groups in
-// the same order), d/dmin, the chunk's scale dword and the mins of the
-// lane's half.
-struct Q4I8 {
-    unsigned dd, sw, mw;
-    uint4 q[2];
-};
-
-__device__ __forceinline__ void q4i8_load(const uint8_t *sb, int c, int lh, Q4I8 &r) {
-    r.dd = *reinterpret_cast<const unsigned *>(sb);
-    r.sw = *reinterpret_cast<const unsigned *>(sb + ((c & 1) ? 12 : 4));
-    r.mw = *reinterpret_cast<const unsigned *>(sb + (lh ? 16 : 8));   // mins 4..7 sit in quant bytes 0..3
-    r.q[0] = *reinterpret_cast<const uint4 *>(sb + 16 + 64 * (c & 1) + 16 * lh);
-    r.q[1] = *reinterpret_cast<const uint4 *>(sb + 16 + 64 * (c & 1) + 16 * (2 + lh));
-}
-
 template <int MODE, int NS>
 __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict__ W0, const uint8_t *__restrict__ W1,
                                                        const int8_t *__restrict__ X, const float *__restrict__ XD,
@@ -770,18 +748,19 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict
     constexpr int NSB = K / 256;
     constexpr int NQ = PF_MT / I8_MT;   // sub-tiles per tile, as k_dispatch counts them
     static_assert(I8_MT == 32, "sub-tile classes");
-    // weight chunks loaded ahead: 3 for long rows (two spill at K = 768)
-    constexpr int AH = NS >= 8 ? I8_AHEAD : 2;
-    extern __shared__ __attribute__((aligned(16))) int8_t i8_lds[];   // [2][I8_MT][2][I8_LD]
-    int *po_s = reinterpret_cast<int *>(i8_lds + 2 * I8_MT * 2 * I8_LD);
-    int *px_s = po_s + I8_MT;
-    float *dx_s = reinterpret_cast<float *>(px_s + I8_MT);   // [NSB][I8_MT] block scale of pair slot
-    _Float16 *xb_s = reinterpret_cast<_Float16 *>(dx_s + 16 * I8_MT);   // [I8_MT][K/8] group sums
-    static_assert(NSB <= 16, "dx_s holds 16 super-blocks");
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, lh = lane >> 5;
-    const long long rb = (long long)(K / 256) * 144;
-    const int xbytes = x_rows * 2 * K;
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void *)X, (short)0, xbytes, 0x00020000);
+    constexpr int WS = PF_WAVES * 32 * 144, XS = 2 * I8_MT * 256;   // a stage: 256 packed rows; 32 rows of two levels, two halves
+    constexpr int D = NSB <= 8 ? 3 : 2;   // weight stages that fit beside the group sums
+    __shared__ __attribute__((aligned(16))) unsigned char lds[D * WS + 2 * XS + I8_MT * (K / 4) + I8_MT * 4 * NSB + I8_MT * 8];
+    static_assert(sizeof(lds) <= 160 * 1024, "LDS");
+    unsigned char *const lx_p = lds + D * WS;
+    _Float16 *const xb_s = reinterpret_cast<_Float16 *>(lx_p + 2 * XS);          // [I8_MT][K/8] group sums
+    float *const dx_s = reinterpret_cast<float *>(xb_s + I8_MT * (K / 8));       // [NSB][I8_MT] block scale of pair slot
+    int *const po_s = reinterpret_cast<int *>(dx_s + NSB * I8_MT), *const px_s = po_s + I8_MT;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31, lh = lane >> 5;
+    constexpr int rb = NSB * 144;
+    const dma_rsrc_t xrs = dma_rsrc(X, (uint32_t)(x_rows * 2 * K));
+    const uint32_t aw = lds_addr(lds) + wave * (32 * 144), ax = lds_addr(lx_p) + wave * 1024;
+    unsigned char *const lw_p = lds + wave * (32 * 144) + li * 144;
     // Items are the sub-tiles that exist, tiles in their heaviest-first order (c[i]
     // tiles of NQ - i sub-tiles each): with NQ item slots per tile, the stride
     // over mostly empty slots left some workgroups twice the mean's items.  E = 128,
@@ -812,38 +791,43 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict
         const PfTile tl = tiles[tix];
         const int n = min(tl.n - I8_MT * qt, I8_MT);   // pairs of this sub-tile (uniform, > 0)
         const int *xrows = (MODE == 0 ? ttok : tpair) + tix * PF_MT + I8_MT * qt;
-        // activation staging: thread -> (pair slot tid >> 4, level (tid >> 3) & 1, 16 bytes at 16 (tid & 7))
-        const int xr = xrows[tid >> 4];
-        const int xoff = xr >= 0 ? (xr * 2 + ((tid >> 3) & 1)) * K + 16 * (tid & 7) : xbytes;
+        // activation copies: slot tid >> 4 of a 128-column half, its 16 segments
+        // (two levels of eight) at segment ^ (slot & 15); slots past the tile's
+        // pairs (id -1) copy row 0, whose results are not stored
+        const int xsg = (tid & 15) ^ ((tid >> 4) & 15);
+        const uint32_t xv = (uint32_t)((max(xrows[tid >> 4], 0) * 2 + (xsg >> 3)) * K + 16 * (xsg & 7));
         if (tid < I8_MT) {
             po_s[tid] = tpair[tix * PF_MT + I8_MT * qt + tid];
             px_s[tid] = xrows[tid];
         }
-        const uint8_t *wrow;
+        // weight copies: the wave's 32 rows of 144 bytes as 288 segments of 16
+        const uint8_t *r0, *r1;   // rows 0..15 and 16..31
         if (MODE == 0) {
-            const int col = cb * PF_COLS + 16 * wave + (li & 15);
-            wrow = (li < 16 ? W0 : W1) + ((long long)tl.e * F + col) * rb;
+            const long long ro = ((long long)tl.e * F + cb * PF_COLS + 16 * wave) * rb;
+            r0 = W0 + ro;
+            r1 = W1 + ro;
         } else {
-            wrow = W0 + ((long long)tl.e * H + cb * PF_ROWS + 32 * wave + li) * rb;
+            r0 = W0 + ((long long)tl.e * H + cb * PF_ROWS + 32 * wave) * rb;
+            r1 = r0 + 16 * rb;
         }
-        auto wload = [&](Q4I8 &w, int c) {
-            c = min(c, NS - 1);
-            q4i8_load(wrow + (long long)(c >> 1) * 144, c, lh, w);
+        const uint8_t *wp[5];
+#pragma unroll
+        for (int i = 0; i < 5; i++) {
+            const int g = min(64 * i + lane, 287), row = g / 9;
+            wp[i] = (row < 16 ? r0 : r1) + (row & 15) * rb + 16 * (g % 9);
+        }
+        auto copy_w = [&](int st, int sb) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) dma16_ptr(aw + st * WS + 1024 * i, wp[i] + sb * 144);
+            if (lane < 32) dma16_ptr(aw + st * WS + 4096, wp[4] + sb * 144);
         };
-        u32x4 xv;
-        auto xload = [&](int c) {
-            c = min(c, NS - 1);
-            xv = __builtin_amdgcn_raw_buffer_load_b128(xrs, xoff < xbytes ? xoff + c * PF_KC : xbytes, 0, 0);
+        auto copy_x = [&](int st, int sb) {
+            dma16(ax + st * XS, xv, xrs, sb * 256);
+            dma16(ax + st * XS + XS / 2, xv, xrs, sb * 256 + 128);
         };
-        auto xstore = [&](int buf) {
-            *reinterpret_cast<u32x4 *>(i8_lds + ((buf * I8_MT + (tid >> 4)) * 2 + ((tid >> 3) & 1)) * I8_LD +
-                                       16 * (tid & 7)) = xv;
-        };
-        Q4I8 w0, w1, w2, w3;
-        wload(w0, 0);
-        wload(w1, min(1, NS - 1));
-        if constexpr (AH == 3) wload(w2, min(2, NS - 1));
-        xload(0);
+        copy_w(0, 0);
+        copy_x(0, 0);
+        if (D == 3 && NSB > 1) copy_w(1, 1);
         __syncthreads();   // po_s / px_s written
         // the pair slots' block scales and group sums into LDS (ordered
         // before the first flush by chunk 0's barrier): the flushes then
@@ -862,9 +846,6 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict
                     *reinterpret_cast<u32x4 *>(xb_s + ps * (K / 8) + 8 * sg) = xrw >= 0 ? v : u32x4{0u, 0u, 0u, 0u};
             }
         }
-        xstore(0);
-        xload(1);
-        __syncthreads();
         i32x16 aa1 = {}, ab1 = {}, aa2 = {}, ab2 = {};
         f32x16 y = {};
         // The MFMAs take the activations as the A operand and the weights as
@@ -873,11 +854,11 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict
         // row's d and dmin are the lane's, the pairs' block scales come from
         // LDS.  Super-block flush:
         //   y += dx (d (F1 + F2/256) - dmin (M1 + M2/256))
-        auto flush = [&](const Q4I8 &w, int sb) {
+        auto flush = [&](unsigned dd, unsigned wmw, int sb) {
             f16x8 am;   // this lane's row's mins m_{4 lh + i}, each twice
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const _Float16 m = (_Float16)(float)((w.mw >> (8 * i)) & 63u);
+                const _Float16 m = (_Float16)(float)((wmw >> (8 * i)) & 63u);
                 am[2 * i] = m;
                 am[2 * i + 1] = m;
             }
@@ -886,7 +867,7 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict
             const f16x8 b2 = *reinterpret_cast<const f16x8 *>(bsr + K / 16);
             const f32x16 m1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(b1, am, f32x16{}, 0, 0, 0);
             const f32x16 m2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(b2, am, f32x16{}, 0, 0, 0);
-            const float dw = f16_ref((uint16_t)(w.dd & 0xFFFFu)), mw = f16_ref((uint16_t)(w.dd >> 16));
+            const float dw = f16_ref((uint16_t)(dd & 0xFFFFu)), mw = f16_ref((uint16_t)(dd >> 16));
             const float4 *dxs = reinterpret_cast<const float4 *>(dx_s + sb * I8_MT);
 #pragma unroll
             for (int c = 0; c < 4; c++) {
@@ -905,52 +886,48 @@ __global__ __launch_bounds__(PF_THREADS) void k_moe_i8(const uint8_t *__restrict
             aa2 = i32x16{};
             ab2 = i32x16{};
         };
-        auto chunk = [&](int s, const Q4I8 &wc, Q4I8 &wn) {
-            wload(wn, s + AH);
-            if (s < NS) {
-                const int8_t *xb = i8_lds + ((s & 1) * I8_MT + li) * 2 * I8_LD + 32 * lh;
+        // half c of a super-block, whose packed row and activations are in LDS
+        auto half = [&](const unsigned char *wr, const unsigned char *xb, int c) {
+            const unsigned sw = *reinterpret_cast<const unsigned *>(wr + (c ? 12 : 4));
+            const uint4 wq[2] = {*reinterpret_cast<const uint4 *>(wr + 16 + 64 * c + 16 * lh),
+                                 *reinterpret_cast<const uint4 *>(wr + 16 + 64 * c + 16 * (2 + lh))};
 #pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    const uint4 q4 = wc.q[ks >> 1];
-                    const uint2 q = (ks & 1) ? make_uint2(q4.z, q4.w) : make_uint2(q4.x, q4.y);
-                    const unsigned sc = (wc.sw >> (8 * (2 * (ks >> 1) + lh))) & 63u;   // sub-block 2(ks>>1) + lh
-                    const unsigned short a = (unsigned short)(sc >> 3), b = (unsigned short)(sc & 7u);
-                    const unsigned n0 = q.x & 0x0F0F0F0Fu, n1 = (q.x >> 4) & 0x0F0F0F0Fu;
-                    const unsigned n2 = q.y & 0x0F0F0F0Fu, n3 = (q.y >> 4) & 0x0F0F0F0Fu;
-                    const u16x2 va = {a, a}, vb = {b, b};
-                    auto mul = [](unsigned v, u16x2 f) {
-                        return __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, v) * f);
-                    };
-                    const i32x4 Aa = {(int)mul(n0, va), (int)mul(n1, va), (int)mul(n2, va), (int)mul(n3, va)};
-                    const i32x4 Ab = {(int)mul(n0, vb), (int)mul(n1, vb), (int)mul(n2, vb), (int)mul(n3, vb)};
-                    // 16-element group 4(ks >> 1) + 2 lh + (ks & 1) of the chunk
-                    const int go = 64 * (ks >> 1) + 16 * (ks & 1);
-                    const i32x4 bv1 = *reinterpret_cast<const i32x4 *>(xb + go);
-                    const i32x4 bv2 = *reinterpret_cast<const i32x4 *>(xb + I8_LD + go);
-                    aa1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv1, Aa, aa1, 0, 0, 0);
-                    ab1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv1, Ab, ab1, 0, 0, 0);
-                    aa2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv2, Aa, aa2, 0, 0, 0);
-                    ab2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv2, Ab, ab2, 0, 0, 0);
-                }
-                if (s & 1) flush(wc, s >> 1);
-                if (s + 1 < NS) xstore((s + 1) & 1);
+            for (int ks = 0; ks < 4; ks++) {
+                const uint4 q4 = wq[ks >> 1];
+                const uint2 q = (ks & 1) ? make_uint2(q4.z, q4.w) : make_uint2(q4.x, q4.y);
+                const unsigned sc = (sw >> (8 * (2 * (ks >> 1) + lh))) & 63u;   // sub-block 2(ks>>1) + lh
+                const unsigned short a = (unsigned short)(sc >> 3), b = (unsigned short)(sc & 7u);
+                const unsigned n0 = q.x & 0x0F0F0F0Fu, n1 = (q.x >> 4) & 0x0F0F0F0Fu;
+                const unsigned n2 = q.y & 0x0F0F0F0Fu, n3 = (q.y >> 4) & 0x0F0F0F0Fu;
+                const u16x2 va = {a, a}, vb = {b, b};
+                auto mul = [](unsigned v, u16x2 f) {
+                    return __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, v) * f);
+                };
+                const i32x4 Aa = {(int)mul(n0, va), (int)mul(n1, va), (int)mul(n2, va), (int)mul(n3, va)};
+                const i32x4 Ab = {(int)mul(n0, vb), (int)mul(n1, vb), (int)mul(n2, vb), (int)mul(n3, vb)};
+                // 16-element group 4(ks >> 1) + 2 lh + (ks & 1) of the chunk
+                const int sg = (4 * (ks >> 1) + (ks & 1) + 2 * lh) ^ (li & 15);
+                const i32x4 bv1 = *reinterpret_cast<const i32x4 *>(xb + 16 * sg);
+                const i32x4 bv2 = *reinterpret_cast<const i32x4 *>(xb + 16 * (sg ^ 8));
+                aa1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv1, Aa, aa1, 0, 0, 0);
+                ab1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv1, Ab, ab1, 0, 0, 0);
+                aa2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv2, Aa, aa2, 0, 0, 0);
+                ab2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bv2, Ab, ab2, 0, 0, 0);
             }
-            xload(s + 2);
-            if (s < NS) __syncthreads();
         };
-        if constexpr (AH == 3) {
-            for (int s = 0; s < NS; s += 4) {
-                chunk(s, w0, w3);
-                chunk(s + 1, w1, w0);
-                chunk(s + 2, w2, w1);
-                chunk(s + 3, w3, w2);
-            }
-        } else {
-            for (int s = 0; s < NS; s += 3) {
-                chunk(s, w0, w2);
-                chunk(s + 1, w1, w0);
-                chunk(s + 2, w2, w1);
-            }
+        for (int sb = 0; sb < NSB; sb++) {
+            // this super-block's copies have landed; with three weight stages the
+            // next one's weights, issued last, stay in flight
+            if (D == 3 && sb + 1 < NSB) dma_wait_barrier_n<5>();
+            else dma_wait_barrier();
+            if (sb + 1 < NSB) copy_x((sb + 1) & 1, sb + 1);
+            if (sb + D - 1 < NSB) copy_w((sb + D - 1) % D, sb + D - 1);
+            const unsigned char *wr = lw_p + sb % D * WS, *xb = lx_p + (sb & 1) * XS + li * 256;
+            const unsigned dd = *reinterpret_cast<const unsigned *>(wr);
+            const unsigned mw = *reinterpret_cast<const unsigned *>(wr + (lh ? 16 : 8));   // mins 4..7 sit in quant bytes 0..3
+            half(wr, xb, 0);
+            half(wr, xb + XS / 2, 1);
+            flush(dd, mw, sb);
         }
         // accumulator register r of lane l: pair slot 8(r/4) + 4 lh + r%4 of
         // the sub-tile, the wave's weight row li
@@ -985,7 +962,7 @@ static hipError_t launch_moe_i8(int ns, unsigned nwg, hipStream_t st, const uint
                                 float *out) {
 #define TBQ_NS(N)                                                                                                   \
     case N:                                                                                                         \
-        hipLaunchKernelGGL((k_moe_i8<MODE, N>), dim3(nwg), dim3(PF_THREADS), I8_LDS_BYTES, st, W0, W1, X, XD, XB,   \
+        hipLaunchKernelGGL((k_moe_i8<MODE, N>), dim3(nwg), dim3(PF_THREADS), 0, st, W0, W1, X, XD, XB,   \
                            x_rows, tpair, ttok, tiles, ntiles, ncb, H, F, out);                                     \
         break;
     switch (ns) {
