@@ -5,7 +5,7 @@
 //
 // Per layer (x: fp32 residual rows [T][H]; h16: fp16 rows with per-row
 // power-of-two scales, the GEMMs' activation operand; the GEMMs are
-// k_hgemm_* (tbq_gemm.hip): Q4_K weights are dequantised inside it, any other
+// k_hgemm_* (tbq_gemm.hip): Q4_K weights are dequantised inside them, any other
 // format to fp16 first (k_dequant_f16, one reused buffer)):
 //   k_pf_norm        x += y (the previous sublayer's output, unscaled by
 //                    its row scales), h16 = rmsnorm(x) * attn_norm
@@ -675,7 +675,7 @@ static size_t pf_up(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Every model with hidden <= 8192, n_heads * head_dim <= 8192 and ffn <=
 // 16384 (the rows the norm, attention-row and SwiGLU kernels hold) takes the batched path for T >= 2.  Q4_K matrices go
-// straight into the GEMM (dequantised on the way into LDS); every other
+// straight into the GEMM (dequantised in its registers); every other
 // format and layout is dequantised to fp16 first (one matrix at a time) and
 // multiplied by the same GEMM.
 bool dense_prefill_batched(const tbq_dense_model *m) {
