@@ -60,7 +60,11 @@ __device__ __forceinline__ void dma_wait_barrier() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// The same with the N memory operations issued last left in flight (they
+// Every LDS read this wave has issued has returned: what it read may be
+// overwritten by copies of its own (rows that no other wave reads).
+__device__ __forceinline__ void lds_read_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// dma_wait_barrier with the N memory operations issued last left in flight (they
 // complete in issue order, so all copies before them have landed).
 template <int N>
 __device__ __forceinline__ void dma_wait_barrier_n() {

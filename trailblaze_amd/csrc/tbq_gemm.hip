@@ -259,6 +259,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     scales(0);
 #pragma unroll
     for (int b = 0; b < 2; b++) a[0][b] = frag(b, 0);
+    lds_read_wait();   // step 0's copies go to other slots, but every copy follows the reads before it
     for (int sb = 0; sb < nsb; sb++) {
         const int nx = min(sb + 1, nsb - 1);
 #pragma unroll

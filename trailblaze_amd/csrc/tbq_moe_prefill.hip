@@ -480,6 +480,9 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
     scales(0);
 #pragma unroll
     for (int b = 0; b < NA; b++) a[0][b] = frag(b, 0);
+    // step 0 copies into quant slot 0, and at D = 4 into the only header slot:
+    // rows this wave alone reads, whose first reads the step's copies must not pass
+    lds_read_wait();
     int xs = 0, qs = 0;   // slots of this step's activations and quants
     const unsigned char *const xb0 = lx_p + li * 128;
     const int xsw = mf_swz8(li);
