@@ -523,3 +523,27 @@ def test_moe_prefill_int8_mixed_tiles(oracle, T, H, F, E, k, spread):
         tb.moe_forward(L, T, dev(xn), dev(resid), out, idx, w, workspace=ws, mode=tb.TBQ_MOE_I8)
     assert np.array_equal(host(idx).reshape(T, 8)[:, :k], ridx[:, :k])
     assert rel_l2(host(out).reshape(T, H) - resid, ref - resid) <= PREFILL_TOL
+
+
+# Scale fields at and below fp16's smallest normal number.  The reference's
+# layout reads a subnormal half as m * 2^-136 (zero beside anything else),
+# ggml's as IEEE does; here they carry about half of the weights' size, so a
+# decoder of the other kind is off by tens of percent.
+@pytest.mark.parametrize("qt,mode", [(fm.Q4_K, tb.TBQ_MOE_BF16), (fm.GGML | fm.Q4_K, tb.TBQ_MOE_BF16),
+                                     (fm.Q4_K, tb.TBQ_MOE_I8)])
+@pytest.mark.parametrize("T", [40, 150])   # one row block per wave at both; one and two 32-pair sub-tiles
+def test_moe_prefill_subnormal_scales(oracle, qt, mode, T):
+    H, F, E, k = 512, 256, 4, 2
+    router, gate, up, down = synth.moe_layer(H, F, E, qt, seed=77)
+    rng = np.random.default_rng(T)
+    for W in (gate, up, down):
+        b = W.reshape(-1, 144)
+        for off in (0, 2):
+            h = np.where(rng.random(len(b)) < 0.5, rng.integers(0x0200, 0x0400, len(b)), rng.integers(0x0400, 0x0600, len(b)))
+            b[:, off:off + 2] = h.astype(np.uint16).view(np.uint8).reshape(-1, 2)
+    xn, resid = synth.activations((T, H), rng) * np.float32(32), np.zeros((T, H), np.float32)
+    print("moe prefill subnormal scales", qt, mode, T, flush=True)
+    out, idx, _ = gpu_moe(xn, resid, router, gate, up, down, F, k, qt, mode=mode)
+    ref, ridx, _ = oracle.moe(xn, resid, router, gate, up, down, F=F, top_k=k, qtype=qt)
+    assert np.array_equal(idx, ridx)
+    assert rel_l2(out, ref) <= 1e-2

@@ -273,6 +273,13 @@ __device__ __forceinline__ float h2f(unsigned bits) {
     return (float)__builtin_bit_cast(_Float16, (unsigned short)(bits & 0xFFFFu));
 }
 
+// Both halves with subnormals made zero: the reference's layout reads one as
+// m * 2^-136 (f16_ref), which no sum here can hold, ggml's as IEEE does.
+__device__ __forceinline__ unsigned f16x2_no_subnormal(unsigned h) {
+    const unsigned lo = (h & 0x7C00u) ? h & 0xFFFFu : 0u;
+    return (h & 0x7C000000u) ? lo | (h & 0xFFFF0000u) : lo;
+}
+
 // ---------------------------------------------------------------------------
 // Expert tile GEMM.  Work items are (tile, row block) pairs, tile-major (ncb =
 // F / (64 NA) row blocks of columns for MODE 0, H / (128 NA) of rows for MODE 1),
@@ -395,8 +402,11 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
             const unsigned char *qrow = lq_p + slot * QS + (wrow + 32 * b) * 32;
             if (s == 0) {
                 hd[b] = *reinterpret_cast<const u32x4 *>(lh_p + sb % HD * (MF_ROWS * 16) + (wave * 64 + 32 * b + li) * 16);
-                // the reference's mins of sub-blocks 4..7 are quant bytes 0..3 (layer4/tb_gguf.c:163-168)
-                if constexpr (!GG) mhi[b] = *reinterpret_cast<const uint32_t *>(qrow + 16 * qsw);
+                if constexpr (!GG) {
+                    // the reference's mins of sub-blocks 4..7 are quant bytes 0..3 (layer4/tb_gguf.c:163-168)
+                    mhi[b] = *reinterpret_cast<const uint32_t *>(qrow + 16 * qsw);
+                    hd[b].x = f16x2_no_subnormal(hd[b].x);
+                }
             }
             if constexpr (GG) {
                 q[b][0] = *reinterpret_cast<const u32x4 *>(qrow + 16 * qsw);
