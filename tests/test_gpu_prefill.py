@@ -145,6 +145,66 @@ def test_prefill_attention_edges(oracle, D, G, P, T):
         assert np.array_equal(got[:, :, :P], cache[:, :, :P].astype(np.float32)) and not np.any(got[:, :, P + T:])
 
 
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_prefill_attention_heaviest_weight_is_exact(oracle, seed):
+    """The softmax's running max is the exact one, so a position that holds
+    most of a query's weight has probability 1 and no fp16 rounding.  Position
+    90 scores 5 above position 20, the highest of the first chunk (N(0,1)
+    scores otherwise): 0.993 of the weight.  The relative error of that weight
+    is read per head off the next layer's V row: the row's error projected on
+    its derivatives by the heads' cached V vectors (fp16 weights and no FFN
+    output, so little else rounds).  A running max that may stay behind by up
+    to 2^8 leaves the position some probability in [1, 256), whose fp16
+    rounding has an RMS of 2.1e-4; the roundings of the other operands (each
+    2^-11 / sqrt(12) an element, projected on 128 dimensions a head) leave 7e-5
+    to 1e-4."""
+    import torch
+    from oracle.dense import DenseOracle, rmsnorm, rope
+    from trailblaze_amd.dense import SyntheticDense
+    NH, D, P, A, B = 8, 128, 100, 20, 90
+    cfg = _cfg(hidden=1024, n_heads=NH, n_kv_heads=NH, head_dim=D, max_ctx=128, vocab=256, qtype_layers=fm.F16,
+               qtype_embd=fm.F16)
+    m = SyntheticDense(cfg, seed, keep_host=True)
+    for name, by in (("wdown", 0), ("wo", 2.0 ** -9)):   # the attention's output as large as the embedding beside it
+        for w in (m._keep[0][name].view(torch.float16), m.host["layers"][0][name].view(np.float16)):
+            w *= by
+    ref = DenseOracle(oracle, cfg, m.host)
+    rng = np.random.default_rng(seed)
+    toks = rng.integers(0, 256, 2)
+    L = ref.layers[0]
+    q = (L["wqkv"][:NH * D] @ rmsnorm(ref.lm[toks[1]], L["attn_norm"], cfg.norm_eps)).reshape(NH, D)
+    q = np.stack([rope(rmsnorm(v, L["q_norm"], cfg.norm_eps), P + 1, cfg.rope_theta) for v in q])
+    for cache, dev in ((ref.kc, m.k_cache), (ref.vc, m.v_cache)):
+        cache[:, :, :P] = rng.standard_normal(cache[:, :, :P].shape)
+        if cache is ref.kc:
+            for at, score in ((A, 12), (B, 17)):
+                cache[0, :, at] = q * (score * np.sqrt(D) / np.sum(q * q, axis=1))[:, None]
+        else:
+            cache[0, :, B] *= 16
+        cache[:] = cache.astype(np.float32)
+        dev.copy_(torch.from_numpy(cache.astype(np.float32)))
+    logits = torch.empty(cfg.vocab, dtype=torch.float32, device="cuda")
+    print("prefill heaviest weight", seed, flush=True)
+    m.prefill(toks, P, logits)
+    ref.decode(toks[0], P)
+
+    def v_row(h=None, by=0.0):
+        if h is not None:
+            ref.vc[0, h, B] *= 1 + by
+        ref.decode(toks[1], P + 1)
+        if h is not None:
+            ref.vc[0, h, B] /= 1 + by
+        return ref.vc[1, :, P + 1].flatten().copy()
+
+    want = v_row()
+    by = 1e-4
+    U = np.stack([(v_row(h, by) - want) / by for h in range(NH)], 1)
+    e = host(m.v_cache).reshape(ref.vc.shape)[1, :, P + 1].flatten() - want
+    c = np.linalg.lstsq(U, e, rcond=None)[0]
+    print(c, flush=True)
+    assert np.sqrt(np.mean(c * c)) <= 1.4e-4
+
+
 @pytest.mark.parametrize("ql,qe", [(fm.Q8_0, fm.Q6_K), (fm.Q5_K, fm.Q8_0), (fm.GGML | fm.Q4_K, fm.GGML | fm.Q6_K),
                                    (fm.GGML | fm.Q3_K, fm.Q4_K)])
 def test_prefill_other_formats(oracle, ql, qe):
