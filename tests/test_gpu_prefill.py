@@ -145,6 +145,36 @@ def test_prefill_attention_edges(oracle, D, G, P, T):
         assert np.array_equal(got[:, :, :P], cache[:, :, :P].astype(np.float32)) and not np.any(got[:, :, P + T:])
 
 
+@pytest.mark.parametrize("D,G,P", [(64, 4, 0), (128, 4, 10), (128, 8, 0), (64, 2, 5)])
+def test_prefill_nan_token_stays_in_its_block(D, G, P):
+    """A token whose embedding holds a NaN leaves the tokens of earlier query
+    blocks (128 / G tokens each) as they are, bit for bit, though it shares a
+    chunk of 64 positions with them."""
+    import torch
+    from trailblaze_amd.dense import SyntheticDense
+    QB = 128 // G
+    bad, T = QB + 3, QB + 20
+    cfg = _cfg(n_heads=8, n_kv_heads=8 // G, head_dim=D, vocab=256, qtype_embd=fm.F32)
+    rng = np.random.default_rng(D + G)
+    toks = rng.integers(0, 255, P + T)
+    logits = torch.empty(cfg.vocab, dtype=torch.float32, device="cuda")
+    rows = []
+    for nan in (False, True):
+        m = SyntheticDense(cfg, 60)
+        if nan:
+            m.lm_head.view(torch.float32).view(256, -1)[255, 7] = float("nan")
+        t = toks.copy()
+        t[P + bad] = 255
+        for pos in range(P):
+            m.decode(int(t[pos]), pos, logits)
+        print("prefill nan token", D, G, P, nan, flush=True)
+        m.prefill(t[P:], P, logits)
+        rows.append([host(c).reshape(2, 8 // G, cfg.max_ctx, D)[:, :, :P + T] for c in (m.k_cache, m.v_cache)])
+    for a, b in zip(*rows):
+        assert np.all(np.isnan(b[0, :, P + bad])) and np.all(np.isfinite(a))
+        assert bits_equal(a[:, :, :P + QB], b[:, :, :P + QB])
+
+
 @pytest.mark.parametrize("seed", [1, 2, 3])
 def test_prefill_attention_heaviest_weight_is_exact(oracle, seed):
     """The softmax's running max is the exact one, so a position that holds

@@ -475,6 +475,21 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(2, 2)))
     int buf = 0;
     for (int c0 = k0; c0 < kend; c0 += PM_KC, buf ^= 1) {
         copy(buf ^ 1, c0 + PM_KC < kend ? c0 + PM_KC : c0);   // the last chunk copies itself again, never read
+        // V past the block's last query is made zero (past the prompt it is
+        // already): its p is 0, and 0 times an infinity or NaN of a later token is not
+        if (c0 + PM_KC > kend && kend < pos0 + T) {   // uniform
+#pragma unroll
+            for (int i = 0; i < D * 8 / (64 * WV); i++) {
+                const int f = threadIdx.x + 64 * WV * i, row = f >> 3, seg = f & 7;
+                pm_h8 *p = reinterpret_cast<pm_h8 *>(st->v[buf] + row * (PM_KC * 2) + 16 * (seg ^ pf_swz8(row)));
+                pm_h8 v = *p;
+#pragma unroll
+                for (int e = 0; e < 8; e++)   // k_pf_kv16's order of the positions
+                    v[e] = c0 + 16 * (seg / 2) + 4 * (seg % 2) + 8 * (e / 4) + e % 4 < kend ? v[e] : (_Float16)0.f;
+                *p = v;
+            }
+            __syncthreads();
+        }
         if (c0 <= qhi) {   // uniform per wave
             const unsigned char *Kb = st->k[buf] + li * (D * 2), *Vb = st->v[buf] + li * (PM_KC * 2);
             pm_f16 sc[2] = {pm_f16{}, pm_f16{}};
