@@ -234,10 +234,9 @@ int tbq_dense_decode(const tbq_dense_model *m, int token, int pos, float *logits
  * decode); otherwise, and for T = 1, the decode step runs once per token
  * (identical to T tbq_dense_decode calls).  tokens_host is read by an
  * asynchronous copy on `stream`: keep it valid until the stream has run
- * the call.  1 <= T <= 65536, pos0 + T <= max_ctx.  The workspace size is
- * for exactly T tokens: a shorter prompt whose products split K can need
- * more than a longer one, so a buffer kept for several lengths is sized by
- * asking for each. */
+ * the call.  1 <= T <= 65536, pos0 + T <= max_ctx.  The workspace size
+ * never falls as T grows: a buffer for T tokens serves every shorter prompt
+ * of the model. */
 size_t tbq_dense_prefill_workspace_size(const tbq_dense_model *m, int T);
 int tbq_dense_prefill(const tbq_dense_model *m, const int *tokens_host, int T, int pos0, float *logits,
                       void *workspace, size_t ws_bytes, void *stream);

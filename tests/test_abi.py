@@ -89,3 +89,25 @@ def test_dense_prefill_workspace_host_side():
     dw = lib.tbq_dense_workspace_size(C.byref(wide))
     assert dw < lib.tbq_dense_prefill_workspace_size(C.byref(wide), 512) <= dw + 512 * 4 + 256
     assert lib.tbq_dense_prefill_workspace_size(C.byref(small), 0) == 0
+
+
+@pytest.mark.parametrize("hidden,heads,kv,dim,ffn,max_ctx,fused", [
+    (1024, 16, 8, 64, 3072, 4096, True), (2048, 16, 8, 128, 6144, 300, False), (2560, 32, 8, 128, 9728, 4096, True),
+    (4096, 32, 4, 128, 12288, 4096, True), (4096, 32, 4, 128, 12288, 40960, False), (256, 2, 2, 128, 256, 128, False),
+    (8448, 8, 2, 128, 9728, 4096, True)])
+def test_dense_prefill_workspace_grows_with_the_prompt(hidden, heads, kv, dim, ffn, max_ctx, fused):
+    """A buffer for T tokens serves every shorter prompt: the size never falls
+    as T grows."""
+    from trailblaze_amd.dense import DenseLayer, DenseModel
+    from trailblaze_amd import formats as fm
+    fake = 1 << 20
+    layers = (DenseLayer * 1)()
+    for name in ("attn_norm", "q_norm", "k_norm", "ffn_norm", "wo", "wdown") + (
+            ("wqkv", "wgu") if fused else ("wq", "wk", "wv", "wgate", "wup")):
+        setattr(layers[0], name, fake)
+    m = DenseModel(1, hidden, heads, kv, dim, ffn, 1024, max_ctx, 1e-6, 1e6, fm.Q4_K, fm.Q6_K, fake, fake, fake, layers,
+                   fake, fake)
+    size = [tb.lib().tbq_dense_prefill_workspace_size(C.byref(m), T) for T in range(1, 1400)]
+    assert size[0] > 0
+    falls = [T for T in range(2, len(size) + 1) if size[T - 1] < size[T - 2]]
+    assert falls == []

@@ -280,6 +280,32 @@ def test_prefill_separate_matrices(oracle):
             assert rel_l2(host(logits), want) <= PREFILL_TOL
 
 
+@pytest.mark.parametrize("short_by", [0, 1, 1 << 20])
+def test_prefill_workspace_of_a_longer_prompt(short_by):
+    """A buffer for 512 tokens serves 480 of them bit for bit as their own
+    does; one with less room for split-K partial sums takes fewer slices."""
+    import ctypes as C
+    import torch
+    from trailblaze_amd.dense import SyntheticDense
+    m = SyntheticDense(_cfg(n_layers=1, hidden=1024, n_heads=8, n_kv_heads=4, head_dim=128, ffn=2048), 71)
+    lib, T = tb.lib(), 480
+    toks = np.random.default_rng(4).integers(0, 512, T).astype(np.int32)
+    logits = torch.empty((2, 512), dtype=torch.float32, device="cuda")
+    own = int(lib.tbq_dense_prefill_workspace_size(C.byref(m.model), T))
+    for i, n in enumerate((own, own - short_by if short_by else
+                           int(lib.tbq_dense_prefill_workspace_size(C.byref(m.model), 512)))):
+        print("prefill workspace", short_by, n, flush=True)
+        ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+        assert lib.tbq_dense_prefill(C.byref(m.model), toks.ctypes.data, T, 0, logits[i].data_ptr(), ws.data_ptr(), n,
+                                     C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+    a, b = host(logits).reshape(2, 512)
+    if short_by:
+        assert rel_l2(b, a) <= 2e-3   # the same fp16 operands, other fp32 sums rounded to fp16 again
+    else:
+        assert bits_equal(a, b)
+
+
 def test_prefill_one_token_is_the_decode_step():
     """T = 1 runs the decode step itself: the same logits and cache bits."""
     import torch

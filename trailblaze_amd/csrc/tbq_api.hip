@@ -455,8 +455,9 @@ int tbq_dense_prefill(const tbq_dense_model *m, const int *tokens_host, int T, i
     for (int t = 0; t < T; t++)
         if (tokens_host[t] < 0 || tokens_host[t] >= m->vocab)
             return fail("tbq_dense_prefill: token %d at %d out of range", tokens_host[t], t);
-    if (ws_bytes < dense_prefill_workspace_bytes(m, T)) return fail("tbq_dense_prefill: workspace too small");
-    return hip_ok(launch_dense_prefill(m, tokens_host, T, pos0, logits, workspace, S(s)), "dense prefill launch");
+    if (ws_bytes < dense_prefill_workspace_min(m, T)) return fail("tbq_dense_prefill: workspace too small");
+    return hip_ok(launch_dense_prefill(m, tokens_host, T, pos0, logits, workspace, ws_bytes, S(s)),
+                  "dense prefill launch");
 }
 
 int tbq_quantize_q8k(const float *x, long long n, void *blocks, void *s) {
@@ -485,7 +486,8 @@ int tbq_gemm(int wqt, const void *W, const void *X16, int T, int N, int K, float
         return fail("tbq_gemm: null or misaligned pointer");
     const size_t need = tbq_gemm_workspace_size(T, N, K);
     if (need && (!ws || ws_bytes < need)) return fail("tbq_gemm: workspace %zu < %zu bytes", ws_bytes, need);
-    return hip_ok(launch_hgemm(wqt, W, (const _Float16 *)X16, T, N, K, C, ldc, (float *)ws, hgemm_cus(), S(s)),
+    return hip_ok(launch_hgemm(wqt, W, (const _Float16 *)X16, T, N, K, C, ldc, (float *)ws, ws_bytes, hgemm_cus(),
+                               S(s)),
                   "gemm launch");
 }
 

@@ -703,12 +703,14 @@ bool dense_prefill_batched(const tbq_dense_model *m) {
 struct PfWs {
     float *x, *y, *qkv, *att, *gu, *sa, *sb, *part, *rope, *gpart;
     _Float16 *h16, *wh, *qb, *k16, *vt;
+    size_t gpart_bytes;
     int cp;   // positions per head of k16 and vt
     int *tok;
     void *dec;
 };
 
-static PfWs pf_ws(const tbq_dense_model *m, int T, void *ws, size_t *total) {
+// *total: the bytes used, without gpart's, which is what the caller's ws_bytes leave.
+static PfWs pf_ws(const tbq_dense_model *m, int T, void *ws, size_t ws_bytes, size_t *total) {
     const size_t H = m->hidden, QD = (size_t)m->n_heads * m->head_dim, F = m->ffn;
     const size_t QKVR = (size_t)(m->n_heads + 2 * m->n_kv_heads) * m->head_dim;
     const size_t wide = std::max(std::max(H, QD), F);
@@ -738,29 +740,43 @@ static PfWs pf_ws(const tbq_dense_model *m, int T, void *ws, size_t *total) {
         w.sa = (float *)take((size_t)T * 4);
         w.sb = (float *)take((size_t)T * 4);
         w.wh = (_Float16 *)take(wmax * 2);
-        // split-K partials of the largest product that splits
-        const int cu = hgemm_cus(), Ti = T;
-        const size_t gp = std::max(
-            std::max(std::max(hgemm_partial_bytes(Ti, (int)QKVR, (int)H, cu), hgemm_partial_bytes(Ti, (int)QD, (int)H, cu)),
-                     std::max(hgemm_partial_bytes(Ti, m->n_kv_heads * m->head_dim, (int)H, cu),
-                              hgemm_partial_bytes(Ti, (int)H, (int)QD, cu))),
-            std::max(std::max(hgemm_partial_bytes(Ti, (int)(2 * F), (int)H, cu), hgemm_partial_bytes(Ti, (int)F, (int)H, cu)),
-                     hgemm_partial_bytes(Ti, (int)H, (int)F, cu)));
-        w.gpart = gp ? (float *)take(gp) : nullptr;
         w.rope = (float *)take((size_t)T * m->head_dim * 4);
         // attention split partials: a prefill reaching position kmax - 1 uses
         // at most min(PA_MAX_SPLIT, ceil(kmax / PA_MIN_KS)) splits, and kmax <= max_ctx
         const int ns = std::min(PA_MAX_SPLIT, (m->max_ctx + PA_MIN_KS - 1) / PA_MIN_KS);
         w.part = ns > 1 ? (float *)take((size_t)T * m->n_heads * ns * pf_rec(m->head_dim) * 4) : nullptr;
+        // a product's split-K partials until their consumer has added them.  (A
+        // region of their own: with the attention's records in the same memory a
+        // prefill of 200 tokens took 250 us instead of 241)
+        w.gpart_bytes = ws_bytes > off ? ws_bytes - off : 0;
+        w.gpart = w.gpart_bytes ? (float *)(p + off) : nullptr;
     }
     if (total) *total = off;
     return w;
 }
 
-size_t dense_prefill_workspace_bytes(const tbq_dense_model *m, int T) {
+size_t dense_prefill_workspace_min(const tbq_dense_model *m, int T) {
     size_t t = 0;
-    pf_ws(m, T, nullptr, &t);
+    pf_ws(m, T, nullptr, 0, &t);
     return t;
+}
+
+// With room for the partial sums of the products that split K (a gate|up
+// matrix's does not) at any T up to this one: never less for a larger T.
+size_t dense_prefill_workspace_bytes(const tbq_dense_model *m, int T) {
+    const size_t base = dense_prefill_workspace_min(m, T);
+    if (!dense_prefill_batched(m) || T < 2) return base;
+    const int H = m->hidden, QD = m->n_heads * m->head_dim, KD = m->n_kv_heads * m->head_dim, F = m->ffn, cu = hgemm_cus();
+    bool qkv = false, q_k_v = false, gate_up = false;
+    for (int l = 0; l < m->n_layers; l++) {
+        (m->layers[l].wqkv ? qkv : q_k_v) = true;
+        gate_up = gate_up || !m->layers[l].wgu;
+    }
+    size_t gp = std::max(hgemm_partial_upto(T, H, QD, cu), hgemm_partial_upto(T, H, F, cu));
+    if (qkv) gp = std::max(gp, hgemm_partial_upto(T, QD + 2 * KD, H, cu));
+    if (q_k_v) gp = std::max(gp, std::max(hgemm_partial_upto(T, QD, H, cu), hgemm_partial_upto(T, KD, H, cu)));
+    if (gate_up) gp = std::max(gp, hgemm_partial_upto(T, F, H, cu));
+    return base + gp;
 }
 
 // tokens: T device ints (in range); T >= 2.
@@ -775,10 +791,10 @@ static hipError_t pf_batched(const tbq_dense_model *m, const PfWs &w, int T, int
     // (with ns set, the K slices' partial sums stay in w.gpart for the
     // consumer to add: k_pf_qk, k_pf_norm and k_pf_scale_row take them)
     auto gemm = [&](int qt, const void *W, int rows, int K, float *C, int ldc, int *ns = nullptr) {
-        if (qt == QT_Q4_K) return launch_hgemm(QT_Q4_K, W, w.h16, T, rows, K, C, ldc, w.gpart, cu, st, ns);
+        if (qt == QT_Q4_K) return launch_hgemm(QT_Q4_K, W, w.h16, T, rows, K, C, ldc, w.gpart, w.gpart_bytes, cu, st, ns);
         const hipError_t e = launch_dequant_f16(qt, W, (long long)rows * K, w.wh, st);
         if (e != hipSuccess) return e;
-        return launch_hgemm(QT_F16, w.wh, w.h16, T, rows, K, C, ldc, w.gpart, cu, st, ns);
+        return launch_hgemm(QT_F16, w.wh, w.h16, T, rows, K, C, ldc, w.gpart, w.gpart_bytes, cu, st, ns);
     };
     const float *ysrc = w.y;   // the previous sublayer's output, as yns slices
     int yns = 1;
@@ -855,8 +871,8 @@ static hipError_t pf_batched(const tbq_dense_model *m, const PfWs &w, int T, int
 }
 
 hipError_t launch_dense_prefill(const tbq_dense_model *m, const int *tokens_host, int T, int pos0, float *logits,
-                                void *ws, hipStream_t st) {
-    const PfWs w = pf_ws(m, T, ws, nullptr);
+                                void *ws, size_t ws_bytes, hipStream_t st) {
+    const PfWs w = pf_ws(m, T, ws, ws_bytes, nullptr);
     if (!dense_prefill_batched(m) || T < 2) {
         // one token, or a row wider than the norm kernel: the decode step per token
         for (int t = 0; t < T; t++) {

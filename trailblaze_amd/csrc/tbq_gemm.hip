@@ -444,8 +444,9 @@ struct HgPlan {
     int tile, S, per;   // index into the table, slices, super-blocks per slice
 };
 
+// max_slices and part_bytes (room for the partial sums) limit the slices.
 template <int NT>
-HgPlan hg_plan(const HgTile (&tab)[NT], int T, int N, int K, int n_cu, int max_slices) {
+HgPlan hg_plan(const HgTile (&tab)[NT], int T, int N, int K, int n_cu, int max_slices, size_t part_bytes) {
     HgPlan best{0, 1, K / 256};
     float bt = 1e30f;
     for (int i = 0; i < NT; i++) {
@@ -453,6 +454,7 @@ HgPlan hg_plan(const HgTile (&tab)[NT], int T, int N, int K, int n_cu, int max_s
         for (int s = 1; s <= std::min(max_slices, K / 256); s++) {
             const int per = (K / 256 + s - 1) / s, S = (K / 256 + per - 1) / per;
             if (S != s) continue;
+            if (s > 1 && (size_t)s * T * N * 4 > part_bytes) break;
             const long long W = tiles * S, n = (W + n_cu - 1) / n_cu;
             const float steps = 4.f * per, mb = (float)T * N * 4e-6f;
             const float step = n == 1 ? tab[i].ke + (tab[i].k1 - tab[i].ke) * W / n_cu : n * tab[i].k2 * 0.5f;
@@ -514,17 +516,35 @@ hipError_t go(int wqt, const void *W, const _Float16 *X, int T, int N, int K, co
     }
 }
 
-HgPlan hg_plan_for(int wqt, int T, int N, int K, int n_cu, int max_slices) {
-    return wqt == QT_F16 ? hg_plan(HG_F16, T, N, K, n_cu, max_slices) : hg_plan(HG_Q4K, T, N, K, n_cu, max_slices);
+HgPlan hg_plan_for(int wqt, int T, int N, int K, int n_cu, int max_slices, size_t part_bytes) {
+    return wqt == QT_F16 ? hg_plan(HG_F16, T, N, K, n_cu, max_slices, part_bytes)
+                         : hg_plan(HG_Q4K, T, N, K, n_cu, max_slices, part_bytes);
+}
+
+// Slices that either weight format's plan would take, given room.
+int hg_slices(int T, int N, int K, int n_cu) {
+    return std::max(hg_plan_for(QT_F16, T, N, K, n_cu, HG_MAX_SLICES, SIZE_MAX).S,
+                    hg_plan_for(QT_Q4_K, T, N, K, n_cu, HG_MAX_SLICES, SIZE_MAX).S);
 }
 
 }  // namespace
 
 // Partial sums of a T x N product over K, whichever weight format runs it.
 size_t hgemm_partial_bytes(int T, int N, int K, int n_cu) {
-    const int s = std::max(hg_plan_for(QT_F16, T, N, K, n_cu, HG_MAX_SLICES).S,
-                           hg_plan_for(QT_Q4_K, T, N, K, n_cu, HG_MAX_SLICES).S);
+    const int s = hg_slices(T, N, K, n_cu);
     return s > 1 ? (size_t)s * T * N * 4 : 0;
+}
+
+// The most that any product of 1 .. T rows wants.  Within 32 rows the tile
+// counts stay and only the price of the partial sums grows, so the slices are
+// at most those of the first row.
+size_t hgemm_partial_upto(int T, int N, int K, int n_cu) {
+    size_t most = 0;
+    for (int t = 1; t <= T; t += 32) {
+        const int s = hg_slices(t, N, K, n_cu);
+        if (s > 1) most = std::max(most, (size_t)s * std::min(t + 31, T) * N * 4);
+    }
+    return most;
 }
 
 bool hgemm_supported(int wqt, int N, int K) {
@@ -540,17 +560,16 @@ hipError_t launch_hgemm_glu(int wqt, const void *W, const _Float16 *X, const flo
     const int N = 2 * F;
     if (!hgemm_supported(wqt, N, K) || F % 64 || T <= 0 || (long long)T * K * 2 >= (1ll << 31))
         return hipErrorNotSupported;
-    return go<true>(wqt, W, X, T, N, K, hg_plan_for(wqt, T, N, K, n_cu, 1), A, lda, xs, st);
+    return go<true>(wqt, W, X, T, N, K, hg_plan_for(wqt, T, N, K, n_cu, 1, 0), A, lda, xs, st);
 }
 
 // wqt: QT_F16 (IEEE fp16 rows, as k_dequant_f16 writes them) or QT_Q4_K.
-// C: T rows of N floats at row stride ldc.  part: hgemm_partial_bytes() of
-// device memory (unused with one slice).
+// C: T rows of N floats at row stride ldc.  part: part_bytes of device memory
+// for the slices' partial sums, which limit them (hgemm_partial_bytes() do not).
 hipError_t launch_hgemm(int wqt, const void *W, const _Float16 *X, int T, int N, int K, float *C, int ldc,
-                        float *part, int n_cu, hipStream_t st, int *nslices) {
+                        float *part, size_t part_bytes, int n_cu, hipStream_t st, int *nslices) {
     if (!hgemm_supported(wqt, N, K) || T <= 0 || (long long)T * K * 2 >= (1ll << 31)) return hipErrorNotSupported;
-    const HgPlan p = hg_plan_for(wqt, T, N, K, n_cu, HG_MAX_SLICES);
-    if (p.S > 1 && !part) return hipErrorInvalidValue;
+    const HgPlan p = hg_plan_for(wqt, T, N, K, n_cu, HG_MAX_SLICES, part ? part_bytes : 0);
     if (nslices && p.S > 1 && ldc != N) return hipErrorInvalidValue;   // slices are packed at row stride N
     const hipError_t err = go<false>(wqt, W, X, T, N, K, p, p.S > 1 ? part : C, p.S > 1 ? N : ldc, nullptr, st);
     if (nslices) *nslices = p.S;

@@ -122,15 +122,18 @@ hipError_t launch_quantize_q8k(const float *in, long long n, void *blocks, hipSt
 hipError_t launch_moe_i8(const MoeArgs &a, void *scratch, hipStream_t st);
 // Prefill weight products (tbq_gemm.hip): C[T][N] (row stride ldc) =
 // X[T][K] . W[N][K]^T, X fp16, W fp16 (QT_F16) or Q4_K rows; N % 4 == 0,
-// K % 256 == 0; part = hgemm_partial_bytes() of scratch.
+// K % 256 == 0; part: part_bytes of scratch for split-K
+// partial sums (hgemm_partial_bytes() for as many slices as the plan would take).
 int hgemm_cus();
 bool hgemm_supported(int wqt, int N, int K);
 size_t hgemm_partial_bytes(int T, int N, int K, int n_cu);
+// at least hgemm_partial_bytes of 1 .. T rows, and never less for a larger T
+size_t hgemm_partial_upto(int T, int N, int K, int n_cu);
 // With nslices set, the K slices' partial sums are left for the consumer to
 // add (in slice order): *nslices = S, and slice z is part + z * T * N (row
 // stride N) when S > 1; with S = 1 the product is in C as usual.
 hipError_t launch_hgemm(int wqt, const void *W, const _Float16 *X, int T, int N, int K, float *C, int ldc,
-                        float *part, int n_cu, hipStream_t st, int *nslices = nullptr);
+                        float *part, size_t part_bytes, int n_cu, hipStream_t st, int *nslices = nullptr);
 // The gate|up product (W: 2F rows, gate then up) with SwiGLU in the
 // epilogue: A[T][F] (row stride lda) = silu(g xs) (u xs), xs = X's row
 // scales; hipErrorNotSupported where F % 64 != 0.
@@ -146,7 +149,9 @@ hipError_t dense_final_logits(const tbq_dense_model *m, const float *x, const fl
 // token where the batched path does not apply).
 bool dense_prefill_batched(const tbq_dense_model *m);
 size_t dense_prefill_workspace_bytes(const tbq_dense_model *m, int T);
+// the same without room for split-K partial sums: the least a call can run with
+size_t dense_prefill_workspace_min(const tbq_dense_model *m, int T);
 hipError_t launch_dense_prefill(const tbq_dense_model *m, const int *tokens_host, int T, int pos0, float *logits,
-                                void *ws, hipStream_t st);
+                                void *ws, size_t ws_bytes, hipStream_t st);
 
 }  // namespace tbq
