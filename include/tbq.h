@@ -279,6 +279,11 @@ int tbq_gemm(int wqt, const void *W, const void *X16, int T, int N, int K, float
 int tbq_expf_device(const float *in, float *out, size_t n, void *stream);
 /* The same function compiled for the host. */
 float tbq_expf_host(float x);
+/* The tile and split that tbq_gemm (glu 0), or the dense prefill's product
+ * with SwiGLU in its epilogue (glu 1: N = 2 ffn), takes for a shape: plan[0]
+ * weight rows x plan[1] tokens, plan[2] K slices.  Host only; 0 if the shape
+ * is not supported. */
+int tbq_gemm_plan(int wqt, int T, int N, int K, int glu, int plan[3]);
 
 #ifdef __cplusplus
 }

@@ -75,8 +75,9 @@ def test_gemm_q4k_fused_matches_f16_path(oracle, T, N, K):
     assert rel_l2(b, ref) <= 1e-3
 
 
-# One shape on each side of the tiles' edges (32, 64, 128 and 256 tokens, 128
-# and 256 weight rows), one super-block, uneven slices, more tiles than CUs.
+# Ragged T and N around 32 to 256, one super-block, uneven slices.  The launch's
+# cost rule takes small tiles for nearly all of these; test_gemm_tiles.py goes
+# through every tile.
 @pytest.mark.parametrize("T,N,K", [
     (1, 4, 256), (31, 124, 512), (33, 132, 256), (64, 260, 8192), (65, 1028, 2304), (127, 256, 5120),
     (129, 6148, 768), (257, 516, 1792), (513, 3076, 256), (1030, 5124, 512),

@@ -5,8 +5,8 @@ token by token, layer4/tb_infer.c:1068-1075), through the C-ABI:
     last token's logits and the K/V cache
     rows of every prompt position within PREFILL_TOL of the float64 oracle
     run token by token, and of libtbq's own decode steps; prompts of 1, 7,
-    130 and 300 tokens (one, two and three 128-token GEMM tiles), from an
-    empty cache and after decoded tokens, head_dim 64 and 128, GQA 2, 4, 8;
+    130 and 300 tokens, from an empty cache and after decoded tokens, head_dim
+    64 and 128, GQA 2, 4, 8 (the GEMMs' tiles: test_gemm_tiles.py);
   * a one-token prefill is the decode step itself (bit-identical);
   * argument checks."""
 import numpy as np

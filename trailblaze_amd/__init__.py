@@ -60,6 +60,7 @@ SYMBOLS = {
     "tbq_gemm": (_i, [_i, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _sz, _vp]),
     "tbq_expf_device": (_i, [_vp, _vp, _sz, _vp]),
     "tbq_expf_host": (_f, [_f]),
+    "tbq_gemm_plan": (_i, [_i, _i, _i, _i, _i, _vp]),
     # include/tbq_gguf.h
     "tbq_gguf_open": (_vp, [C.c_char_p]),
     "tbq_gguf_close": (None, [_vp]),

@@ -500,4 +500,8 @@ int tbq_expf_device(const float *in, float *out, size_t n, void *s) {
 
 float tbq_expf_host(float x) { return expf_glibc(x); }
 
+int tbq_gemm_plan(int wqt, int T, int N, int K, int glu, int plan[3]) {
+    return plan && hgemm_plan(wqt, T, N, K, glu != 0, hgemm_cus(), plan) ? 1 : 0;
+}
+
 }  // extern "C"

@@ -551,6 +551,15 @@ bool hgemm_supported(int wqt, int N, int K) {
     return (wqt == QT_F16 || wqt == QT_Q4_K) && N > 0 && N % 4 == 0 && K > 0 && K % 256 == 0;
 }
 
+bool hgemm_plan(int wqt, int T, int N, int K, bool glu, int n_cu, int plan[3]) {
+    if (!hgemm_supported(wqt, N, K) || T <= 0 || (glu && N % 128)) return false;
+    const HgPlan p = hg_plan_for(wqt, T, N, K, n_cu, glu ? 1 : HG_MAX_SLICES, SIZE_MAX);
+    plan[0] = wqt == QT_F16 ? HG_F16[p.tile].rows : HG_Q4K[p.tile].rows;
+    plan[1] = wqt == QT_F16 ? HG_F16[p.tile].tok : HG_Q4K[p.tile].tok;
+    plan[2] = p.S;
+    return true;
+}
+
 // The gate/up product with SwiGLU in the epilogue: W holds 2F rows (gate then
 // up), A[T][F] (row stride lda) = silu(g xs) (u xs).  K is never split here
 // (the SwiGLU of partial sums is not defined).  hipErrorNotSupported where F

@@ -129,6 +129,8 @@ bool hgemm_supported(int wqt, int N, int K);
 size_t hgemm_partial_bytes(int T, int N, int K, int n_cu);
 // at least hgemm_partial_bytes of 1 .. T rows, and never less for a larger T
 size_t hgemm_partial_upto(int T, int N, int K, int n_cu);
+// the tile (weight rows, tokens) and slices a product takes, given room
+bool hgemm_plan(int wqt, int T, int N, int K, bool glu, int n_cu, int plan[3]);
 // With nslices set, the K slices' partial sums are left for the consumer to
 // add (in slice order): *nslices = S, and slice z is part + z * T * N (row
 // stride N) when S > 1; with S = 1 the product is in C as usual.
