@@ -839,7 +839,6 @@ static hipError_t pf_batched(const tbq_dense_model *m, const PfWs &w, int T, int
         // a fused gate|up matrix: SwiGLU in the GEMM's epilogue, then the
         // activation rows to fp16; otherwise the gate and up products and
         // k_pf_swiglu_f16
-        bool glu = false;
         if (L.wgu) {
             const int qt = qt_of(L.qt_gu);
             const void *Wg = L.wgu;
@@ -847,17 +846,13 @@ static hipError_t pf_batched(const tbq_dense_model *m, const PfWs &w, int T, int
                 break;
             if (qt != QT_Q4_K) Wg = w.wh;
             err = launch_hgemm_glu(qt == QT_Q4_K ? QT_Q4_K : QT_F16, Wg, w.h16, w.sa, T, F, H, w.gu, F, cu, st);
-            if (err == hipSuccess) glu = true;
-            else if (err == hipErrorNotSupported) err = gemm(qt, L.wgu, 2 * F, H, w.gu, 2 * F);
+            if (err == hipSuccess) err = launch_rows_f16(w.gu, T, F, w.h16, w.sb, st);
         } else {
             err = gemm(qt_of(L.qt_gate), L.wgate, F, H, w.gu, 2 * F);
             if (err == hipSuccess) err = gemm(qt_of(L.qt_up), L.wup, F, H, w.gu + F, 2 * F);
-        }
-        if (err != hipSuccess) break;
-        if (glu)
-            err = launch_rows_f16(w.gu, T, F, w.h16, w.sb, st);
-        else
+            if (err != hipSuccess) break;
             hipLaunchKernelGGL(k_pf_swiglu_f16, dim3(T), dim3(PS_THREADS), 0, st, w.gu, w.sa, F, w.h16, w.sb);
+        }
         if (err != hipSuccess) break;
         err = gemm(qt_of(L.qt_down), L.wdown, H, F, w.y, H, &yns);
         ysrc = yns > 1 ? w.gpart : w.y;

@@ -82,12 +82,15 @@ struct PfSub {
 // (= pair / k, the token).
 // ---------------------------------------------------------------------------
 constexpr int PF_MAX_TILES = 65536 * 8 / PF_MT + 256;
-// up to this many pairs, k_dispatch keeps the expert indices in registers
-// (read once) and the permutation in LDS (16 bits a pair): a permutation in
-// global memory is read back, after its own stores, by a loop of dependent
-// round trips (15992 pairs: 31 -> 19.5 us)
-constexpr int PF_LDS_PAIRS = 16384, PF_LDS_TILES = PF_LDS_PAIRS / PF_MT + 256;
-
+// NE > 0 (up to 1024 NE pairs): a thread keeps its NE pairs' expert indices in
+// registers (read once) and the permutation is in LDS (16 bits a pair); NE = 0:
+// any number, the permutation in global memory, read back after its own stores
+// by a loop of dependent round trips (15992 pairs: 31 -> 19.5 us with NE = 16).
+// One workgroup of code that no other launch keeps in the instruction cache is
+// bound by its length as well, hence an instance per range: in one kernel with
+// both forms and sixteen pairs a thread 4096 pairs took 10.9 us, with eight 8.9,
+// and NE = 4 takes 8.5 (2400 pairs: 6.3, 5.3 and 5.0).
+template <int NE>
 __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_idx, int T, int k, int E,
                                                    int *__restrict__ perm, PfTile *__restrict__ tiles,
                                                    int *__restrict__ ntiles, int *__restrict__ tpair,
@@ -96,18 +99,14 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_i
     static_assert(PF_MT == 128 && NQ == 4, "tile classes");
     __shared__ int hist[256], off[257], cur[256], wsum[4];
     __shared__ int qcnt[NQ + 1], qbase[NQ + 2];
-    // the tile list, and where the pairs fit the permutation behind it
-    constexpr int SMALL = 2 * PF_LDS_TILES + PF_LDS_PAIRS / 2;
-    __shared__ int lists[SMALL > 2 * PF_MAX_TILES ? SMALL : 2 * PF_MAX_TILES];
-    constexpr int NE = PF_LDS_PAIRS / 1024;   // expert indices per thread
+    constexpr int TILES = NE ? NE * 1024 / PF_MT + 256 : PF_MAX_TILES;
+    __shared__ int t_e[TILES], t_start[TILES];
+    __shared__ unsigned short perm_s[NE ? NE * 1024 : 1];
     const int tid = threadIdx.x, P = T * k;
-    const bool small = P <= PF_LDS_PAIRS;   // uniform
-    int *t_e = lists, *t_start = lists + (small ? PF_LDS_TILES : PF_MAX_TILES);
-    unsigned short *perm_s = reinterpret_cast<unsigned short *>(lists + 2 * PF_LDS_TILES);
     if (tid < 256) { hist[tid] = 0; cur[tid] = 0; }
     if (tid <= NQ) qcnt[tid] = 0;
-    int es[NE];
-    if (small) {
+    int es[NE ? NE : 1];
+    if constexpr (NE > 0) {
 #pragma unroll
         for (int m = 0; m < NE; m++) {
             const int p = tid + 1024 * m;
@@ -117,7 +116,7 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_i
     __syncthreads();
     // a pair whose expert index is outside [0, E) (never produced by the
     // router) joins no tile; the combine skips its slot
-    if (small) {
+    if constexpr (NE > 0) {
 #pragma unroll
         for (int m = 0; m < NE; m++)
             if ((unsigned)es[m] < (unsigned)E) atomicAdd(&hist[es[m]], 1);
@@ -189,7 +188,7 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_i
             t_start[t] = off[tid] + s0;
         }
     }
-    if (small) {
+    if constexpr (NE > 0) {
 #pragma unroll
         for (int m = 0; m < NE; m++) {
             const int e = es[m];
@@ -209,10 +208,23 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int *__restrict__ sel_i
         const int t = i >> 7, j = i & (PF_MT - 1), te = t_e[t], st = t_start[t];
         const int e = te & 0xFFFF, n = te >> 16;
         if (j == 0) tiles[t] = PfTile{e, n};
-        const int p = j < n ? (small ? perm_s[st + j] : perm[st + j]) : -1;
+        int p = -1;
+        if (j < n) p = NE ? perm_s[st + j] : perm[st + j];
         tpair[i] = p;
         ttok[i] = p >= 0 ? p / k : -1;
     }
+}
+
+static void launch_dispatch(const MoeArgs &a, int *perm, PfTile *tiles, int *ntiles, int *tpair, int *ttok, hipStream_t st) {
+#define TBQ_DISPATCH(NE)                                                                                            \
+    hipLaunchKernelGGL(k_dispatch<NE>, dim3(1), dim3(1024), 0, st, a.sel_idx, a.T, a.k, a.E, perm, tiles, ntiles, \
+                       tpair, ttok)
+    const long long P = (long long)a.T * a.k;
+    if (P <= 4096) TBQ_DISPATCH(4);
+    else if (P <= 8192) TBQ_DISPATCH(8);
+    else if (P <= 16384) TBQ_DISPATCH(16);
+    else TBQ_DISPATCH(0);
+#undef TBQ_DISPATCH
 }
 
 // ---------------------------------------------------------------------------
@@ -375,7 +387,7 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
 #pragma unroll
         for (int i = 0; i < NB; i++) dma16(ax + slot * XS + MF_WAVES * i * 1024, xv[i], xr, min(step, nst - 1) * 128);
     };
-    auto copy_q = [&](int slot, int step) {   // steps past the end: empty descriptors, no memory access
+    auto copy_q = [&](int slot, int step) {   // steps past the end copy bytes of the last super-block again, never read
         const uint32_t so = (min(step, nst - 1) >> 2) * 144 + (step & 3) * 32;
         if constexpr (MIX) dma16_ptr(aq + slot * QS, qp + so);
         else dma16(aq + slot * QS, qv, r0, so);
@@ -1095,8 +1107,7 @@ hipError_t launch_moe_prefill_q4k_i8(const MoeArgs &a, void *scratch, hipStream_
     _Float16 *ab = (_Float16 *)w;
     hipError_t err = launch_rows_q8(a.xn, a.T, a.H, x8, xd, xb, st);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(k_dispatch, dim3(1), dim3(1024), 0, st, a.sel_idx, a.T, a.k, a.E, perm, tiles, ntiles, tpair,
-                       ttok);
+    launch_dispatch(a, perm, tiles, ntiles, tpair, ttok, st);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
     const int ncb0 = a.F / PF_COLS, ncb1 = a.H / PF_ROWS;
@@ -1208,8 +1219,7 @@ hipError_t launch_moe_prefill_q4k(const MoeArgs &a, void *scratch, hipStream_t s
         const hipError_t e = launch_rows_f16(a.xn, a.T, a.H, x16, xinv, st, gg);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_dispatch, dim3(1), dim3(1024), 0, st, a.sel_idx, a.T, a.k, a.E, perm, tiles, ntiles, tpair,
-                       ttok);
+    launch_dispatch(a, perm, tiles, ntiles, tpair, ttok, st);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     const uint8_t *wg = (const uint8_t *)a.gate, *wu = (const uint8_t *)a.up, *wd = (const uint8_t *)a.down;
