@@ -470,6 +470,9 @@ def test_moe_prefill_i8_small_batches(oracle, H, F, E, k):
     (1, 256, 512, 2, 1), (31, 512, 256, 3, 2), (33, 256, 256, 4, 2), (64, 768, 512, 2, 2), (65, 256, 768, 4, 1),
     (97, 512, 256, 2, 1), (128, 256, 256, 3, 1), (129, 512, 256, 2, 2),
     (33, 256, 4096, 64, 8), (129, 256, 4096, 64, 8), (97, 4096, 256, 128, 8),
+    # two row blocks per wave on 256 CUs, 16 tiles (128 pairs, and 1 to 128): gate/up, then down
+    (161, 256, 4096, 8, 8), (193, 256, 4096, 8, 8), (256, 256, 4096, 8, 8),
+    (129, 4096, 256, 8, 8), (161, 4096, 256, 8, 8), (193, 4096, 256, 8, 8), (256, 4096, 256, 8, 8),
 ])
 def test_moe_prefill_tile_edges(oracle, qt, T, H, F, E, k):
     import torch

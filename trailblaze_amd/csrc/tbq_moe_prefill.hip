@@ -294,7 +294,8 @@ __device__ __forceinline__ unsigned f16x2_no_subnormal(unsigned h) {
 
 // ---------------------------------------------------------------------------
 // Expert tile GEMM.  Work items are (tile, row block) pairs, tile-major (ncb =
-// F / (64 NA) row blocks of columns for MODE 0, H / (128 NA) of rows for MODE 1),
+// F / (64 NA) row blocks of columns for MODE 0, H / (128 NA) of rows for MODE 1;
+// NA by mf_two_blocks, from the tiles that the dispatch made),
 // the tiles heaviest first.  The grid is persistent (two workgroups of four
 // waves per CU): workgroup b starts with item b, then takes tickets from the
 // counter ntiles[1 + MODE] (zeroed by k_dispatch): item grid + ticket, the
@@ -539,7 +540,9 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
 #pragma unroll
                     for (int b = 0; b < NA; b++)
                         acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kk & 1][b], bf[kk & 1][t], acc[b][t], 0, 0, 0);
-                if constexpr (!GG && NA == 2 && NB >= 3) {   // keep the decode between the MFMAs: run ahead, it spills
+                // keep the decode between the MFMAs: run ahead, it spills in the loop
+                // (the few registers that still do hold per-item state)
+                if constexpr (!GG && NA == 2 && NB >= 3) {
 #pragma unroll
                     for (int i = 0; i < NA * NB; i++) {
                         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
@@ -589,51 +592,83 @@ __device__ __forceinline__ void mf_item(unsigned char *lds, const uint8_t *w0, c
     }
 }
 
-template <int MODE, bool GG, int NA>
+// Row blocks per wave, by the items that two blocks would make (a) for the slots
+// (two workgroups per CU) and the pairs per tile (p).  Two read the activations
+// half as often and decode between twice the MFMAs; one halves the items, which
+// shortens the last round and fills a chip with few of them.  Two are better
+// from 40 (down: 32) pairs per tile on, but not where few items, or a last round
+// nearly empty, leave slots idle; below that they gain where one round is just
+// filled (gate/up: up to a second round's start), and otherwise the weights'
+// lines of twice the rows in flight do not stay in L2.  Fitted over 194 layers of
+// H 1024..3072, F 512..1536, E 32..128, k 2..8 and 33..2048 tokens, half of them
+// Zipf-skewed: 0.5% from the best choice for each, one block everywhere 1.5%,
+// two everywhere 5.9% (2048 x 768, 128 experts, 900 tokens: 246 us with one, 227
+// with two; 700 Zipf-skewed: 198 and 213).  Over 120 other layers 4 were more
+// than 1% slower than on the 8-wave workgroups of 256 rows before these kernels.
+template <int MODE>
+__device__ __forceinline__ bool mf_two_blocks(int a, int pairs, int tiles, int slots) {
+    if (a > slots && 10 * a < (MODE == 0 ? 13 : 15) * slots) return false;
+    if constexpr (MODE == 0) {
+        if (pairs >= 40 * tiles) return 5 * a >= 4 * slots;
+        return 8 * a >= 7 * slots && 5 * a <= 8 * slots;
+    } else {
+        if (pairs >= 32 * tiles) return 2 * a >= slots && (2 * a < 5 * slots || pairs >= 64 * tiles);
+        return 10 * a >= 9 * slots && a <= slots;
+    }
+}
+
+template <int MODE, bool GG>
 __global__ __launch_bounds__(64 * MF_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_moe_f16(
     const uint8_t *__restrict__ W0, const uint8_t *__restrict__ W1, const _Float16 *__restrict__ X, int x_rows,
     const float *__restrict__ xinv, const int *__restrict__ tpair, const int *__restrict__ ttok,
-    const PfTile *__restrict__ tiles, int *__restrict__ ntiles, int ncb, int H, int F, float *__restrict__ out) {
+    const PfTile *__restrict__ tiles, int *__restrict__ ntiles, int pairs, int slots, int H, int F, float *__restrict__ out) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char mf_lds_p[];
-    const int K = MODE == 0 ? H : F, nitems = *ntiles * ncb;
+    const int K = MODE == 0 ? H : F, nt = *ntiles;
     const uint32_t rb = (uint32_t)(K >> 8) * 144u;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     MfLists &ml = *reinterpret_cast<MfLists *>(mf_lds_p + MF_RING);
     const dma_rsrc_t sr = dma_rsrc(xinv, (uint32_t)x_rows * 4u);
     const int lane = threadIdx.x & 63;
-    for (int item = blockIdx.x; item < nitems;) {
-        const int tix = item / ncb, cb = item % ncb;
-        const PfTile tl = tiles[tix];
-        const int *xrows = (MODE == 0 ? ttok : tpair) + (long long)tix * PF_MT;
-        // the tile's pair ids and row scales to LDS for the epilogue (rows
-        // past its pairs: row 0's scale, not used)
-        if (wave < 2) {
-            const uint32_t r = (uint32_t)max(xrows[64 * wave + lane], 0);
-            dma4(lds_addr(ml.tp) + 256 * wave, 4u * (64 * wave + lane), dma_rsrc(tpair + (long long)tix * PF_MT, PF_MT * 4));
-            dma4(lds_addr(ml.xsc) + 256 * wave, 4u * r, sr);
+    const int n2 = MODE == 0 ? F / (MF_ROWS / 2) : H / MF_ROWS;   // row blocks at NA = 2
+    auto run = [&](auto na) {
+        constexpr int NA = decltype(na)::value;
+        const int ncb = NA == 1 ? 2 * n2 : n2, nitems = nt * ncb;
+        for (int item = blockIdx.x; item < nitems;) {
+            const int tix = item / ncb, cb = item % ncb;
+            const PfTile tl = tiles[tix];
+            const int *xrows = (MODE == 0 ? ttok : tpair) + (long long)tix * PF_MT;
+            // the tile's pair ids and row scales to LDS for the epilogue (rows
+            // past its pairs: row 0's scale, not used)
+            if (wave < 2) {
+                const uint32_t r = (uint32_t)max(xrows[64 * wave + lane], 0);
+                dma4(lds_addr(ml.tp) + 256 * wave, 4u * (64 * wave + lane), dma_rsrc(tpair + (long long)tix * PF_MT, PF_MT * 4));
+                dma4(lds_addr(ml.xsc) + 256 * wave, 4u * r, sr);
+            }
+            const int e = __builtin_amdgcn_readfirstlane(tl.e), n = __builtin_amdgcn_readfirstlane(tl.n);
+            const int col = (cb * MF_WAVES + wave) * (MODE == 0 ? 16 : 32) * NA;
+            const uint8_t *w0 = W0 + ((long long)e * (MODE == 0 ? F : H) + col) * rb;
+            const uint8_t *w1 = MODE == 0 ? W1 + ((long long)e * F + col) * rb : w0 + 32ll * rb;
+            int nxt = 0;
+            auto body = [&](auto nb) {
+                mf_item<MODE, GG, NA, decltype(nb)::value>(mf_lds_p, w0, w1, rb, K, X, (uint32_t)x_rows * (uint32_t)(K * 2),
+                                                       xrows, ml.tp, ml.xsc, n, col, MODE == 0 ? F : H, out,
+                                                       ntiles + 1 + MODE, nxt);
+            };
+            switch ((n + 31) / 32) {   // uniform
+            case 1: body(PfSub<1>{}); break;
+            case 2: body(PfSub<2>{}); break;
+            case 3: body(PfSub<3>{}); break;
+            default: body(PfSub<4>{}); break;
+            }
+            // every wave is past its last read of the rings and lists when all
+            // have passed this barrier
+            if (threadIdx.x == 0) ml.next = nxt;
+            dma_wait_barrier();
+            item = __builtin_amdgcn_readfirstlane(ml.next);
         }
-        const int e = __builtin_amdgcn_readfirstlane(tl.e), n = __builtin_amdgcn_readfirstlane(tl.n);
-        const int col = (cb * MF_WAVES + wave) * (MODE == 0 ? 16 : 32) * NA;
-        const uint8_t *w0 = W0 + ((long long)e * (MODE == 0 ? F : H) + col) * rb;
-        const uint8_t *w1 = MODE == 0 ? W1 + ((long long)e * F + col) * rb : w0 + 32ll * rb;
-        int nxt = 0;
-        auto body = [&](auto nb) {
-            mf_item<MODE, GG, NA, decltype(nb)::value>(mf_lds_p, w0, w1, rb, K, X, (uint32_t)x_rows * (uint32_t)(K * 2),
-                                                   xrows, ml.tp, ml.xsc, n, col, MODE == 0 ? F : H, out,
-                                                   ntiles + 1 + MODE, nxt);
-        };
-        switch ((n + 31) / 32) {   // uniform
-        case 1: body(PfSub<1>{}); break;
-        case 2: body(PfSub<2>{}); break;
-        case 3: body(PfSub<3>{}); break;
-        default: body(PfSub<4>{}); break;
-        }
-        // every wave is past its last read of the rings and lists when all
-        // have passed this barrier
-        if (threadIdx.x == 0) ml.next = nxt;
-        dma_wait_barrier();
-        item = __builtin_amdgcn_readfirstlane(ml.next);
-    }
+    };
+    if (mf_two_blocks<MODE>(nt * n2, pairs, nt, slots)) run(PfSub<2>{});   // uniform
+    else run(PfSub<1>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -1007,47 +1042,27 @@ size_t prefill_workspace_bytes(int T, int k, int E, int H, int F) {
            up((size_t)T * H * 2) + up(P * 4) + up((size_t)T * 4);
 }
 
-// Persistent grid of the expert GEMMs: one workgroup per CU (about 200
-// VGPRs per lane hold two of the eight waves per SIMD, so a second
-// workgroup would only queue behind the first), never more than the item
-// count bound.
+// Persistent grid of the int8 expert GEMMs: one workgroup per CU (130 to 157 KiB
+// of its LDS: a second would only queue behind the first), never more than the
+// item count bound.
 static unsigned pf_grid(unsigned max_items) {
     const unsigned g = (unsigned)(tbq_cu_count() > 0 ? tbq_cu_count() : 256);
     return max_items < g ? max_items : g;
-}
-
-template <int MODE, bool GG, int NA>
-static hipError_t launch_moe_f16_na(unsigned max_items, hipStream_t st, const uint8_t *W0, const uint8_t *W1,
-                                 const _Float16 *X, int x_rows, const float *xinv, const int *tpair, const int *ttok,
-                                 const PfTile *tiles, int *ntiles, int ncb, int H, int F, float *out) {
-    // more than 64 KiB of dynamic LDS is opted into once per kernel
-    static const hipError_t attr =
-        hipFuncSetAttribute((const void *)k_moe_f16<MODE, GG, NA>, hipFuncAttributeMaxDynamicSharedMemorySize, MF_LDS);
-    if (attr != hipSuccess) return attr;
-    const unsigned g = 2u * (unsigned)(tbq_cu_count() > 0 ? tbq_cu_count() : 256);   // two workgroups per CU
-    hipLaunchKernelGGL((k_moe_f16<MODE, GG, NA>), dim3(max_items < g ? max_items : g), dim3(64 * MF_WAVES), MF_LDS, st, W0,
-                       W1, X, x_rows, xinv, tpair, ttok, tiles, ntiles, ncb, H, F, out);
-    return hipGetLastError();
 }
 
 template <int MODE, bool GG>
 static hipError_t launch_moe_f16(const MoeArgs &a, int max_tiles, hipStream_t st, const uint8_t *W0, const uint8_t *W1, const _Float16 *X,
                                  int x_rows, const float *xinv, const int *tpair, const int *ttok, const PfTile *tiles,
                                  int *ntiles, int H, int F, float *out) {
-    const int n2 = MODE == 0 ? F / (MF_ROWS / 2) : H / MF_ROWS;   // row blocks at NA = 2
-    // Row blocks per wave.  One is better while the items (about P / 128 + E / 2
-    // tiles) are fewer than two rounds of the 512 workgroup slots: twice the
-    // items of half the length fill the chip and hide a step's latencies (60
-    // tokens, 32 experts 52.7 -> 43.7 us a layer, 128 tokens 63.9 -> 50.8, 512
-    // Zipf-skewed of 128 experts 173 -> 166.6); two read the activations half as
-    // often and decode between twice the MFMAs (1999 tokens of 128 experts 401
-    // against 391 us with one; 1500 of 64 the same).
-    const long long P = (long long)a.T * a.k, tiles_est = P / PF_MT + (P < a.E ? P : a.E) / 2;
-    if (tiles_est * n2 <= 1024)
-        return launch_moe_f16_na<MODE, GG, 1>((unsigned)(2 * max_tiles * n2), st, W0, W1, X, x_rows, xinv, tpair, ttok,
-                                              tiles, ntiles, 2 * n2, H, F, out);
-    return launch_moe_f16_na<MODE, GG, 2>((unsigned)(max_tiles * n2), st, W0, W1, X, x_rows, xinv, tpair, ttok, tiles,
-                                          ntiles, n2, H, F, out);
+    // more than 64 KiB of dynamic LDS is opted into once per kernel
+    static const hipError_t attr =
+        hipFuncSetAttribute((const void *)k_moe_f16<MODE, GG>, hipFuncAttributeMaxDynamicSharedMemorySize, MF_LDS);
+    if (attr != hipSuccess) return attr;
+    const unsigned slots = 2u * (unsigned)(tbq_cu_count() > 0 ? tbq_cu_count() : 256);   // two workgroups per CU
+    const unsigned items = 2u * (unsigned)max_tiles * (unsigned)(MODE == 0 ? F / (MF_ROWS / 2) : H / MF_ROWS);   // at NA = 1
+    hipLaunchKernelGGL((k_moe_f16<MODE, GG>), dim3(items < slots ? items : slots), dim3(64 * MF_WAVES), MF_LDS, st, W0, W1, X,
+                       x_rows, xinv, tpair, ttok, tiles, ntiles, a.T * a.k, (int)slots, H, F, out);
+    return hipGetLastError();
 }
 
 // K values the MFMA kernel is instantiated for (K = 128 * NS).
