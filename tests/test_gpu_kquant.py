@@ -149,11 +149,11 @@ def test_matvec_kq_kernel(oracle, qt, M, K):
 
 @pytest.mark.parametrize("qt", [fm.Q3_K, fm.Q4_K, fm.Q6_K, fm.Q8_0, fm.GGML | fm.Q4_K])
 @pytest.mark.parametrize("M,K", [(63, 1024), (8192, 1024), (8193, 1024), (4096, 2048), (4097, 2048), (17, 4096),
-                                 (2048, 4096), (2049, 4096)])
+                                 (1024, 4096), (1025, 4096), (2048, 4096), (2049, 4096)])
 def test_matvec_kq_short_matrices(oracle, qt, M, K):
-    """Rows of 16, 32 and 64 units on both sides of the row count where
-    workgroups of 16 waves would leave half the compute units without one
-    (256 units of 64, 32 and 16 rows), where 4-wave workgroups take over."""
+    """Rows of 16, 32 and 64 units on both sides of the row count where 4-wave
+    workgroups take over: workgroups of 16 waves (64, 32 and 16 rows) would
+    leave half of 256 compute units without one, three quarters at 64 units."""
     rng = np.random.default_rng(M * 17 + K + 3 * (qt & 255))
     W = synth.kquant_matrix(qt, M, K, rng)
     x = synth.activations(K, rng)

@@ -1318,14 +1318,17 @@ static hipError_t launch_kq_q(const void *W, int M, int K, const float *x, float
     // (Q8_0, 256 CUs, K = 1024: gate|up with SwiGLU 2 x 3072 rows on 48
     // workgroups, spilling under 128 registers, 12.4 -> 4.5 us; 2048 rows 5.1 ->
     // 3.4; 1024 rows with the residual 5.0 -> 3.2; 1024x3072 5.0 -> 3.6); with
-    // more workgroups than that each CU stages x four times over for nothing
-    auto few = [&](int rows) { return 2 * (((long long)M + rows - 1) / rows) <= n_cu; };
+    // more workgroups than that each CU stages x four times over for nothing.
+    // Rows of more than 32 units only where the 4-wave ones are at most one per
+    // CU: staging 4096 columns twice on a CU costs more than it gains (1024x4096
+    // Q2_K 0.92 of the time, Q6_K 0.81; 2048x4096 1.10 and 1.04)
+    auto few = [&](int rows, int share) { return share * (((long long)M + rows - 1) / rows) <= n_cu; };
     if (U <= 16) {
-        if (few(NW * 4)) return launch_kq_shape<QT, 16, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
+        if (few(NW * 4, 2)) return launch_kq_shape<QT, 16, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
         return launch_kq_shape<QT, 16, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
     }
     if (U <= 32) {
-        if (few(NW * 2)) return launch_kq_shape<QT, 32, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
+        if (few(NW * 2, 2)) return launch_kq_shape<QT, 32, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
         return launch_kq_shape<QT, 32, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
     }
     // Tall matrices of 64-unit rows: the segmented mapping, 16 rows per
@@ -1347,7 +1350,7 @@ static hipError_t launch_kq_q(const void *W, int M, int K, const float *x, float
     if constexpr (QT != QT_Q8_0 && QT != QT_GQ8_0)
         if (U < 64 && (U & (U - 1)) != 0) return launch_kq_seg<QT, KQ_SEG_NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
     if (U <= 64) {
-        if (few(NW)) return launch_kq_shape<QT, 64, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
+        if (few(NW, 4)) return launch_kq_shape<QT, 64, 1, 4, PRO, GLU, 4>(W, M, K, x, y, st, n_cu, pro);
         return launch_kq_shape<QT, 64, 1, NW, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
     }
     if (U <= 128) return launch_kq_shape<QT, 64, 2, NW / 2, PRO, GLU>(W, M, K, x, y, st, n_cu, pro);
