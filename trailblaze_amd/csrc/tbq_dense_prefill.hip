@@ -403,8 +403,8 @@ __global__ __launch_bounds__(64) void k_pf_scale_row(const float *__restrict__ y
 // stores), and k_pf_attn_rows merges the splits a row reaches.
 //
 // Bound by the softmax's VALU work beside the MFMAs.  T = 1999 after 1024
-// cached positions, 32 / 8 heads of 128: 293 -> 93 us (0.7 PFLOP/s), T = 512
-// from position 0: 25.2 -> 14.6 us, against converting the fp32 cache rows in
+// cached positions, 32 / 8 heads of 128: 293 -> 99 us (0.65 PFLOP/s), T = 512
+// from position 0: 25.2 -> 14 to 16 us, against converting the fp32 cache rows in
 // every query block, 32 positions at a time between two barriers (and 5 to 11
 // us of k_pf_kv16, which that form did without).  Two workgroups of 4 waves
 // per CU; 8 waves (half the copies, one workgroup per CU) were 1% slower on the

@@ -12,10 +12,10 @@
 //                     (exact, undone in the GEMM epilogues): x for gate/up,
 //                     the SwiGLU activations for down.
 //   k_moe_f16<0>      act[p] = swiglu(x_t . W_gate[e], x_t . W_up[e]) for a
-//                     tile of <= 128 pairs x 128 columns (256 weight rows:
-//                     128 gate and 128 up rows), K = H, fp32 out.
-//   k_moe_f16<1>      y[p] = act[p] . W_down[e] for <= 128 pairs x 256 rows,
-//                     K = F.
+//                     tile of <= 128 pairs x 64 or 128 columns (as many gate
+//                     and as many up rows), K = H, fp32 out.
+//   k_moe_f16<1>      y[p] = act[p] . W_down[e] for <= 128 pairs x 128 or 256
+//                     rows, K = F.
 //   (k_combine)       out = resid + sum over slots in slot order (tbq_moe.hip).
 //
 // Weights never pass through LDS as fp16: their packed bytes are staged and
@@ -327,12 +327,13 @@ __device__ __forceinline__ unsigned f16x2_no_subnormal(unsigned h) {
 // ^ swizzle(row), so column reads spread over all banks.
 //
 // Against one 8-wave workgroup per CU whose lanes loaded their own rows' bytes
-// (a cache line per lane and load), whole layer: 60 tokens of 32 experts 55.3 ->
-// 43.7 us, 300 of 128 91.1 -> 79.5, Qwen3-30B-A3B with 512 Zipf-skewed tokens
-// 176.4 -> 166.6, 1999 of ggml's layout 433 -> 391.  Left at 512 tokens: 204 +
-// 153 MB read (39 + 29 us at the copy rate) while the heaviest experts' tiles,
-// which set the end, wait for the same memory; at NA = 2 the two GEMMs take 127
-// us, without copies 88, without the dequantisation as well 71.
+// (a cache line per lane and load), whole layer of 128 experts, top 8, H 2048, F
+// 768, in us: 40 tokens 150 -> 145, 512 Zipf-skewed 164 -> 155, 900 even 238 -> 229,
+// 1999 of ggml's layout 427 -> 374; 8% over 300 random layers, 11 of them slower by
+// more than 1% (at most 7%, nearly all of H = 1536).  Left at 512 tokens: 183 + 140
+// MB read (35 + 27 us at the copy rate) while the heaviest experts' tiles, which
+// set the end, wait for the same memory; at NA = 2 the two GEMMs took 127 us,
+// without copies 88, without the dequantisation as well 71.
 // ---------------------------------------------------------------------------
 constexpr int MF_WAVES = 4, MF_ROWS = 64 * MF_WAVES;   // rows at two blocks per wave
 constexpr int mf_depth(int nb) { return nb == 1 ? 5 : nb == 2 ? 4 : 3; }
