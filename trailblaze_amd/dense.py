@@ -111,10 +111,12 @@ class SyntheticDense:
         token's logits into `logits`, K/V of every position appended."""
         import torch
         toks = np.ascontiguousarray(tokens, dtype=np.int32)
-        n = int(lib().tbq_dense_prefill_workspace_size(C.byref(self.model), len(toks)))
         ws = getattr(self, "_pf_ws", None)
-        if n > 0 and (ws is None or ws.numel() < n):
-            ws = self._pf_ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+        if ws is None or len(toks) > self._pf_len:   # a workspace serves every shorter prompt
+            n = int(lib().tbq_dense_prefill_workspace_size(C.byref(self.model), len(toks)))
+            if n > 0:
+                ws = self._pf_ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+                self._pf_len = len(toks)
         self._pf_tokens = toks   # read by an asynchronous copy on the stream
         # (n == 0: bad arguments, which the call itself reports)
         _check(lib().tbq_dense_prefill(C.byref(self.model), toks.ctypes.data, len(toks), pos0, _ptr(logits),
